@@ -18,6 +18,7 @@
 #include "mesh.hpp"
 #include "refelem.hpp"
 #include "stage_kernels.hpp"
+#include "stage_sym.hpp"
 
 using namespace dg;
 
@@ -76,6 +77,63 @@ void build_fragments(const RefElem& re, std::vector<double>& VqF, std::vector<do
                 const int j = 16 * m + (l & 15), f = s / SF, g = 4 * (s % SF) + (l >> 4);
                 if (j < Np && g < Nfq) LF[(size_t(s) * MT + m) * 64 + l] = re.Lift[size_t(j) * 3 * Nfq + f * Nfq + g];
             }
+}
+
+// Fragments of the mirror-symmetric FP64 stage kernel in the order of SymDims: lane l of a fragment holds operator
+// row 16 tile + l % 16 and K row 4 step + l / 16.
+template <int N>
+bool build_sym(const RefElem& re, std::vector<double>& F, std::vector<int>& rows) {
+    using D = SymDims<N>;
+    const RefElem::Mirror& mi = re.mirror;
+    if (mi.npair != D::npair || mi.nrow != D::nrow || mi.qpair != D::qpair || mi.qrow != D::qrow) return false;
+    const int Nq = re.Nq, Nfq = re.Nfq;
+    F.assign(D::nF, 0.0);
+    size_t at = 0;
+    // one fragment: entry (row, k) of an nr x nk operator given by val, zero beyond
+    auto put = [&](int tile, int nr, auto&& val) {
+        for (int l = 0; l < 64; ++l, ++at) {
+            const int i = 16 * tile + (l & 15);
+            if (i < nr) F[at] = val(i, l >> 4);
+        }
+    };
+    for (int t = 0; t < D::TE; ++t)
+        for (int s = 0; s < D::KE; ++s)
+            put(t, mi.qrow, [&](int i, int k) { return 4 * s + k < mi.nrow ? mi.Ve[size_t(i) * mi.nrow + 4 * s + k] : 0.0; });
+    for (int t = 0; t < D::TO; ++t)
+        for (int s = 0; s < D::KO; ++s)
+            put(t, mi.qpair,
+                [&](int i, int k) { return 4 * s + k < mi.npair ? mi.Vo[size_t(i) * mi.npair + 4 * s + k] : 0.0; });
+    auto rows_of = [&](const std::vector<double>& E, const std::vector<double>& O, int ncol, auto&& column) {
+        for (int m = 0; m < D::ME; ++m)
+            put(m, mi.nrow, [&](int i, int k) { const int c = column(k); return c >= 0 ? E[size_t(i) * ncol + c] : 0.0; });
+        for (int m = 0; m < D::MO; ++m)
+            put(m, mi.npair, [&](int i, int k) { const int c = column(k); return c >= 0 ? O[size_t(i) * ncol + c] : 0.0; });
+    };
+    for (int ks = 0; ks < D::KT; ++ks) {
+        rows_of(mi.Pe, mi.Po, Nq, [&](int k) { return 4 * ks + k < mi.qrow ? mi.pa[4 * ks + k] : -1; });
+        if (ks < D::KP)
+            rows_of(mi.Pe, mi.Po, Nq, [&](int k) { return 4 * ks + k < mi.qpair ? mi.pb[4 * ks + k] : -1; });
+    }
+    for (int f = 0; f < 2; ++f)   // face 0 (its fluxes already combined with the mirror image on face 2), face 1
+        for (int j = 0; j < D::SF; ++j)
+            rows_of(mi.Le, mi.Lo, 3 * Nfq, [&](int k) { return 4 * j + k < Nfq ? f * Nfq + 4 * j + k : -1; });
+    rows.assign(4 * D::KE, 0);
+    for (int i = 0; i < mi.nrow; ++i) rows[i] = mi.a[i] | mi.b[i] << 8;
+    return at == F.size();
+}
+
+bool build_sym_fragments(const RefElem& re, std::vector<double>& F, std::vector<int>& rows) {
+    switch (re.N) {
+        case 1: return build_sym<1>(re, F, rows);
+        case 2: return build_sym<2>(re, F, rows);
+        case 3: return build_sym<3>(re, F, rows);
+        case 4: return build_sym<4>(re, F, rows);
+        case 5: return build_sym<5>(re, F, rows);
+        case 6: return build_sym<6>(re, F, rows);
+        case 7: return build_sym<7>(re, F, rows);
+        case 8: return build_sym<8>(re, F, rows);
+        default: return false;
+    }
 }
 
 // bf16 with round-to-nearest-even of a finite float
@@ -210,16 +268,21 @@ RefDev* dgh_ctx_s::refdev(int N) {
         fail(DGH_ERR_UNSUPPORTED, "order N=%d not supported (1..8)", N);
         return nullptr;
     }
-    std::vector<double> VqF, PF, LF, VqF32, PF32, LF32;
+    std::vector<double> VqF32, PF32, LF32;
     std::vector<uint32_t> VqS, PS, LS;
-    build_fragments<double>(rd->re, VqF, PF, LF);
+    std::vector<double> symF;
+    std::vector<int> symRows;
+    if (!build_sym_fragments(rd->re, symF, symRows)) {
+        fail(DGH_ERR_UNSUPPORTED, "order N=%d: the reference element is not mirror symmetric", N);
+        return nullptr;
+    }
     build_fragments<float>(rd->re, VqF32, PF32, LF32);
     build_split_fragments(rd->re, VqS, PS, LS);
-    bool ok = upload(&rd->VqF64, VqF) && upload(&rd->PF64, PF) && upload(&rd->LF64, LF) &&
-              upload(&rd->Vf64, rd->re.Vf) && upload(&rd->VqF32, cast_vec<float>(VqF32)) &&
+    bool ok = upload(&rd->Vf64, rd->re.Vf) && upload(&rd->VqF32, cast_vec<float>(VqF32)) &&
               upload(&rd->PF32, cast_vec<float>(PF32)) && upload(&rd->LF32, cast_vec<float>(LF32)) &&
               upload(&rd->Vf32, cast_vec<float>(rd->re.Vf)) && upload(&rd->fmask, rd->re.fmask) &&
-              upload(&rd->VqS, VqS) && upload(&rd->PS, PS) && upload(&rd->LS, LS);
+              upload(&rd->VqS, VqS) && upload(&rd->PS, PS) && upload(&rd->LS, LS) && upload(&rd->symF, symF) &&
+              upload(&rd->symRows, symRows);
     if (!ok) return nullptr;
     RefDev* p = rd.get();
     refs[N] = std::move(rd);
@@ -250,9 +313,9 @@ MeshDev::~MeshDev() {
     for (auto& w : ws) { dfree(w.second.res); dfree(w.second.tmp); }
 }
 RefDev::~RefDev() {
-    dfree(VqF64); dfree(PF64); dfree(LF64); dfree(Vf64);
+    dfree(Vf64);
     dfree(VqF32); dfree(PF32); dfree(LF32); dfree(Vf32); dfree(fmask);
-    dfree(VqS); dfree(PS); dfree(LS);
+    dfree(VqS); dfree(PS); dfree(LS); dfree(symF); dfree(symRows);
     dfree(insSr); dfree(insSs); dfree(insLift); dfree(insDr); dfree(insDs);
 }
 FieldDev::~FieldDev() { dfree(d); }
@@ -654,11 +717,12 @@ static int stage_launch(dgh_ctx c, MeshDev* m, const dgh_rhs_desc* d, const doub
     a.geo = f64 ? static_cast<const void*>(m->geo64) : static_cast<const void*>(m->geo32);
     a.conn = m->conn;
     const bool split = d->prec == DGH_PREC_BF16X3;
-    a.VqF = f64 ? static_cast<const void*>(rd->VqF64) : split ? static_cast<const void*>(rd->VqS) : rd->VqF32;
-    a.PF = f64 ? static_cast<const void*>(rd->PF64) : split ? static_cast<const void*>(rd->PS) : rd->PF32;
-    a.LF = f64 ? static_cast<const void*>(rd->LF64) : split ? static_cast<const void*>(rd->LS) : rd->LF32;
+    // FP64: the mirror-half fragments and node rows of stage_sym.hip
+    a.VqF = f64 ? static_cast<const void*>(rd->symF) : split ? static_cast<const void*>(rd->VqS) : rd->VqF32;
+    a.PF = f64 ? nullptr : split ? static_cast<const void*>(rd->PS) : rd->PF32;
+    a.LF = f64 ? nullptr : split ? static_cast<const void*>(rd->LS) : rd->LF32;
     a.Vf = f64 ? static_cast<const void*>(rd->Vf64) : static_cast<const void*>(rd->Vf32);
-    a.fmask = rd->fmask;
+    a.fmask = f64 ? rd->symRows : rd->fmask;
     a.bcq = (m->bcq && m->bc_nvar == nvar) ? m->bcq : nullptr;
     a.ax = d->ax;
     a.ay = d->ay;

@@ -18,10 +18,12 @@ namespace dg {
 // reference-element operators resident on the device (one per order N)
 struct RefDev {
     RefElem re;
-    double *VqF64 = nullptr, *PF64 = nullptr, *LF64 = nullptr, *Vf64 = nullptr;
+    double* Vf64 = nullptr;
     float *VqF32 = nullptr, *PF32 = nullptr, *LF32 = nullptr, *Vf32 = nullptr;
     uint32_t *VqS = nullptr, *PS = nullptr, *LS = nullptr;   // bf16x3 split fragments
     int* fmask = nullptr;
+    double* symF = nullptr;    // FP64 stage kernel: mirror-half fragments and node rows a | b << 8 (stage_sym.hip)
+    int* symRows = nullptr;
     // projection-solver operators (built on first use): Pr Vq, Ps Vq, Lift, Dr, Ds in FP64
     double *insSr = nullptr, *insSs = nullptr, *insLift = nullptr, *insDr = nullptr, *insDs = nullptr;
     ~RefDev();

@@ -279,6 +279,27 @@ static void matmul(int m, int k, int n, const real* A, const real* B, real* C) {
         }
 }
 
+// Pairs the points (r, s) with their mirror images (s, r): pairs first, then the points on the axis.
+static bool mirror_rows(const rvec& r, const rvec& s, std::vector<int>& a, std::vector<int>& b, int& npair) {
+    const int n = int(r.size());
+    std::vector<int> axis;
+    for (int i = 0; i < n; ++i) {
+        int j = -1;
+        for (int k = 0; k < n && j < 0; ++k)
+            if (std::fabs(r[k] - s[i]) < 1e-12L && std::fabs(s[k] - r[i]) < 1e-12L) j = k;
+        if (j < 0) return false;
+        if (j == i) axis.push_back(i);
+        else if (i < j) {
+            a.push_back(i);
+            b.push_back(j);
+        }
+    }
+    npair = int(a.size());
+    a.insert(a.end(), axis.begin(), axis.end());
+    b.insert(b.end(), axis.begin(), axis.end());
+    return 2 * npair + int(axis.size()) == n;
+}
+
 bool build_refelem(int N, RefElem& re) {
     if (N < 1 || N > 8) return false;
     const int order = 3 * (N + 1);
@@ -365,6 +386,32 @@ bool build_refelem(int N, RefElem& re) {
                 En[re.fmask[f * Nfp + a] * (3 * Nfp) + f * Nfp + b] += m1;
             }
     matmul(Np, Np, 3 * Nfp, invM.data(), En.data(), LiftN.data());
+
+    // mirror halves of Vq, Pr (whose rows a, b give Ps as well: Ps[a,p] = Pr[b,p']) and Lift
+    {
+        RefElem::Mirror& mi = re.mirror;
+        if (!mirror_rows(r, s, mi.a, mi.b, mi.npair) || !mirror_rows(cr, cs, mi.pa, mi.pb, mi.qpair)) return false;
+        mi.nrow = int(mi.a.size());
+        mi.qrow = int(mi.pa.size());
+        for (int p = 0; p < mi.qrow; ++p)
+            for (int i = 0; i < mi.nrow; ++i) {
+                const real va = Vq[size_t(mi.pa[p]) * Np + mi.a[i]], vb = Vq[size_t(mi.pa[p]) * Np + mi.b[i]];
+                mi.Ve.push_back(double(i < mi.npair ? 0.5L * (va + vb) : 0.5L * va));
+                if (p < mi.qpair && i < mi.npair) mi.Vo.push_back(double(0.5L * (va - vb)));
+            }
+        for (int i = 0; i < mi.nrow; ++i) {
+            for (int q = 0; q < Nq; ++q) {
+                const real pa = Pr[size_t(mi.a[i]) * Nq + q], pb = Pr[size_t(mi.b[i]) * Nq + q];
+                mi.Pe.push_back(double(0.5L * (pa + pb)));
+                if (i < mi.npair) mi.Po.push_back(double(0.5L * (pa - pb)));
+            }
+            for (int c = 0; c < 3 * Nfq; ++c) {
+                const real la = Lift[size_t(mi.a[i]) * 3 * Nfq + c], lb = Lift[size_t(mi.b[i]) * 3 * Nfq + c];
+                mi.Le.push_back(double(0.5L * (la + lb)));
+                if (i < mi.npair) mi.Lo.push_back(double(0.5L * (la - lb)));
+            }
+        }
+    }
 
     // TVB limiter: mean = (V^-1 u)_0 psi_0; the P1 part keeps the modes (0,0), (0,1), (1,0) of the
     // (i, j) ordering, i.e. indices 0, 1, N+1; edge midpoints of edges 0, 1, 2 in (r, s)

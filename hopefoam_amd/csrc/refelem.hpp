@@ -23,6 +23,16 @@ struct RefElem {
     std::vector<double> Pr, Ps;          // Np x Nq : M^-1 Drq^T diag(cw), M^-1 Dsq^T diag(cw)
     std::vector<double> Lift;            // Np x (3*Nfq): M^-1 E_f Vf^T diag(gw)
     std::vector<double> LiftN;           // Np x (3*Nfp): M^-1 E (face mass on the face nodes), strong form
+    // mirror halves (r <-> s) of the operators, formed in long double: node rows i = (a, b) with b the mirror of a,
+    // pairs first, then the nodes on the axis (b = a); point rows likewise.  Every array has the row count of its
+    // name's kind; an axis node's sum is twice its value, its difference 0 (stage_sym.hip).
+    struct Mirror {
+        int npair = 0, nrow = 0, qpair = 0, qrow = 0;
+        std::vector<int> a, b, pa, pb;
+        std::vector<double> Ve, Vo;      // qrow x nrow, qpair x npair: value at pa = Ve sums + Vo differences
+        std::vector<double> Pe, Po;      // nrow x Nq, npair x Nq: half sum / difference of rows a, b of Pr
+        std::vector<double> Le, Lo;      // nrow x 3 Nfq, npair x 3 Nfq: the same of Lift
+    } mirror;
     // TVB limiter operators
     std::vector<double> tvb_p4;          // 4 x Np: cell mean, then the P1 part at the edge midpoints
     std::vector<double> tvb_phi;         // Np x 3: P1 functions with phi_i(m_k) = delta_ik at the nodes

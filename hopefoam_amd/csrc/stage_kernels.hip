@@ -1,4 +1,4 @@
-// DG right-hand side + fused LSERK4 stage kernels for gfx950 (CDNA4).
+// DG right-hand side + fused LSERK4 stage kernels for gfx950 (CDNA4), FP32 and bf16x3 (FP64: stage_sym.hip).
 //
 // One wavefront owns 16 elements (one per MFMA column).  Per element e the kernel evaluates
 // the reference's over-integrated weak form
@@ -28,47 +28,10 @@
 #include "dg_common.hpp"
 #include "lds_stage.hpp"
 #include "lim_moments.hpp"
+#include "stage_device.hpp"
 #include "stage_kernels.hpp"
 
 namespace dg {
-
-typedef double d4_t __attribute__((ext_vector_type(4)));
-typedef float f4_t __attribute__((ext_vector_type(4)));
-
-template <typename T>
-struct Vec4;
-template <>
-struct Vec4<double> { typedef d4_t type; };
-template <>
-struct Vec4<float> { typedef f4_t type; };
-
-// Row of the 16x16 accumulator held in register r of a lane of row group rg (= lane / 16).
-template <typename T>
-struct RowMap {
-    __host__ __device__ static constexpr int row(int rg, int r) { return dg::mfma_row<T>(rg, r); }
-};
-
-__device__ __forceinline__ d4_t mfma4(double a, double b, d4_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f4_t mfma4(float a, float b, f4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// Reciprocal and square root of the flux arithmetic.  FP64: the square root correctly rounded; the reciprocal
-// v_rcp_f64 refined by two Newton steps r += r (1 - x r) in fused multiply-adds (each step squares the relative
-// error, so the result is within an ulp of 1 / x), five instructions instead of the eleven of an IEEE division
-// (the densities it is taken of are positive and normal).  FP32: the hardware's v_rcp_f32 / v_sqrt_f32 (about
-// 1 ulp), far below the FP32 and bf16x3 paths' contraction round-off, in one instruction instead of the ten of an
-// IEEE division or square root.
-__device__ __forceinline__ double inv(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(fma(-x, r, 1.0), r, r);
-    return fma(fma(-x, r, 1.0), r, r);
-}
-__device__ __forceinline__ float inv(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double fsqrt(double x) { return sqrt(x); }
-__device__ __forceinline__ float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
 // ---------------------------------------------------------------- bf16x3 split products
 // x = hi + lo with hi = bf16(x) and lo = bf16(x - hi), both rounded to nearest even, so the pair carries about
@@ -101,104 +64,6 @@ __device__ __forceinline__ f4_t mfma3(const uint4 A, const Split4& B, f4_t c) {
     c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(al, B.h, c, 0, 0, 0);
     c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, B.l, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, B.h, c, 0, 0, 0);
-}
-
-// ---------------------------------------------------------------- physics
-template <int PHYS, typename T>
-struct VolumeFlux;
-
-template <typename T>
-struct VolumeFlux<PHYS_ADVECT, T> {
-    static constexpr int NV = 1;
-    __device__ static void eval(const T* q, T ax, T ay, T, T rx, T ry, T sx, T sy, T* fr, T* fs) {
-        const T F = ax * q[0], G = ay * q[0];
-        fr[0] = rx * F + ry * G;
-        fs[0] = sx * F + sy * G;
-    }
-};
-
-// dgEulerFoam.C:81-90: gther_U = rhoU / rho, gther_p = (gamma-1)(E - rho |U|^2 / 2); volume
-// terms div(U rho), div(U rhoU) + grad(p), div(U E) + div(U p).  Formed directly in the reference directions:
-// with the contravariant momenta m_r = rx rhou + ry rhov, m_s = sx rhou + sy rhov and U_r = m_r / rho,
-//   rx F + ry G = (m_r, rhou U_r + p rx, rhov U_r + p ry, (E + p) U_r),  likewise for s,
-// the same values as rx F + ry G of the Cartesian fluxes in about half the operations.
-template <typename T>
-struct VolumeFlux<PHYS_EULER, T> {
-    static constexpr int NV = 4;
-    __device__ static void eval(const T* q, T, T, T gamma, T rx, T ry, T sx, T sy, T* fr, T* fs) {
-        const T ru = q[1], rv = q[2], E = q[3];
-        const T irho = inv(q[0]);
-        const T p = (gamma - T(1)) * (E - T(0.5) * ((ru * ru + rv * rv) * irho));
-        const T mr = rx * ru + ry * rv, ms = sx * ru + sy * rv;
-        const T Ur = mr * irho, Us = ms * irho, Ep = E + p;
-        fr[0] = mr;
-        fr[1] = ru * Ur + p * rx;
-        fr[2] = rv * Ur + p * ry;
-        fr[3] = Ep * Ur;
-        fs[0] = ms;
-        fs[1] = ru * Us + p * sx;
-        fs[2] = rv * Us + p * sy;
-        fs[3] = Ep * Us;
-    }
-};
-
-// Roe flux in the face-normal frame without entropy fix (RoeFlux.C:109-181); M = own side, P = other.
-template <typename T>
-__device__ __forceinline__ void roe_flux(T g, T nx, T ny, const T* M, const T* P, T* F) {
-    const T QP2 = nx * P[1] + ny * P[2], QM2 = nx * M[1] + ny * M[2];
-    const T QP3 = nx * P[2] - ny * P[1], QM3 = nx * M[2] - ny * M[1];
-    const T rhoP = P[0], rhoM = M[0];
-    const T uM = QM2 / rhoM, uP = QP2 / rhoP, vM = QM3 / rhoM, vP = QP3 / rhoP;
-    const T pM = (g - T(1)) * (M[3] - T(0.5) * (QM2 * uM + QM3 * vM));
-    const T pP = (g - T(1)) * (P[3] - T(0.5) * (QP2 * uP + QP3 * vP));
-    const T HM = (M[3] + pM) / rhoM, HP = (P[3] + pP) / rhoP;
-    T fr = (QM2 + QP2) / T(2);
-    T fu = (QM2 * uM + pM + QP2 * uP + pP) / T(2);
-    T fv = (QM3 * uM + QP3 * uP) / T(2);
-    T fe = (uM * (M[3] + pM) + uP * (P[3] + pP)) / T(2);
-    const T rMs = sqrt(rhoM), rPs = sqrt(rhoP);
-    const T rhob = rMs * rPs;
-    const T u = (rMs * uM + rPs * uP) / (rMs + rPs);
-    const T v = (rMs * vM + rPs * vP) / (rMs + rPs);
-    const T H = (rMs * HM + rPs * HP) / (rMs + rPs);
-    const T c2 = (g - T(1)) * (H - T(0.5) * (u * u + v * v));
-    const T c = sqrt(fabs(c2));
-    const T dw1 = (T(-0.5) * rhob * (uP - uM) / c + T(0.5) * (pP - pM) / c2) * fabs(u - c);
-    const T dw2 = ((rhoP - rhoM) - (pP - pM) / c2) * fabs(u);
-    const T dw3 = (rhob * (vP - vM)) * fabs(u);
-    const T dw4 = (T(0.5) * rhob * (uP - uM) / c + T(0.5) * (pP - pM) / c2) * fabs(u + c);
-    fr -= (dw1 + dw2 + dw4) / T(2);
-    fu -= (dw1 * (u - c) + dw2 * u + dw4 * (u + c)) / T(2);
-    fv -= (dw1 * v + dw2 * v + dw3 + dw4 * v) / T(2);
-    fe -= (dw1 * (H - u * c) + dw2 * (u * u + v * v) / T(2) + dw3 * v + dw4 * (H + u * c)) / T(2);
-    F[0] = fr;
-    F[1] = nx * fu - ny * fv;
-    F[2] = ny * fu + nx * fv;
-    F[3] = fe;
-}
-
-// local Lax-Friedrichs (Rusanov) flux with pointwise |u.n| + c
-template <typename T>
-__device__ __forceinline__ void llf_flux(T g, T nx, T ny, const T* M, const T* P, T* F) {
-    const T iM = inv(M[0]), iP = inv(P[0]);
-    const T uM = M[1] * iM, vM = M[2] * iM, uP = P[1] * iP, vP = P[2] * iP;
-    const T pM = (g - T(1)) * (M[3] - T(0.5) * M[0] * (uM * uM + vM * vM));
-    const T pP = (g - T(1)) * (P[3] - T(0.5) * P[0] * (uP * uP + vP * vP));
-    const T unM = uM * nx + vM * ny, unP = uP * nx + vP * ny;
-    const T lM = fabs(unM) + fsqrt(fabs(g * pM * iM)), lP = fabs(unP) + fsqrt(fabs(g * pP * iP));
-    const T lam = lM > lP ? lM : lP;
-    const T FM[4] = {M[0] * unM, M[1] * unM + pM * nx, M[2] * unM + pM * ny, (M[3] + pM) * unM};
-    const T FP[4] = {P[0] * unP, P[1] * unP + pP * nx, P[2] * unP + pP * ny, (P[3] + pP) * unP};
-#pragma unroll
-    for (int v = 0; v < 4; ++v) F[v] = T(0.5) * (FM[v] + FP[v]) + T(0.5) * lam * (M[v] - P[v]);
-}
-
-// ---------------------------------------------------------------- stage kernel
-// Orders a wave's LDS writes before its later LDS reads by other lanes of the same wave.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Persistent blocks, one per CU: 8 waves (2 per SIMD) for FP32 up to N = 6, else 4 waves with the
@@ -237,29 +102,6 @@ struct StageLds {
     static constexpr size_t elems = trace_elems + (pf_lds ? nP : 0) + (vq_lds ? nV : 0) + (lf_lds ? nL : 0);
 };
 
-
-// Other side's face nodes of variable rg for face f of element e (connectivity c): neighbour nodes in reversed
-// order, or fixedValue ghost nodes.  The Nfp loads are issued with no branch around them: a face without such
-// data (its flux copies the own trace) reads a valid address of its own element, and the caller drops the values
-// (the return value says whether they are used), so the loads of several faces can be in flight together.
-template <int N, int NV, typename OT>
-__device__ __forceinline__ bool gather_face(const StageArgs& a, int c, int f, int e, int rg, OT (&o)[N + 1]) {
-    constexpr int Np = (N + 1) * (N + 2) / 2, Nfp = N + 1;
-    constexpr size_t GS = size_t(NV) * Np * 16;
-    const int v = rg < NV ? rg : 0;
-    const bool nb = c >= 0;
-    const bool fx = !nb && -c - 1 == BC_FIXED && a.bcq != nullptr;
-    const int en = nb ? c >> 2 : e, fn = nb ? c & 3 : 0;
-    const double* qn = a.q_in + size_t(en >> 4) * GS + size_t(v) * Np * 16 + (en & 15);
-    const double* bq = fx ? a.bcq + ((size_t(v) * a.K + e) * 3 + f) * Nfp : qn;
-#pragma unroll
-    for (int k = 0; k < Nfp; ++k) {
-        const int node = fn == 0 ? face_node<N>(0, N - k) : (fn == 1 ? face_node<N>(1, N - k) : face_node<N>(2, N - k));
-        const double* src = fx ? bq + k : qn + node * 16;   // one load from the selected address
-        o[k] = OT(*src);
-    }
-    return nb || fx;
-}
 
 // SPLIT: bf16x3 split products for the three contractions (T = float for everything else)
 template <int N, int PHYS, typename T, bool SPLIT, bool MOM>
@@ -479,10 +321,9 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
                 for (int v = 0; v < NV; ++v) qc[v] = mfma4(A, qb[v][s], qc[v]);
             }
         }
-        // unrolled in full for FP64 up to N = 6 (at N = 6 its stage measured 7 % shorter; beyond, it spills); the
-        // bf16x3 kernel spills unrolled in full and gained nothing unrolled by two, the two-wave FP32 kernel spills
-        constexpr int kTileUnroll = (sizeof(T) == 8 && N <= 6) ? D::QT : 1;
-#pragma unroll kTileUnroll
+        // not unrolled: the bf16x3 kernel spills unrolled in full and gained nothing unrolled by two, the two-wave
+        // FP32 kernel spills
+#pragma unroll 1
         for (int t = 0; t < D::QT; ++t) {
             const int tn = t + 1 < D::QT ? t + 1 : D::QT + D::FT - 1;   // last step: a face tile (harmless)
 #pragma unroll
@@ -566,7 +407,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
         double* __restrict__ res_g = a.res + gbase;
         // bf16x3 update (the full register file of one wave per SIMD; up to 8 tile-variables, 128 VGPRs): the
         // residual and q_in of every output tile are requested here, before the faces, and arrive while the face
-        // work runs.  (The FP32 kernel would spill them and reads them in the update; FP64 holds its own.)
+        // work runs.  (The FP32 kernel would spill them and reads them in the update.)
         constexpr bool kHoist = sizeof(T) == 4 && WPB == 4 && D::MT * NV <= 8;
         constexpr int MH = kHoist ? D::MT : 1;
         double rmh[MH][4][NV], qmh[MH][4][NV];
@@ -586,10 +427,10 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
 
         // ---- faces.  The other side's face nodes of all three faces (lane (col, rg): variable rg) are requested
         // together, so their latency is paid once and behind other work rather than once per face: bf16x3 requests
-        // them at the group start (above) and holds them through the volume phase; FP64, short of registers for
-        // that (it would spill), before the own-trace MFMAs below.  With one wave per SIMD (FP64, bf16x3) the face
-        // geometry comes with them and the nodes stay FP64 until used; the two-wave FP32 kernel, short of
-        // registers, converts the nodes as they arrive and loads each face's geometry when it gets there.
+        // them at the group start (above) and holds them through the volume phase, FP32 with one wave per SIMD before
+        // the own-trace MFMAs below.  With one wave per SIMD the face geometry comes with them and the nodes stay FP64
+        // until used; the two-wave FP32 kernel, short of registers, converts the nodes as they arrive and loads each
+        // face's geometry when it gets there.
         if (kWide && !SPLIT && (NV == 4 || rg < NV)) {
 #pragma unroll
             for (int f = 0; f < 3; ++f) keep[f] = gather_face<N, NV>(a, cn[f], f, e, rg, oth[f]);
@@ -604,13 +445,9 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
         }
         // Own traces at the face Gauss points come out of the interpolation GEMM (face tiles:
         // register r of tile tf holds lift K step 4 tf + r, Gauss point 4 (step % SF) + rg).
-        // (FP64 forms them later, in the face loop, from the lanes' own nodal values shuffled within each element's
-        // four lanes and Vf: a quarter of the flops of the face tiles, on the VALU, which takes as long per f64 flop
-        // as the matrix pipe, the kernel's busiest unit)
-        constexpr bool kOwnValu = sizeof(T) == 8;
-        T4 own[kOwnValu ? 1 : D::FT][NV];
+        T4 own[D::FT][NV];
 #pragma unroll
-        for (int tf = 0; tf < (kOwnValu ? 0 : D::FT); ++tf) {
+        for (int tf = 0; tf < D::FT; ++tf) {
 #pragma unroll
             for (int v = 0; v < NV; ++v) own[tf][v] = T4{0, 0, 0, 0};
             if constexpr (SPLIT) {
@@ -632,19 +469,6 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
         if (!kWide && (NV == 4 || rg < NV)) {   // FP32: after the own-trace MFMAs, whose accumulators are live
 #pragma unroll
             for (int f = 0; f < 3; ++f) keep[f] = gather_face<N, NV>(a, cn[f], f, e, rg, oth[f]);
-        }
-        // FP64: residual registers for the stage update, requested before the face work that hides them
-        // (the FP32 kernel has no register room for them and reads them in the update)
-        constexpr bool kPrefetchRes = sizeof(T) == 8;
-        double rold[NV][kPrefetchRes ? D::KS1 : 1];
-        if (kPrefetchRes && a.mode != 0) {
-#pragma unroll
-            for (int v = 0; v < NV; ++v)
-#pragma unroll
-                for (int s = 0; s < D::KS1; ++s) {
-                    const int node = gemm1_node<T>(s, rg);
-                    rold[v][s] = node < Np ? a.res[size_t(grp) * GS + (v * Np + node) * 16 + col] : 0.0;
-                }
         }
         T F0[NV], G0[NV];   // SPLIT: physical flux of the constant state, for its normal flux on the faces
         if constexpr (SPLIT) VF::eval(q0, ax, ay, gamma, T(1), T(0), T(0), T(1), F0, G0);
@@ -673,17 +497,6 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
             wave_sync();
             const T nx = fnx[fg], ny = fny[fg], fsc = ffs[fg];
             const bool copy_own = cn[f] < 0 && -cn[f] - 1 != BC_FIXED;
-            // FP64: the element's own nodes on face f, from the lanes of its row groups (node n sits in row group
-            // n % 4 at K step n / 4); every lane takes part in the shuffles
-            T fnode[kOwnValu ? NV : 1][kOwnValu ? Nfp : 1];
-            if constexpr (kOwnValu) {
-#pragma unroll
-                for (int k = 0; k < Nfp; ++k) {
-                    const int node = face_node<N>(f, k);
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) fnode[v][k] = __shfl(qb[v][node >> 2], col + 16 * (node & 3), 64);
-                }
-            }
 #pragma unroll
             for (int j = 0; j < SF; ++j) {
                 const int st = f * SF + j;
@@ -693,20 +506,8 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
                 for (int v = 0; v < NV; ++v) bf[v] = T(0);
                 if (g < Nfq) {
                     T qM[NV], qP[NV], Fs[NV];
-                    if constexpr (kOwnValu) {   // the own trace at Gauss point g
 #pragma unroll
-                        for (int v = 0; v < NV; ++v) qM[v] = T(0);
-#pragma unroll
-                        for (int k = 0; k < Nfp; ++k) {
-                            const T w = Vf[g * Nfp + k];
-#pragma unroll
-                            for (int v = 0; v < NV; ++v) qM[v] += w * fnode[v][k];
-                        }
-                    } else {
-#pragma unroll
-                        for (int v = 0; v < NV; ++v)
-                            qM[v] = SPLIT ? own[st / 4][v][st % 4] + q0[v] : own[st / 4][v][st % 4];
-                    }
+                    for (int v = 0; v < NV; ++v) qM[v] = SPLIT ? own[st / 4][v][st % 4] + q0[v] : own[st / 4][v][st % 4];
 #pragma unroll
                     for (int v = 0; v < NV; ++v) {
                         qP[v] = copy_own ? qM[v] : tr[g * TR_G + v * 16 + col];
@@ -788,14 +589,10 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
             double rm[4][NV], qm[4][NV];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int s = 4 * m + r;
                 const int j = 16 * m + RowMap<T>::row(rg, r);
 #pragma unroll
                 for (int v = 0; v < NV; ++v) {
-                    if (kPrefetchRes) {
-                        rm[r][v] = s < D::KS1 ? rold[v][s < D::KS1 ? s : 0] : 0.0;
-                        qm[r][v] = s < D::KS1 ? double(qb[v][s < D::KS1 ? s : 0]) : 0.0;
-                    } else if (kHoist) {
+                    if (kHoist) {
                         rm[r][v] = rmh[m < MH ? m : 0][r][v];
                         qm[r][v] = qmh[m < MH ? m : 0][r][v];
                     } else if (a.mode != 0) {
@@ -888,7 +685,7 @@ static hipError_t launch_n(int N, const StageArgs& a, int ncu, hipStream_t st) {
 template <int PHYS>
 static hipError_t launch_prec(int N, int prec, const StageArgs& a, int ncu, hipStream_t st) {
     switch (prec) {
-        case PREC_FP64: return launch_n<PHYS, double>(N, a, ncu, st);
+        case PREC_FP64: return launch_stage_sym(N, PHYS, a, ncu, st);
         case PREC_FP32: return launch_n<PHYS, float>(N, a, ncu, st);
         case PREC_BF16X3: return launch_n<PHYS, float, true>(N, a, ncu, st);
         default: return hipErrorInvalidValue;

@@ -30,6 +30,9 @@ struct StageArgs {
 };
 
 hipError_t launch_stage(int N, int phys, int prec, const StageArgs& a, int ncu, hipStream_t st);
+// the FP64 stage on the mirror halves of the operators (stage_sym.hip): VqF the fragments in stage_sym.hpp's order,
+// fmask the node rows (a | b << 8, padded to whole K steps)
+hipError_t launch_stage_sym(int N, int phys, const StageArgs& a, int ncu, hipStream_t st);
 hipError_t launch_field_diff(const double* a, const double* b, double* out, size_t n, int ncu, hipStream_t st);
 hipError_t launch_mfma_layout_probe(double* out, hipStream_t st);
 hipError_t launch_mfma_probe(const double* A, const double* B, double* D64, const float* Af, const float* Bf,
