@@ -178,6 +178,15 @@ __device__ __forceinline__ void llf_flux(T g, T nx, T ny, const T* M, const T* P
 }
 
 // ---------------------------------------------------------------- stage kernel
+// A value at a wavefront-uniform base plus an unsigned byte offset of the lane: one scalar base and one 32-bit register,
+// where a signed element index makes the compiler keep a 64-bit address per access.
+__device__ __forceinline__ double at_lane(const double* base, unsigned off) {
+    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off);
+}
+__device__ __forceinline__ void put_lane(double* base, unsigned off, double x) {
+    *reinterpret_cast<double*>(reinterpret_cast<char*>(base) + off) = x;
+}
+
 // Orders a wave's LDS writes before its later LDS reads by other lanes of the same wave.
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -66,12 +66,19 @@ __device__ __forceinline__ f4_t mfma3(const uint4 A, const Split4& B, f4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, B.h, c, 0, 0, 0);
 }
 
-// Persistent blocks, one per CU: 8 waves (2 per SIMD) for FP32 up to N = 6, else 4 waves with the
-// full 512-register budget each (the bf16x3 kernel holds its split operands and shifted fluxes in registers:
-// at two waves per SIMD it spills, measured 14 % slower at N = 6).  When they fit, the operator fragments are
-// staged into LDS once per block and shared by its waves.
+// Persistent blocks: 8 waves (2 per SIMD) up to N = 6, else 4 waves with the full 512-register budget each.  With one
+// flux and one mode per instantiation and scalar group addresses neither kernel spills at two waves per SIMD (with both
+// fluxes in one kernel FP32 spilled 32 registers and bf16x3 needed 456).  Measured, LF, K = 131072, N = 6: FP32 251 ->
+// 172 us, bf16x3 150 us with one wave per SIMD, 134 with two (146 before).  A block's waves take groups apart, so that
+// every compute unit gets one before any gets two: K = 11834, N = 6 FP32 50.8 -> 25.8 us, bf16x3 23.3 -> 20.8 us.  When
+// they fit, the operator fragments are staged into LDS once per block and shared by its waves.
 template <int N, typename T, bool SPLIT = false>
-constexpr int waves_per_block() { return (N <= 6 && sizeof(T) == 4 && !SPLIT) ? 8 : 4; }
+constexpr int waves_per_block() { return N <= 6 ? 8 : 4; }
+
+// wavefronts per SIMD that the scheduler may aim at: no more than the block brings (the LDS holds one block), so that
+// it does not trade the batching of loads for an occupancy that cannot be had; small kernels as many as fit
+template <int N, int PHYS, typename T, bool SPLIT>
+constexpr int stage_per_simd() { return PHYS == PHYS_EULER && N >= 3 ? waves_per_block<N, T, SPLIT>() / 4 : 8; }
 
 template <int N, int NV, typename T, bool SPLIT>
 struct StageLds {
@@ -104,8 +111,10 @@ struct StageLds {
 
 
 // SPLIT: bf16x3 split products for the three contractions (T = float for everything else)
-template <int N, int PHYS, typename T, bool SPLIT, bool MOM>
-__global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_kernel(StageArgs a) {
+template <int N, int PHYS, typename T, bool SPLIT, bool MOM, int FLUX, bool UPDATE>
+__global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
+    __attribute__((amdgpu_waves_per_eu(1, stage_per_simd<N, PHYS, T, SPLIT>())))
+    void stage_kernel(StageArgs a) {
     using D = Dims<N>;
     using T4 = typename Vec4<T>::type;
     using VF = VolumeFlux<PHYS, T>;
@@ -131,9 +140,12 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
         for (int i = threadIdx.x; i < kMomFrag; i += blockDim.x) p4l[i] = a.p4f[i];
 
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    // in a scalar register: a group's addresses are then a scalar base and a lane offset
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15;   // element within the group
     const int rg = lane >> 4;    // row group of the 16x16 tiles
+    // byte offsets of the lane in a group's node rows: K step order (row 4 s + rg) and accumulator order (row 4 rg + r)
+    const unsigned lane8 = lane * 8u, row8 = (rg * 64u + col) * 8u;
     const int K = a.K;
     const int groups = (K + 15) >> 4;
     const T* __restrict__ VqF = static_cast<const T*>(a.VqF);
@@ -183,7 +195,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
     // by the next group, and since vector memory operations complete in order, waiting for any of them early
     // would also wait for the DMA.
     const int gstride = nbx * WPB;
-    int grp = g_lo + bx * WPB + wave;
+    int grp = g_lo + wave * nbx + bx;   // a block's wavefronts nbx groups apart: a small mesh spreads over the chip first
     int cn_next[3] = {0, 0, 0};
     T geo_next[4] = {T(0), T(0), T(0), T(0)};
     if (grp < g_hi) {
@@ -228,13 +240,19 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
 
         // B fragments of the interpolation GEMM (coalesced loads); they are also this lane's rows of q_in
         T qb[NV][D::KS1];
+        {
+            double qd[NV][D::KS1];   // every load before the first conversion (scheduled one by one they serialise)
 #pragma unroll
-        for (int v = 0; v < NV; ++v)
+            for (int v = 0; v < NV; ++v)
 #pragma unroll
-            for (int s = 0; s < D::KS1; ++s) {
-                const int node = gemm1_node<T>(s, rg);
-                qb[v][s] = node < Np ? T(qg[(v * Np + node) * 16 + col]) : T(0);
-            }
+                for (int s = 0; s < D::KS1; ++s)
+                    qd[v][s] = gemm1_node<T>(s, rg) < Np ? at_lane(qg + (v * Np + 4 * s) * 16, lane8) : 0.0;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+#pragma unroll
+                for (int s = 0; s < D::KS1; ++s) qb[v][s] = T(qd[v][s]);
+        }
 
         // bf16x3: the contractions see the state and the fluxes relative to the element's constant state q0 (its
         // node 0).  This is exact: interpolation reproduces constants (qc = q0 + Vq (q - q0)), and the constant
@@ -244,7 +262,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
         T q0[NV], fr0[NV], fs0[NV];
         if constexpr (SPLIT) {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) q0[v] = T(qg[(v * Np) * 16 + col]);
+            for (int v = 0; v < NV; ++v) q0[v] = T(at_lane(qg + v * Np * 16, col * 8u));
             VF::eval(q0, ax, ay, gamma, rx, ry, sx, sy, fr0, fs0);
         }
         // the other side's face nodes and the face geometry (the face phase below says when each kernel asks)
@@ -267,6 +285,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
         }
         if constexpr (L::prefetch) {
             // every lane's reads of the buffer have returned before the DMA of the next group overwrites it
+            __builtin_amdgcn_sched_barrier(0);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (more) {
                 dma_to_lds<L::qpre_bytes>(a.q_in + size_t(grp + gstride) * GS, qpre + wave * (L::qpre_bytes / 8),
@@ -321,8 +340,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
                 for (int v = 0; v < NV; ++v) qc[v] = mfma4(A, qb[v][s], qc[v]);
             }
         }
-        // not unrolled: the bf16x3 kernel spills unrolled in full and gained nothing unrolled by two, the two-wave
-        // FP32 kernel spills
+        // not unrolled: both kernels spill
 #pragma unroll 1
         for (int t = 0; t < D::QT; ++t) {
             const int tn = t + 1 < D::QT ? t + 1 : D::QT + D::FT - 1;   // last step: a face tile (harmless)
@@ -405,25 +423,20 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
         const double* __restrict__ qin_g = a.q_in + gbase;
         double* __restrict__ out_g = a.q_out + gbase;
         double* __restrict__ res_g = a.res + gbase;
-        // bf16x3 update (the full register file of one wave per SIMD; up to 8 tile-variables, 128 VGPRs): the
-        // residual and q_in of every output tile are requested here, before the faces, and arrive while the face
-        // work runs.  (The FP32 kernel would spill them and reads them in the update.)
-        constexpr bool kHoist = sizeof(T) == 4 && WPB == 4 && D::MT * NV <= 8;
-        constexpr int MH = kHoist ? D::MT : 1;
-        double rmh[MH][4][NV], qmh[MH][4][NV];
-        if (kHoist && a.mode != 0) {
+        double rmh[D::MT][4][NV], qmh[D::MT][4][NV];   // residual and q_in of the update
+        auto load_update = [&]() {
 #pragma unroll
-            for (int m = 0; m < MH; ++m)
+            for (int m = 0; m < D::MT; ++m)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int j = 16 * m + RowMap<T>::row(rg, r);
 #pragma unroll
                     for (int v = 0; v < NV; ++v) {
-                        rmh[m][r][v] = j < Np ? res_g[(v * Np + j) * 16 + col] : 0.0;
-                        qmh[m][r][v] = j < Np ? qin_g[(v * Np + j) * 16 + col] : 0.0;
+                        rmh[m][r][v] = j < Np ? at_lane(res_g + (v * Np + 16 * m + r) * 16, row8) : 0.0;
+                        qmh[m][r][v] = j < Np ? at_lane(qin_g + (v * Np + 16 * m + r) * 16, row8) : 0.0;
                     }
                 }
-        }
+        };
 
         // ---- faces.  The other side's face nodes of all three faces (lane (col, rg): variable rg) are requested
         // together, so their latency is paid once and behind other work rather than once per face: bf16x3 requests
@@ -466,7 +479,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
                 }
             }
         }
-        if (!kWide && (NV == 4 || rg < NV)) {   // FP32: after the own-trace MFMAs, whose accumulators are live
+        if (!kWide && !SPLIT && (NV == 4 || rg < NV)) {   // FP32: after the own-trace MFMAs, whose accumulators are live
 #pragma unroll
             for (int f = 0; f < 3; ++f) keep[f] = gather_face<N, NV>(a, cn[f], f, e, rg, oth[f]);
         }
@@ -480,7 +493,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
 #pragma unroll
         for (int f = 0; f < 3; ++f) {
             const int fg = f;
-            if constexpr (!kWide) {
+            if constexpr (!kWide && !SPLIT) {
                 fnx[f] = geo[(G_NX0 + 3 * f) * K + e];
                 fny[f] = geo[(G_NY0 + 3 * f) * K + e];
                 ffs[f] = geo[(G_FS0 + 3 * f) * K + e];
@@ -517,15 +530,21 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
                         qP[1] -= T(2) * mn * nx;
                         qP[2] -= T(2) * mn * ny;
                     }
-                    if (PHYS == PHYS_ADVECT) {   // upwind, or the central "average" flux without the |vn| term
+                    // the flux as a unit of its own: operands and results pass through registers as they are, so that the
+                    // compiler forms the same fused multiply-adds whatever surrounds it
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) asm volatile("" : "+v"(qM[v]), "+v"(qP[v]));
+                    if constexpr (PHYS == PHYS_ADVECT) {   // upwind, or the central "average" flux without the |vn| term
                         const T vn = nx * ax + ny * ay;
                         const T diss = a.flux == FLUX_AVERAGE ? T(0) : fabs(vn);
                         Fs[0] = (vn * qM[0] + vn * qP[0]) * T(0.5) + diss * (qM[0] - qP[0]) * T(0.5);
-                    } else if (a.flux == FLUX_ROE) {
+                    } else if constexpr (FLUX == FLUX_ROE) {
                         roe_flux<T>(gamma, nx, ny, qM, qP, Fs);
                     } else {
                         llf_flux<T>(gamma, nx, ny, qM, qP, Fs);
                     }
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) asm volatile("" : "+v"(Fs[v]));
                     if constexpr (SPLIT) {   // minus the constant state's normal flux
 #pragma unroll
                         for (int v = 0; v < NV; ++v) Fs[v] -= F0[v] * nx + G0[v] * ny;
@@ -571,13 +590,13 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
 
-        // ---- output in the field layout: rows j = 16m + row(rg, r) of column col.  For FP64, node j is
-        // gemm1_node(4m + r, rg), whose q_in this lane holds in qb and whose residual it prefetched.
+        // ---- output in the field layout: rows j = 16m + row(rg, r) of column col.
         // bf16x3 with a moments output: K step s = 4 m + r of the f64 moment product takes row group rg's row
         // 16 m + 4 rg + r = node lim_mnode(s, rg), the new state this lane has just formed, in the moments kernel's
-        // order and with its fragments (so the two give the same bits); rows beyond Np enter as zeros.  (Only the
-        // one-wave-per-SIMD bf16x3 kernel has the registers for the accumulators; FP32 and FP64 leave the moments to
-        // the limiter's own kernel.)
+        // order and with its fragments (so the two give the same bits); rows beyond Np enter as zeros.  (FP32 and FP64
+        // leave the moments to the limiter's own kernel.)
+        // every load of the update before its first store: the compiler keeps loads behind stores that could alias
+        if constexpr (UPDATE) load_update();
         const bool want_mom = kMom;   // the launcher takes this instantiation for a moments output and an update
         double mpart[kMom ? NV : 1][4];   // the moments' per-lane partial sums (lim_moments.hpp)
 #pragma unroll
@@ -586,21 +605,6 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
             for (int k = 0; k < 4; ++k) mpart[v][k] = 0.0;
 #pragma unroll
         for (int m = 0; m < D::MT; ++m) {
-            double rm[4][NV], qm[4][NV];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int j = 16 * m + RowMap<T>::row(rg, r);
-#pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    if (kHoist) {
-                        rm[r][v] = rmh[m < MH ? m : 0][r][v];
-                        qm[r][v] = qmh[m < MH ? m : 0][r][v];
-                    } else if (a.mode != 0) {
-                        rm[r][v] = j < Np ? res_g[(v * Np + j) * 16 + col] : 0.0;
-                        qm[r][v] = j < Np ? qin_g[(v * Np + j) * 16 + col] : 0.0;
-                    }
-                }
-            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int j = 16 * m + RowMap<T>::row(rg, r);
@@ -610,15 +614,15 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
                 if (j < Np) {   // padding columns (e_raw >= K) keep evolving a copy of element K-1
 #pragma unroll
                     for (int v = 0; v < NV; ++v) {
-                        const int idx = (v * Np + j) * 16 + col;
+                        const int row = (v * Np + 16 * m + r) * 16;
                         const double rhs = double(acc[v][m][r]);
-                        if (a.mode == 0) {
-                            out_g[idx] = rhs;
+                        if constexpr (!UPDATE) {
+                            put_lane(out_g + row, row8, rhs);
                         } else {
-                            const double rn = a.rk_a * rm[r][v] + a.dt * rhs;
-                            res_g[idx] = rn;
-                            qnew[v] = qm[r][v] + a.rk_b * rn;
-                            out_g[idx] = qnew[v];
+                            const double rn = a.rk_a * rmh[m][r][v] + a.dt * rhs;
+                            put_lane(res_g + row, row8, rn);
+                            qnew[v] = qmh[m][r][v] + a.rk_b * rn;
+                            put_lane(out_g + row, row8, qnew[v]);
                         }
                     }
                 }
@@ -638,33 +642,42 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>())) void stage_k
 
 // Persistent grid: as many blocks as the device keeps resident at once (a multiple of 8 so that every
 // XCD gets the same share), capped by the number of element groups.
-template <int N, int PHYS, typename T, bool SPLIT, bool MOM>
+template <int N, int PHYS, typename T, bool SPLIT, bool MOM, int FLUX, bool UPDATE>
 static hipError_t launch_inst(const StageArgs& a, int ncu, hipStream_t st) {
     constexpr int threads = 64 * waves_per_block<N, T, SPLIT>();
     static int per_cu = -1;
     if (per_cu < 0) {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, stage_kernel<N, PHYS, T, SPLIT, MOM>, threads, 0) !=
-            hipSuccess)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, stage_kernel<N, PHYS, T, SPLIT, MOM, FLUX, UPDATE>, threads,
+                                                         0) != hipSuccess)
             n = 1;
         per_cu = n < 1 ? 1 : n;
     }
     const int groups = (a.K + 15) / 16;
-    const int wpb = waves_per_block<N, T, SPLIT>();
-    int nb = (groups + wpb - 1) / wpb;
-    if (nb > ncu * per_cu) nb = ncu * per_cu;
+    int nb = groups < ncu * per_cu ? groups : ncu * per_cu;
     nb = nb < 8 ? 8 : (nb + 7) / 8 * 8;
     if (a.block_cap > 0 && nb > a.block_cap) nb = a.block_cap < 8 ? 8 : a.block_cap / 8 * 8;
-    hipLaunchKernelGGL((stage_kernel<N, PHYS, T, SPLIT, MOM>), dim3(nb), dim3(threads), 0, st, a);
+    hipLaunchKernelGGL((stage_kernel<N, PHYS, T, SPLIT, MOM, FLUX, UPDATE>), dim3(nb), dim3(threads), 0, st, a);
     return hipGetLastError();
+}
+
+template <int N, int PHYS, typename T, bool SPLIT, int FLUX>
+static hipError_t launch_flux(const StageArgs& a, int ncu, hipStream_t st) {
+    if (a.mode == 0) return launch_inst<N, PHYS, T, SPLIT, false, FLUX, false>(a, ncu, st);
+    if constexpr (SPLIT) {
+        if (a.mom_out != nullptr) return launch_inst<N, PHYS, T, SPLIT, true, FLUX, true>(a, ncu, st);
+    }
+    return launch_inst<N, PHYS, T, SPLIT, false, FLUX, true>(a, ncu, st);
 }
 
 template <int N, int PHYS, typename T, bool SPLIT>
 static hipError_t launch_one(const StageArgs& a, int ncu, hipStream_t st) {
-    if constexpr (SPLIT) {
-        if (a.mom_out != nullptr && a.mode != 0) return launch_inst<N, PHYS, T, SPLIT, true>(a, ncu, st);
+    if constexpr (PHYS == PHYS_ADVECT) {
+        return launch_flux<N, PHYS, T, SPLIT, FLUX_UPWIND>(a, ncu, st);
+    } else {
+        return a.flux == FLUX_ROE ? launch_flux<N, PHYS, T, SPLIT, FLUX_ROE>(a, ncu, st)
+                                  : launch_flux<N, PHYS, T, SPLIT, FLUX_LF>(a, ncu, st);
     }
-    return launch_inst<N, PHYS, T, SPLIT, false>(a, ncu, st);
 }
 
 template <int PHYS, typename T, bool SPLIT = false>

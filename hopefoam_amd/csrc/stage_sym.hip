@@ -131,19 +131,13 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
         na[s] = ((ab & 255u) * 16 + col) * 8;
         if (s < KO) nb[s < KO ? s : 0] = ((ab >> 8) * 16 + col) * 8;
     }
-    auto at = [](const double* base, unsigned off) {
-        return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off);
-    };
-    auto put = [](double* base, unsigned off, double x) {
-        *reinterpret_cast<double*>(reinterpret_cast<char*>(base) + off) = x;
-    };
     auto load_nodes = [&](const double* src, double (&x)[NV][KE], double (&y)[NV][KO]) {
 #pragma unroll
         for (int v = 0; v < NV; ++v)
 #pragma unroll
             for (int s = 0; s < KE; ++s) {
-                x[v][s] = at(src + v * Np * 16, na[s]);
-                if (s < KO) y[v][s < KO ? s : 0] = at(src + v * Np * 16, nb[s < KO ? s : 0]);
+                x[v][s] = at_lane(src + v * Np * 16, na[s]);
+                if (s < KO) y[v][s < KO ? s : 0] = at_lane(src + v * Np * 16, nb[s < KO ? s : 0]);
             }
     };
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the fragments and the first group have landed
@@ -232,7 +226,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
                 for (int v = 0; v < NV; ++v) {
                     double be, bo;
                     if constexpr (kLds) {
-                        const double x = at(qw + v * Np * 16, na[s]), y = s < KO ? at(qw + v * Np * 16, nb[so]) : x;
+                        const double x = at_lane(qw + v * Np * 16, na[s]), y = s < KO ? at_lane(qw + v * Np * 16, nb[so]) : x;
                         be = x + y;
                         bo = x - y;
                     } else {
@@ -400,6 +394,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
             load_nodes(qn, ua, ub);
         }
         if constexpr (kLds) {
+            __builtin_amdgcn_sched_barrier(0);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads of the buffer have returned
             if (grp + gstride < g_hi)
                 dma_to_lds_whole<GS * sizeof(double)>(a.q_in + size_t(grp + gstride) * GS, qw, lane);
@@ -414,18 +409,18 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
                 const bool on = 4 * s + 3 < D::nrow || 4 * s + rg < D::nrow;
                 const bool pair = s < KO && (4 * s + 3 < D::npair || 4 * s + rg < D::npair);
                 if constexpr (!UPDATE) {
-                    if (on) put(ov, na[s], E + O);
-                    if (pair) put(ov, nb[so], E - O);
+                    if (on) put_lane(ov, na[s], E + O);
+                    if (pair) put_lane(ov, nb[so], E - O);
                 } else {
                     const double r1 = a.rk_a * ra[v][s] + a.dt * (E + O);
                     if (on) {
-                        put(rv, na[s], r1);
-                        put(ov, na[s], ua[v][s] + a.rk_b * r1);
+                        put_lane(rv, na[s], r1);
+                        put_lane(ov, na[s], ua[v][s] + a.rk_b * r1);
                     }
                     if (pair) {
                         const double r2 = a.rk_a * rb[v][so] + a.dt * (E - O);
-                        put(rv, nb[so], r2);
-                        put(ov, nb[so], ub[v][so] + a.rk_b * r2);
+                        put_lane(rv, nb[so], r2);
+                        put_lane(ov, nb[so], ub[v][so] + a.rk_b * r2);
                     }
                 }
             }
