@@ -360,6 +360,7 @@ int dgh_destroy(dgh_ctx c) {
     c->sipg.clear();
     c->mlps.clear();
     c->ens.clear();
+    c->staging.release();
     (void)hipEventDestroy(c->ev0);
     (void)hipEventDestroy(c->ev1);
     (void)hipStreamDestroy(c->stream);
@@ -629,38 +630,32 @@ int dgh_field_destroy(dgh_ctx c, int fh) {
     return DGH_OK;
 }
 
-// host [var][K][Np] <-> device layout (dev_index in dg_common.hpp); padding repeats element K-1
+// host [var][K][Np] <-> device layout (transfer.cpp); padding repeats element K-1
+static int field_transfer(dgh_ctx c, FieldDev* f, double* host, bool to_device) {
+    (void)hipSetDevice(c->device);
+    NodalArray a;
+    a.dev = f->d;
+    a.nvar = f->nvar;
+    a.K = f->K;
+    a.Np = f->Np;
+    a.groups = round_up(f->K, 16) / 16;
+    return c->hip(transfer_array(c->device, c->stream, c->staging, a, host, to_device), to_device ? "upload" : "download")
+               ? DGH_OK
+               : c->last;
+}
+
 int dgh_field_upload(dgh_ctx c, int fh, const double* host) {
     if (!c || !host) return DGH_ERR_ARG;
     FieldDev* f = c->field(fh);
     if (!f) return c->last;
-    const int Kp = round_up(f->K, 16);
-    std::vector<double> dev(f->n);
-    for (int v = 0; v < f->nvar; ++v)
-        for (int e = 0; e < Kp; ++e) {
-            const double* src = host + (size_t(v) * f->K + std::min(e, f->K - 1)) * f->Np;
-            for (int n = 0; n < f->Np; ++n) dev[dev_index(e, v, n, f->nvar, f->Np)] = src[n];
-        }
-    if (!c->hip(hipMemcpyAsync(f->d, dev.data(), f->n * sizeof(double), hipMemcpyHostToDevice, c->stream), "upload") ||
-        !c->hip(hipStreamSynchronize(c->stream), "upload sync"))
-        return c->last;
-    return DGH_OK;
+    return field_transfer(c, f, const_cast<double*>(host), true);
 }
 
 int dgh_field_download(dgh_ctx c, int fh, double* host) {
     if (!c || !host) return DGH_ERR_ARG;
     FieldDev* f = c->field(fh);
     if (!f) return c->last;
-    std::vector<double> dev(f->n);
-    if (!c->hip(hipMemcpyAsync(dev.data(), f->d, f->n * sizeof(double), hipMemcpyDeviceToHost, c->stream), "download") ||
-        !c->hip(hipStreamSynchronize(c->stream), "download sync"))
-        return c->last;
-    for (int v = 0; v < f->nvar; ++v)
-        for (int e = 0; e < f->K; ++e) {
-            double* dst = host + (size_t(v) * f->K + e) * f->Np;
-            for (int n = 0; n < f->Np; ++n) dst[n] = dev[dev_index(e, v, n, f->nvar, f->Np)];
-        }
-    return DGH_OK;
+    return field_transfer(c, f, host, false);
 }
 
 int dgh_field_copy(dgh_ctx c, int dst, int src) {

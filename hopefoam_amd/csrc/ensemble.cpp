@@ -381,24 +381,14 @@ extern "C" int dgh_ensemble_destroy(dgh_ctx c, int h) {
 // host [K][Np] <-> device group layout of one nodal array of case i
 static int ens_copy(dgh_ctx c, EnsDev& E, int i, int array, double* host, bool to_device) {
     const EnsHostCase& h = E.hc[i];
-    const size_t n = size_t(h.Kp) * h.Np;
-    std::vector<double> buf(n, 0.0);
-    double* dptr = E.data + E.cases[i].off_u + size_t(array) * n;
-    if (to_device) {
-        for (int e = 0; e < h.Kp; ++e)
-            for (int j = 0; j < h.Np; ++j)
-                buf[dev_index(e, 0, j, 1, h.Np)] = host[size_t(std::min(e, h.K - 1)) * h.Np + j];
-        if (!c->hip(hipMemcpyAsync(dptr, buf.data(), n * sizeof(double), hipMemcpyHostToDevice, c->stream), "upload") ||
-            !c->hip(hipStreamSynchronize(c->stream), "sync"))
-            return c->last;
-    } else {
-        if (!c->hip(hipMemcpyAsync(buf.data(), dptr, n * sizeof(double), hipMemcpyDeviceToHost, c->stream), "download") ||
-            !c->hip(hipStreamSynchronize(c->stream), "sync"))
-            return c->last;
-        for (int e = 0; e < h.K; ++e)
-            for (int j = 0; j < h.Np; ++j) host[size_t(e) * h.Np + j] = buf[dev_index(e, 0, j, 1, h.Np)];
-    }
-    return DGH_OK;
+    NodalArray a;
+    a.dev = E.data + E.cases[i].off_u + size_t(array) * h.Kp * h.Np;
+    a.K = h.K;
+    a.Np = h.Np;
+    a.groups = h.Kp / 16;
+    return c->hip(transfer_array(c->device, c->stream, c->staging, a, host, to_device), to_device ? "upload" : "download")
+               ? DGH_OK
+               : c->last;
 }
 
 extern "C" int dgh_ensemble_set(dgh_ctx c, int h, int i, const double* u) {

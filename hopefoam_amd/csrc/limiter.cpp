@@ -420,23 +420,14 @@ int dg_limit_fused_moments(dgh_ctx c, MeshDev* m, const dgh_rhs_desc* d, const d
 // the flags and the count of a limiter call (flags, count: its device arrays) to the host
 static int limit_results(dgh_ctx c, const dgh_lim_desc* d, int K, const int* flags, const unsigned* count,
                          int* troubled, int* ntroubled) {
-    if (troubled &&
-        !c->hip(hipMemcpyAsync(troubled, flags, size_t(K) * sizeof(int), hipMemcpyDeviceToHost, c->stream),
-                "troubled download"))
-        return c->last;
+    if (!troubled && !ntroubled) return DGH_OK;
     const bool every_cell = d->kind == DGH_LIM_ALL || d->kind == DGH_LIM_TRIANGLE;   // count = K, not counted
-    if (ntroubled && every_cell) {
-        if (!c->hip(hipStreamSynchronize(c->stream), "sync")) return c->last;
-        *ntroubled = K;
-    } else if (ntroubled) {
-        unsigned n = 0;
-        if (!c->hip(hipMemcpyAsync(&n, count, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream), "count") ||
-            !c->hip(hipStreamSynchronize(c->stream), "sync"))
-            return c->last;
-        *ntroubled = int(n);
-    } else if (troubled && !c->hip(hipStreamSynchronize(c->stream), "sync")) {
+    unsigned n = unsigned(K);
+    if (!c->hip(fetch_small(c->stream, c->staging, troubled, troubled ? flags : nullptr, size_t(K) * sizeof(int), &n,
+                            ntroubled && !every_cell ? count : nullptr, sizeof n),
+                "limiter results"))
         return c->last;
-    }
+    if (ntroubled) *ntroubled = int(n);
     return DGH_OK;
 }
 

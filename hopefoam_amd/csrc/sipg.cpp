@@ -48,6 +48,7 @@ struct SipgDev {
     SipgOps<double> d;
     SipgOps<float> s;
     bool have32 = false;
+    double* bdata[2] = {nullptr, nullptr};   // Dirichlet and Neumann data of sipg_rhs, allocated when first given
     double* part = nullptr;
     CgState* st = nullptr;       // [4]: the iteration's two states, the published state, auxiliary norms
     double* part_b[2] = {nullptr, nullptr};   // the update kernel's partials by iteration parity (part holds the
@@ -555,19 +556,20 @@ int dgh_sipg_rhs_neumann(dgh_ctx c, int h, int f, const double* gbc, const doubl
     if (f == b) return c->fail(DGH_ERR_ARG, "dgh_sipg_rhs: f and b must differ"), DGH_ERR_ARG;
     (void)hipSetDevice(c->device);
     const size_t n = size_t(S->K) * 3 * (S->N + 1);
+    // the boundary data's device buffers stay with the handle: an allocation and a free per call cost more than the
+    // kernel
     double* dg[2] = {nullptr, nullptr};
     const double* host[2] = {gbc, gnb};
     bool ok = true;
     for (int i = 0; i < 2 && ok; ++i) {
         if (!host[i]) continue;
-        ok = c->hip(hipMalloc(reinterpret_cast<void**>(&dg[i]), n * sizeof(double)), "hipMalloc boundary data") &&
-             c->hip(hipMemcpyAsync(dg[i], host[i], n * sizeof(double), hipMemcpyHostToDevice, c->stream),
+        ok = (S->bdata[i] || dev_alloc(c, *S, &S->bdata[i], n)) &&
+             c->hip(hipMemcpyAsync(S->bdata[i], host[i], n * sizeof(double), hipMemcpyHostToDevice, c->stream),
                     "boundary data upload");
+        dg[i] = S->bdata[i];
     }
     ok = ok && c->hip(sipg_rhs(S->N, sipg_args(*S, S->d), ff->d, dg[0], dg[1], fb->d, c->stream), "sipg rhs") &&
          c->hip(hipStreamSynchronize(c->stream), "sync");
-    for (double* p : dg)
-        if (p) (void)hipFree(p);
     return ok ? DGH_OK : c->last;
 }
 

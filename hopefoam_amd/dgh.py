@@ -462,7 +462,7 @@ class Field:
         c._ck(c.L.dgh_field_upload(c.h, self.h, a.reshape(-1)), "dgh_field_upload")
 
     def download(self):
-        out = np.zeros(self.nvar * self.mesh.K * self.mesh.Np)
+        out = np.empty(self.nvar * self.mesh.K * self.mesh.Np)
         c = self.mesh.ctx
         c._ck(c.L.dgh_field_download(c.h, self.h, out), "dgh_field_download")
         return out.reshape(self.shape)
@@ -596,7 +596,7 @@ class Ensemble:
     def get(self, i, what=0):
         c = self.cases[i]
         n = c["K"] * c["Np"] * (2 if what == 2 else 1)
-        out = np.zeros(n)
+        out = np.empty(n)
         self.ctx._ck(self.ctx.L.dgh_ensemble_get(self.ctx.h, self.h, i, what, out), "dgh_ensemble_get")
         return out.reshape((2, c["K"], c["Np"]) if what == 2 else (c["K"], c["Np"]))
 
