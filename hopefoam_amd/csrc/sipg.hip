@@ -257,8 +257,10 @@ __device__ __forceinline__ void trace_group(const T* __restrict__ sA, const T (&
             if (item < NFQ3) {
                 const int f = item / Nfq;
                 const T dn = select3(f, ar0, ar1, ar2) * acc[TI + t][r] + select3(f, as0, as1, as2) * acc[2 * TI + t][r];
-                trace[trace_index(g, item, 0, j, NFQ3)] = acc[t][r];
-                trace[trace_index(g, item, 1, j, NFQ3)] = dn;
+                T* tg = trace + (size_t(g) * NFQ3 + 16 * t) * 32;   // the group's tile of items (trace_index)
+                const unsigned at = (item - 16 * t) * 32 + j;
+                tg[at] = acc[t][r];
+                tg[at + 16] = dn;
             }
         }
 }
@@ -272,7 +274,8 @@ __global__ __launch_bounds__(256) void sipg_trace_kernel(SipgArgs<T> a, const T*
     __shared__ T sA[3 * TI * KS * 64];
     for (int i = threadIdx.x; i < 3 * TI * KS * 64; i += 256) sA[i] = a.TrF[i];
     __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, j = lane & 15;
+    const int kq = lane >> 4;
     const int groups = (a.K + 15) >> 4;
     for (int g = blockIdx.x * 4 + wave; g < groups; g += gridDim.x * 4) {
         const size_t base = size_t(g) * Np * 16;
@@ -287,50 +290,57 @@ __global__ __launch_bounds__(256) void sipg_trace_kernel(SipgArgs<T> a, const T*
     }
 }
 
-// What the update kernel reads of one group ahead of the CG scalars (lane: element lane % 16, nodes 4 s + lane / 16
-// < Np; other entries unset): the inputs of the chain r -> u = B r -> traces (r, w, S p; init: rhs in r, and w), the
-// point-Jacobi diagonal or the element's inverse-block index, and the face geometry of the traces.  The rest (u, p,
-// x) is read when needed: nothing downstream waits for the p and x updates.
+// What the update kernel reads of one group ahead of the CG scalars (lane: element lane % 16, nodes 4 s + lane / 16 < Np,
+// which is value 64 s + lane of the group; other entries unset): every vector it updates, the point-Jacobi diagonal or
+// the element's inverse-block index, and the face geometry of the traces.  All of it before the first store: the
+// compiler keeps a load behind a store that could alias, so a load between the stores of p, S p, x and r costs one
+// memory latency per K step.
 template <typename T, int KS>
 struct UpdateIn {
-    T w[KS], ap[KS], r[KS], d[KS];
+    T w[KS], ap[KS], r[KS], d[KS], u[KS], p[KS], x[KS];
     T fg[6];
     int bt;
 };
 
-template <int N, typename T, bool BLOCK>
-__device__ __forceinline__ void update_load(const SipgArgs<T>& a, const CgLoop<T>& c, int init, int g, int lane,
+template <int N, typename T, bool BLOCK, bool INIT>
+__device__ __forceinline__ void update_load(const SipgArgs<T>& a, const CgLoop<T>& c, int g, int lane,
                                             UpdateIn<T, SipgTiles(N).KS>& in) {
     constexpr SipgTiles S(N);
     constexpr int Np = S.Np, KS = S.KS;
-    const int j = lane & 15, kq = lane >> 4;
     const size_t base = size_t(g) * Np * 16;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-        const int k = 4 * s + kq;
-        if (k < Np) {
-            const size_t idx = base + size_t(k) * 16 + j;
-            in.w[s] = c.w[idx];
-            if (init) {
-                in.r[s] = c.rhs[idx];
-            } else {
-                in.ap[s] = c.ap[idx];
-                in.r[s] = c.r[idx];
-            }
-            if constexpr (!BLOCK) in.d[s] = c.dinv[idx];
+        if (4 * s + (lane >> 4) >= Np) continue;
+        const size_t at = base + 64 * s;
+        in.w[s] = c.w[at + lane];
+        if constexpr (INIT) {
+            in.r[s] = c.rhs[at + lane];
+        } else {
+            in.ap[s] = c.ap[at + lane];
+            in.r[s] = c.r[at + lane];
+            in.u[s] = c.u[at + lane];
+            in.p[s] = c.p[at + lane];
+            in.x[s] = c.x[at + lane];
         }
+        if constexpr (!BLOCK) in.d[s] = c.dinv[at + lane];
     }
-    if constexpr (BLOCK) in.bt = c.bidx[g * 16 + j];   // padded to whole groups
+    if constexpr (BLOCK) in.bt = c.bidx[g * 16 + (lane & 15)];   // padded to whole groups
     load_face_geo<T>(a, g, lane, in.fg);
 }
 
 // The update kernel of PCG iteration i (Chronopoulos & Gear; one wavefront per group as in the trace kernel):
 // finishes the previous reduction (cg_advance), then p = u + beta p, ap = w + beta ap (p = u, ap = w in the first
-// iteration), x += alpha p, r -= alpha ap, u = B r with its face traces, and the u.u, r.u partials.  init: only
+// iteration), x += alpha p, r -= alpha ap, u = B r with its face traces, and the u.u, r.u partials.  INIT: only
 // r = rhs - w, u = B r, traces and partials (w = S x on entry).  B = diag(dinv) (point Jacobi) or the element's
-// block inverse binv[bidx[e]] applied from a per-wavefront LDS copy of the group's r.
-template <int N, typename T, bool BLOCK>
-__global__ __launch_bounds__(256, N <= 6 ? 2 : 1) void cg_update_kernel(SipgArgs<T> a, CgLoop<T> c, int init,
+// block inverse binv[bidx[e]] as matrix products, one for each distinct block of the group.
+// A chip-sized mesh gives each wavefront one group, so the kernel is one chain: the reduction, the group's loads, the
+// products, the stores.  What shortens it is having every load of the group in flight before the first store and
+// per-lane addresses of 32 bits beside a scalar base (order 5, 32768 elements, FP64, per iteration with the apply
+// kernel: block Jacobi 34.2 -> 32.2 us, point Jacobi 32.7 -> 31.5; FP32 corrections 26.2 -> 23.1; order 3, 2640
+// elements: 13.4 -> 12.8).  Requesting the group's first two inverse blocks ahead of the reduction as well costs more in
+// registers than it hides (order 5: 33.3, order 6: 22.2 -> 24.1).
+template <int N, typename T, bool BLOCK, bool INIT>
+__global__ __launch_bounds__(256, N <= 6 ? 2 : 1) void cg_update_kernel(SipgArgs<T> a, CgLoop<T> c,
                                                         const CgState* __restrict__ st_in, CgState* __restrict__ st_out,
                                                         const double* __restrict__ pb_in, double* __restrict__ pb_out) {
     constexpr SipgTiles S(N);
@@ -341,23 +351,25 @@ __global__ __launch_bounds__(256, N <= 6 ? 2 : 1) void cg_update_kernel(SipgArgs
     constexpr size_t kTrBytes = size_t(3 * TI * KS * 64) * sizeof(T);
     __shared__ __attribute__((aligned(16))) T sA[dma_span(kTrBytes) / sizeof(T)];
     const int nb = gridDim.x;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, j = lane & 15;
+    const int kq = lane >> 4;
     const int groups = (a.K + 15) >> 4;
     // The trace fragments (LDS DMA) and the first group's inputs do not depend on the CG scalars: they are
     // requested before the reduction that yields them, so the latencies overlap.
     dma_stage_to_lds<kTrBytes>(sA, a.TrF);
     const int g0 = blockIdx.x * 4 + wave;
     UpdateIn<T, KS> in;
-    if (g0 < groups) update_load<N, T, BLOCK>(a, c, init, g0, lane, in);
-    cg_advance(st_in, st_out, pb_in, c.part_a, nb, init ? CG_FINISH_NONE : CG_FINISH_AUTO, ls);
+    if (g0 < groups) update_load<N, T, BLOCK, INIT>(a, c, g0, lane, in);
+    cg_advance(st_in, st_out, pb_in, c.part_a, nb, INIT ? CG_FINISH_NONE : CG_FINISH_AUTO, ls);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the fragments have landed (and no DMA outlives the block)
     if (ls.done) return;
     __syncthreads();
-    const bool first = !init && ls.its == 0;
-    const T alpha = init ? T(0) : T(ls.alpha), bc = T(ls.bcoef);
+    // first iteration: p = u, S p = w (bcoef is 0, and what p and S p hold is not looked at)
+    const bool first = !INIT && ls.its == 0;
+    const T alpha = INIT ? T(0) : T(ls.alpha), bc = T(ls.bcoef);
     double acc[2] = {0.0, 0.0};
     for (int g = g0; g < groups; g += gridDim.x * 4) {
-        if (g != g0) update_load<N, T, BLOCK>(a, c, init, g, lane, in);
+        if (g != g0) update_load<N, T, BLOCK, INIT>(a, c, g, lane, in);
         const size_t base = size_t(g) * Np * 16;
         const int e = g * 16 + j;
         const bool live = e < a.K;
@@ -367,23 +379,23 @@ __global__ __launch_bounds__(256, N <= 6 ? 2 : 1) void cg_update_kernel(SipgArgs
             const int k = 4 * s + kq;
             rv[s] = T(0);
             if (k < Np) {
-                const size_t idx = base + size_t(k) * 16 + j;
+                const size_t idx = base + 64 * s + lane;
                 T r;
-                if (init) {
+                if constexpr (INIT) {
                     r = in.r[s] - in.w[s];
                 } else {
-                    const T av = first ? in.w[s] : in.w[s] + bc * in.ap[s];
-                    // one rounding (fused), whatever the compiler makes of the init branch beside it
+                    const T ap = first ? T(0) : in.ap[s], p = first ? T(0) : in.p[s];
+                    const T av = fma(bc, ap, in.w[s]), pv = fma(bc, p, in.u[s]);
                     r = fma(-alpha, av, in.r[s]);
-                    const T pv = first ? c.u[idx] : c.u[idx] + bc * c.p[idx];
                     c.p[idx] = pv;
                     c.ap[idx] = av;
-                    c.x[idx] += alpha * pv;
+                    c.x[idx] = fma(alpha, pv, in.x[s]);
                 }
                 c.r[idx] = r;
                 rv[s] = r;
             }
         }
+        __builtin_amdgcn_sched_barrier(0);   // the inputs are done with before the products' operands come in
         if constexpr (BLOCK) {
             // u = B_t r for each distinct inverse block t of the group, on the matrix cores: r is already in
             // B-fragment layout and the fragments' row order puts output node 4 s' + kq in register s' % 4 of
@@ -395,14 +407,15 @@ __global__ __launch_bounds__(256, N <= 6 ? 2 : 1) void cg_update_kernel(SipgArgs
             for (;;) {
                 const unsigned long long todo = __ballot(!mine);
                 if (todo == 0ull) break;
-                const int t = __shfl(bt, __ffsll(static_cast<long long>(todo)) - 1, 64);
-                const T* F = c.binv + size_t(t) * MT * KS * 64 + lane;
+                const int t =
+                    __builtin_amdgcn_readfirstlane(__shfl(bt, __ffsll(static_cast<long long>(todo)) - 1, 64));
+                const T* F = c.binv + size_t(t) * MT * KS * 64;
                 V4 bacc[MT];
 #pragma unroll
                 for (int m = 0; m < MT; ++m) {
                     bacc[m] = V4{T(0), T(0), T(0), T(0)};
 #pragma unroll
-                    for (int s = 0; s < KS; ++s) bacc[m] = smfma(F[(m * KS + s) * 64], rv[s], bacc[m]);
+                    for (int s = 0; s < KS; ++s) bacc[m] = smfma(F[(m * KS + s) * 64 + lane], rv[s], bacc[m]);
                 }
                 if (bt == t) {
                     mine = true;
@@ -421,13 +434,14 @@ __global__ __launch_bounds__(256, N <= 6 ? 2 : 1) void cg_update_kernel(SipgArgs
         for (int s = 0; s < KS; ++s) {
             const int k = 4 * s + kq;
             if (k < Np) {
-                c.u[base + size_t(k) * 16 + j] = ub[s];
+                c.u[base + 64 * s + lane] = ub[s];
                 if (live) {
                     acc[0] += double(ub[s]) * double(ub[s]);
                     acc[1] += double(ub[s]) * double(rv[s]);
                 }
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
         trace_group<N, T>(sA, ub, in.fg, g, lane, c.trace);
     }
     write_partials<2>(acc, pb_out);
@@ -495,7 +509,8 @@ __global__ __launch_bounds__(256, N <= 6 ? 2 : 1) void sipg_apply_kernel(SipgArg
     typedef typename SV4<T>::type V4;
     constexpr size_t kApBytes = size_t(MT * KA * 64) * sizeof(T);
     __shared__ __attribute__((aligned(16))) T sA[dma_span(kApBytes) / sizeof(T)];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, j = lane & 15;
+    const int kq = lane >> 4;
     const int groups = (a.K + 15) >> 4;
     // The fragments (LDS DMA) and the first group's inputs are requested before anything waits, so their latencies
     // overlap (a finished CG state reads them for nothing, once).
@@ -749,18 +764,18 @@ hipError_t sipg_rhs(int N, const SipgArgs<double>& a, const double* f, const dou
 }
 
 // the update kernel: reads state st_in and partials pb_in (+ the apply's), writes st_out and pb_out
-template <typename T>
-static hipError_t cg_update_launch(int N, const SipgArgs<T>& a, const CgLoop<T>& c, int init, const CgState* st_in,
+template <bool INIT, typename T>
+static hipError_t cg_update_launch(int N, const SipgArgs<T>& a, const CgLoop<T>& c, const CgState* st_in,
                                    CgState* st_out, const double* pb_in, double* pb_out, hipStream_t s) {
     if (c.binv) {
 #define CALL(n)                                                                                                      \
-    hipLaunchKernelGGL((cg_update_kernel<n, T, true>), dim3(sipg_blocks(a)), dim3(256), 0, s, a, c, init, st_in, \
+    hipLaunchKernelGGL((cg_update_kernel<n, T, true, INIT>), dim3(sipg_blocks(a)), dim3(256), 0, s, a, c, st_in, \
                        st_out, pb_in, pb_out)
         DG_SIPG_DISPATCH(N, CALL)
 #undef CALL
     } else {
 #define CALL(n)                                                                                                       \
-    hipLaunchKernelGGL((cg_update_kernel<n, T, false>), dim3(sipg_blocks(a)), dim3(256), 0, s, a, c, init, st_in, \
+    hipLaunchKernelGGL((cg_update_kernel<n, T, false, INIT>), dim3(sipg_blocks(a)), dim3(256), 0, s, a, c, st_in, \
                        st_out, pb_in, pb_out)
         DG_SIPG_DISPATCH(N, CALL)
 #undef CALL
@@ -770,7 +785,7 @@ static hipError_t cg_update_launch(int N, const SipgArgs<T>& a, const CgLoop<T>&
 
 template <typename T>
 hipError_t cg_start(int N, const SipgArgs<T>& a, const CgLoop<T>& c, hipStream_t s) {
-    hipError_t err = cg_update_launch<T>(N, a, c, 1, c.st + 1, c.st, c.part_b[0], c.part_b[1], s);
+    hipError_t err = cg_update_launch<true, T>(N, a, c, c.st + 1, c.st, c.part_b[0], c.part_b[1], s);
     if (err != hipSuccess) return err;
     return sipg_apply_only<T>(N, a, c.u, c.trace, c.w, 1, c.st, c.part_a, s);
 }
@@ -778,7 +793,7 @@ hipError_t cg_start(int N, const SipgArgs<T>& a, const CgLoop<T>& c, hipStream_t
 template <typename T>
 hipError_t cg_iteration(int N, const SipgArgs<T>& a, const CgLoop<T>& c, int i, hipStream_t s) {
     const int q = i & 1;
-    hipError_t err = cg_update_launch<T>(N, a, c, 0, c.st + q, c.st + (q ^ 1), c.part_b[q ^ 1], c.part_b[q], s);
+    hipError_t err = cg_update_launch<false, T>(N, a, c, c.st + q, c.st + (q ^ 1), c.part_b[q ^ 1], c.part_b[q], s);
     if (err != hipSuccess) return err;
     return sipg_apply_only<T>(N, a, c.u, c.trace, c.w, 1, c.st + (q ^ 1), c.part_a, s);
 }
