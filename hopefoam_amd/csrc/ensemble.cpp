@@ -20,6 +20,9 @@ using namespace dg;
 
 namespace dg {
 
+// streams of an ensemble's orders: the hardware queues a process has by default
+static constexpr int kEnsChains = 4;
+
 static constexpr const double* kA = kLserkA;
 static constexpr const double* kB = kLserkB;
 
@@ -49,8 +52,24 @@ struct EnsDev {
     size_t ndata = 0;
     long long dofs = 0;
     std::map<long long, hipGraphExec_t> graphs;   // key: nsteps * 2 + starting buffer
+    // Orders are independent of each other from the first stage to the last, and one order's cases rarely fill the
+    // chip: they are dealt out to at most kEnsChains streams (chain[N]; chain 0 is the context's stream, the others
+    // are forked from it and joined to it by events within the call, under capture as well).  64 cases of orders 2 to 8,
+    // 5.3e6 values: 219 us per stage on one stream, 131 on four (158 launched without a graph).
+    int nchain = 1;
+    int chain[9] = {0};
+    hipStream_t side[kEnsChains] = {nullptr};
+    hipEvent_t forked = nullptr, joined[kEnsChains] = {nullptr};
     ~EnsDev() {
         (void)hipSetDevice(device);
+        for (hipStream_t s : side)
+            if (s) {
+                (void)hipStreamSynchronize(s);   // a call that failed half-way may not have joined it
+                (void)hipStreamDestroy(s);
+            }
+        if (forked) (void)hipEventDestroy(forked);
+        for (hipEvent_t e : joined)
+            if (e) (void)hipEventDestroy(e);
         for (auto& g : graphs) (void)hipGraphExecDestroy(g.second);
         for (void* p : {(void*)dcases, (void*)data, (void*)geo, (void*)conn, (void*)items})
             if (p) (void)hipFree(p);
@@ -174,8 +193,54 @@ static void ens_grids(dgh_ctx c, EnsDev& E) {
     }
 }
 
-// one LSERK4 stage (mode 1) or the right-hand side into res (mode 0), reading u buffer `cur`: per order,
-// the q pass then the right-hand-side pass over that order's cases (cases of different orders are independent)
+// Deals the orders out to the chains, the most expensive first, each to the chain with the least work: the cost of an
+// order is its groups of 16 elements per compute unit's four SIMDs (a started round counts whole) times the matrix
+// steps of both passes, and a constant for the two launches.
+static bool ens_chains(dgh_ctx c, EnsDev& E) {
+    std::vector<std::pair<double, int>> order;
+    for (int N = 1; N <= 8; ++N) {
+        if (!E.grid[N]) continue;
+        size_t groups = 0;
+        for (const EnsHostCase& h : E.hc)
+            if (h.N == N) groups += (h.K + 15) / 16;
+        const size_t rounds = (groups + 4 * c->ncu - 1) / (4 * c->ncu);
+        const int MT = ens_mfma_mt(N), KS = ens_mfma_ks(N), KSL = ens_mfma_ksl(N);
+        order.push_back({double(rounds) * MT * (4 * KS + 3 * KSL) + 120.0, N});
+    }
+    std::sort(order.rbegin(), order.rend());
+    double load[kEnsChains] = {0};
+    E.nchain = std::max(1, std::min(kEnsChains, int(order.size())));
+    for (const auto& o : order) {
+        const int k = int(std::min_element(load, load + E.nchain) - load);
+        E.chain[o.second] = k;
+        load[k] += o.first;
+    }
+    if (E.nchain > 1 && !E.forked && !c->hip(hipEventCreateWithFlags(&E.forked, hipEventDisableTiming), "event"))
+        return false;
+    for (int k = 1; k < E.nchain; ++k)
+        if (!E.side[k] && (!c->hip(hipStreamCreateWithFlags(&E.side[k], hipStreamNonBlocking), "stream") ||
+                           !c->hip(hipEventCreateWithFlags(&E.joined[k], hipEventDisableTiming), "event")))
+            return false;
+    return true;
+}
+
+static bool ens_fork(dgh_ctx c, EnsDev& E) {
+    if (E.nchain > 1 && !c->hip(hipEventRecord(E.forked, c->stream), "fork")) return false;
+    for (int k = 1; k < E.nchain; ++k)
+        if (!c->hip(hipStreamWaitEvent(E.side[k], E.forked, 0), "fork")) return false;
+    return true;
+}
+
+static bool ens_join(dgh_ctx c, EnsDev& E) {
+    bool ok = true;
+    for (int k = 1; k < E.nchain; ++k)
+        ok = c->hip(hipEventRecord(E.joined[k], E.side[k]), "join") &&
+             c->hip(hipStreamWaitEvent(c->stream, E.joined[k], 0), "join") && ok;
+    return ok;
+}
+
+// one LSERK4 stage (mode 1) or the right-hand side into res (mode 0), reading u buffer `cur`: per order, on its
+// chain's stream, the q pass then the right-hand-side pass over that order's cases
 static bool ens_stage(dgh_ctx c, EnsDev& E, int cur, int mode, double ra, double rb) {
     EnsArgs a = ens_args(E);
     a.cur = cur;
@@ -185,8 +250,9 @@ static bool ens_stage(dgh_ctx c, EnsDev& E, int cur, int mode, double ra, double
     for (int N = 1; N <= 8; ++N) {
         if (!E.grid[N]) continue;
         for (int x = 0; x < 9; ++x) a.chunk[x] = E.chunk[N][x];
-        if (!c->hip(launch_ens_q(N, E.split[N], a, E.grid[N], c->stream), "ensemble q pass") ||
-            !c->hip(launch_ens_rhs(N, E.split[N], a, E.grid[N], c->stream), "ensemble rhs pass"))
+        hipStream_t s = E.chain[N] ? E.side[E.chain[N]] : c->stream;
+        if (!c->hip(launch_ens_q(N, E.split[N], a, E.grid[N], s), "ensemble q pass") ||
+            !c->hip(launch_ens_rhs(N, E.split[N], a, E.grid[N], s), "ensemble rhs pass"))
             return false;
     }
     return true;
@@ -235,6 +301,7 @@ static bool ens_finalize_items(dgh_ctx c, EnsDev& E) {
     build_items(E, {}, E.split, items, E.chunk);
     if (!upload_items(c, E, items)) return false;
     ens_grids(c, E);
+    if (!ens_chains(c, E)) return false;
     for (auto& g : E.graphs) (void)hipGraphExecDestroy(g.second);
     E.graphs.clear();
     return true;
@@ -350,11 +417,9 @@ extern "C" int dgh_ensemble_create(dgh_ctx c, const dgh_ens_desc* d, int ncases,
                         fr[size_t(MT * KS + m * KS + st) * 64 + l] = re.Ds[size_t(i) * Np + j];
                     }
                 }
-                for (int st = 0; st < KSL; ++st) {
-                    const int j = 4 * st + k;
-                    if (i < Np && j < 3 * Nfp)
-                        fr[size_t(2 * MT * KS + m * KSL + st) * 64 + l] = re.LiftN[size_t(i) * 3 * Nfp + j];
-                }
+                for (int st = 0; st < KSL; ++st)   // lift: point st of face k
+                    if (i < Np && k < 3)
+                        fr[size_t(2 * MT * KS + m * KSL + st) * 64 + l] = re.LiftN[size_t(i) * 3 * Nfp + k * Nfp + st];
             }
         if (!c->upload(&E->ops[h.N], op) || !c->upload(&E->opsM[h.N], fr)) return c->last;
         E->split[h.N] = default_split(h.N);
@@ -419,7 +484,9 @@ extern "C" int dgh_ensemble_rhs(dgh_ctx c, int h) {
     EnsDev* E = ens_get(c, h);
     if (!E) return c->last;
     (void)hipSetDevice(c->device);
-    if (!ens_stage(c, *E, E->cur, 0, 0.0, 0.0) || !c->hip(hipStreamSynchronize(c->stream), "sync")) return c->last;
+    bool ok = ens_fork(c, *E) && ens_stage(c, *E, E->cur, 0, 0.0, 0.0);
+    ok = ens_join(c, *E) && ok;
+    if (!c->hip(hipStreamSynchronize(c->stream), "sync") || !ok) return c->last;
     return DGH_OK;
 }
 
@@ -434,12 +501,13 @@ extern "C" int dgh_ensemble_run(dgh_ctx c, int h, int nsteps, int use_graph, flo
     const int start = E->cur;
     auto record = [&](int cur0) {
         int cur = cur0;
-        for (int step = 0; step < nsteps; ++step)
-            for (int s = 0; s < 5; ++s) {
-                if (!ens_stage(c, *E, cur, 1, kA[s], kB[s])) return false;
+        bool ok = ens_fork(c, *E);
+        for (int step = 0; step < nsteps && ok; ++step)
+            for (int s = 0; s < 5 && ok; ++s) {
+                ok = ens_stage(c, *E, cur, 1, kA[s], kB[s]);
                 cur ^= 1;
             }
-        return true;
+        return ens_join(c, *E) && ok;   // also after a failure: nothing may still run when the call returns its error
     };
     hipGraphExec_t exec = nullptr;
     if (use_graph) {

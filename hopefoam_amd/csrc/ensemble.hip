@@ -23,7 +23,10 @@
 // neighbour traces an item reads were brought into the same XCD's L2 by the items next to it.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "ensemble.hpp"
+#include "lds_stage.hpp"
 
 namespace dg {
 
@@ -54,47 +57,96 @@ __device__ __forceinline__ d4_t mfma64(double a, double b, d4_t c) {
 }
 
 // MFMA variant: a wave owns 16 elements (group grp of the case); lane (col, rg) = (lane % 16, lane / 16).
-// B operands: K step s holds node 4 s + rg of element col.  A operands: the operator fragments in LDS.
-// Accumulators: register r of row tile m holds row 16 m + rg + 4 r of element col.
+// B operands: K step s of the volume products holds node 4 s + rg of element col; K step k of the lift holds point k
+// of face rg (the fragments' fourth row of a step is zero), so a lane reads the geometry, the neighbour and its
+// address of one face only.  A operands: the operator fragments in LDS.
+// Accumulators: register r of row tile m holds row 16 m + rg + 4 r of element col, node 4 s + rg with s = 4 m + r:
+// a lane owns the same nodes on both sides of the products, and the update has u in registers.
+// The passes are bound by latency (an ensemble's order rarely has more than two groups per SIMD), so everything a
+// group needs is requested before anything is used: one memory latency for the group's own values and connectivity,
+// one for the neighbours'.  Microseconds per stage (both passes) of 7 to 13 cases of one order, elements in all, with a
+// face's points running over the K steps, face geometry per point and the loads left where the products need them -> now:
+//   order 8, 50048: 82 -> 60    6, 36136: 41.6 -> 35.5    5, 30076: 30.4 -> 28.9    4, 16404: 15.2 -> 12.7
+//   order 7, 20780: 42 -> 43 (nine matrix steps of the lift in place of six)         3, 20918: 12.2 -> 11.1
 template <int N>
-__device__ void ens_q_mfma(const EnsArgs& a, const EnsCase& cs, const double* ops, int grp, int lane) {
-    constexpr int Np = ens_np(N), Nfp = N + 1;
-    constexpr int MT = ens_mfma_mt(N), KS = ens_mfma_ks(N), KSL = ens_mfma_ksl(N);
-    const int Kp = cs.Kp, col = lane & 15, rg = lane >> 4;
-    const int e0 = grp * 16 + col;
-    const bool live = e0 < cs.K;
-    const int e = live ? e0 : cs.K - 1;
-    const size_t arr = size_t(Kp) * Np;
-    const double* __restrict__ u = a.data + cs.off_u + size_t(a.cur) * arr;
-    double* __restrict__ qx = a.data + cs.off_u + ENS_QX * arr;
-    double* __restrict__ qy = a.data + cs.off_u + ENS_QY * arr;
-    const double* __restrict__ g = a.geo + cs.off_geo;
-    const int* __restrict__ cn = a.conn + cs.off_conn;
-    const double* __restrict__ DrF = ops;
-    const double* __restrict__ DsF = ops + MT * KS * 64;
-    const double* __restrict__ LF = ops + 2 * MT * KS * 64;
-    double ub[KS];
+struct EnsLane {
+    const double *up;       // u of the neighbour's node 0
+    unsigned own[N + 1];    // offset of point k of the lane's face in the group's nodes
+    unsigned nbr[N + 1];    // the matching point's offset from up
+    double nx, ny, fs, tf;
+    bool own_side;
+};
+
+// offset (in values, 16 per node) of point k of face f, f varying over the lanes
+template <int N>
+__device__ __forceinline__ unsigned face_off(int f, int k) {
+    return 16u * unsigned(f == 0 ? face_node<N>(0, k) : f == 1 ? face_node<N>(1, k) : face_node<N>(2, k));
+}
+
+// the lane's face (face 2 on the fourth row) of its element; ug: u of the group, ue: u of element 0
+template <int N>
+__device__ __forceinline__ void ens_lane(const EnsArgs& a, const EnsCase& cs, const double* u, int grp, int col, int rg,
+                                         EnsLane<N>& L) {
+    constexpr int Np = ens_np(N);
+    const unsigned Kp = cs.Kp, e = unsigned(grp) * 16 + col, f = rg < 3 ? rg : 2;
+    const double* g = a.geo + cs.off_geo;
+    const int c = (a.conn + cs.off_conn)[f * Kp + e];
+    L.nx = g[(4 + 4 * f) * Kp + e];
+    L.ny = g[(5 + 4 * f) * Kp + e];
+    L.fs = g[(6 + 4 * f) * Kp + e];
+    L.tf = g[(7 + 4 * f) * Kp + e];
+    const int en = c >> 3, fn = (c >> 1) & 3;
+    L.own_side = c & 1;
+    L.up = u + size_t(en >> 4) * (Np * 16) + (en & 15);
 #pragma unroll
-    for (int s = 0; s < KS; ++s) ub[s] = 4 * s + rg < Np ? u[nidx(e, 4 * s + rg, Np)] : 0.0;
-    // jumps at face node 4 s + rg (face f = idx / Nfp, point k = idx % Nfp)
-    double gxb[KSL], gyb[KSL];
-#pragma unroll
-    for (int s = 0; s < KSL; ++s) {
-        const int idx = 4 * s + rg;
-        gxb[s] = gyb[s] = 0.0;
-        if (idx < 3 * Nfp) {
-            const int f = idx / Nfp, k = idx - f * Nfp;
-            const int c = cn[f * Kp + e];
-            const int en = c >> 3, fn = (c >> 1) & 3;
-            if (!(c & 1)) {
-                const double um = u[nidx(e, face_node<N>(f, k), Np)];
-                const double up = u[nidx(en, face_node<N>(fn, N - k), Np)];
-                const double d = g[(6 + 4 * f) * Kp + e] * (um - up);
-                gxb[s] = g[(4 + 4 * f) * Kp + e] * d;
-                gyb[s] = g[(5 + 4 * f) * Kp + e] * d;
-            }
-        }
+    for (int k = 0; k <= N; ++k) {
+        L.own[k] = face_off<N>(f, k) + col;
+        L.nbr[k] = face_off<N>(fn, N - k);
     }
+}
+
+// One group's inputs of the q pass, requested together
+template <int N>
+struct EnsQIn {
+    double ub[ens_mfma_ks(N)], um[N + 1], up[N + 1], m[4];
+    double nx, ny, fs;
+    bool own_side;
+};
+
+template <int N>
+__device__ __forceinline__ void ens_q_load(const EnsArgs& a, const EnsCase& cs, int grp, int lane, EnsQIn<N>& in) {
+    constexpr int Np = ens_np(N), KS = ens_mfma_ks(N);
+    const int left = cs.K - grp * 16, c0 = lane & 15, col = c0 < left ? c0 : left - 1, rg = lane >> 4;
+    const size_t arr = size_t(cs.Kp) * Np;
+    const double* u = a.data + cs.off_u + size_t(a.cur) * arr;
+    const double* ug = u + size_t(grp) * (Np * 16);
+    const double* g = a.geo + cs.off_geo + grp * 16;
+    EnsLane<N> L;
+    ens_lane<N>(a, cs, u, grp, col, rg, L);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) in.ub[s] = 4 * s + rg < Np ? ug[unsigned(64 * s + 16 * rg + col)] : 0.0;
+#pragma unroll
+    for (int k = 0; k <= N; ++k) in.um[k] = ug[L.own[k]];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) in.m[i] = (g + size_t(i) * cs.Kp)[unsigned(col)];
+#pragma unroll
+    for (int k = 0; k <= N; ++k) in.up[k] = L.up[L.nbr[k]];
+    in.nx = L.nx;
+    in.ny = L.ny;
+    in.fs = L.fs;
+    in.own_side = L.own_side;
+}
+
+template <int N>
+__device__ __forceinline__ void ens_q_mfma(const EnsArgs& a, const EnsCase& cs, const double* ops, int grp, int lane,
+                                           const EnsQIn<N>& in) {
+    constexpr int Np = ens_np(N), Nfp = N + 1;
+    constexpr int MT = ens_mfma_mt(N), KS = ens_mfma_ks(N);
+    const int rg = lane >> 4;
+    const size_t arr = size_t(cs.Kp) * Np;
+    const double* DrF = ops;
+    const double* DsF = ops + MT * KS * 64;
+    const double* LF = ops + 2 * MT * KS * 64;
     d4_t ar[MT], as[MT], lx[MT], ly[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) ar[m] = as[m] = lx[m] = ly[m] = d4_t{0, 0, 0, 0};
@@ -102,122 +154,149 @@ __device__ void ens_q_mfma(const EnsArgs& a, const EnsCase& cs, const double* op
     for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            ar[m] = mfma64(DrF[(m * KS + s) * 64 + lane], ub[s], ar[m]);
-            as[m] = mfma64(DsF[(m * KS + s) * 64 + lane], ub[s], as[m]);
+            ar[m] = mfma64(DrF[(m * KS + s) * 64 + lane], in.ub[s], ar[m]);
+            as[m] = mfma64(DsF[(m * KS + s) * 64 + lane], in.ub[s], as[m]);
         }
 #pragma unroll
-    for (int s = 0; s < KSL; ++s)
+    for (int k = 0; k < Nfp; ++k) {
+        const double d = in.own_side ? 0.0 : in.fs * (in.um[k] - in.up[k]);
+        const double gx = in.nx * d, gy = in.ny * d;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            const double L = LF[(m * KSL + s) * 64 + lane];
-            lx[m] = mfma64(L, gxb[s], lx[m]);
-            ly[m] = mfma64(L, gyb[s], ly[m]);
+            const double L = LF[(m * Nfp + k) * 64 + lane];
+            lx[m] = mfma64(L, gx, lx[m]);
+            ly[m] = mfma64(L, gy, ly[m]);
         }
-    if (!live) return;
-    const double rx = g[0 * Kp + e], ry = g[1 * Kp + e], sx = g[2 * Kp + e], sy = g[3 * Kp + e];
+    }
+    const bool live = (lane & 15) < cs.K - grp * 16;
+    double* qx = a.data + cs.off_u + ENS_QX * arr + size_t(grp) * (Np * 16);
+    double* qy = qx + (ENS_QY - ENS_QX) * arr;
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int i = 16 * m + rg + 4 * r;
-            if (i < Np) {
-                qx[nidx(e0, i, Np)] = rx * ar[m][r] + sx * as[m][r] - lx[m][r];
-                qy[nidx(e0, i, Np)] = ry * ar[m][r] + sy * as[m][r] - ly[m][r];
+            const int s = 4 * m + r;
+            if (live && 4 * s + rg < Np) {
+                qx[unsigned(64 * s + lane)] = in.m[0] * ar[m][r] + in.m[2] * as[m][r] - lx[m][r];
+                qy[unsigned(64 * s + lane)] = in.m[1] * ar[m][r] + in.m[3] * as[m][r] - ly[m][r];
             }
         }
 }
 
+// B operands of one group's right-hand side: the flux differences at the face points for the lift, and for the volume
+// products -Fr = -(rx Fx + ry Fy), -Fs = -(sx Fx + sy Fy), F = a u - nu q (negated so that the volume and lift products
+// share one accumulator); and u at the nodes for the update.
 template <int N>
-__device__ void ens_rhs_mfma(const EnsArgs& a, const EnsCase& cs, const double* ops, int grp, int lane) {
-    constexpr int Np = ens_np(N), Nfp = N + 1;
-    constexpr int MT = ens_mfma_mt(N), KS = ens_mfma_ks(N), KSL = ens_mfma_ksl(N);
-    const int Kp = cs.Kp, col = lane & 15, rg = lane >> 4;
-    const int e0 = grp * 16 + col;
-    const bool live = e0 < cs.K;
-    const int e = live ? e0 : cs.K - 1;
-    const size_t arr = size_t(Kp) * Np;
-    double* __restrict__ base = a.data + cs.off_u;
-    const double* __restrict__ u = base + size_t(a.cur) * arr;
-    double* __restrict__ un = base + size_t(a.cur ^ 1) * arr;
-    double* __restrict__ res = base + ENS_RES * arr;
-    const double* __restrict__ qx = base + ENS_QX * arr;
-    const double* __restrict__ qy = base + ENS_QY * arr;
-    const double* __restrict__ g = a.geo + cs.off_geo;
-    const int* __restrict__ cn = a.conn + cs.off_conn;
-    const double* __restrict__ DrF = ops;
-    const double* __restrict__ DsF = ops + MT * KS * 64;
-    const double* __restrict__ LF = ops + 2 * MT * KS * 64;
-    const double ax = cs.ax, ay = cs.ay, nu = cs.nu;
-    const double rx = g[0 * Kp + e], ry = g[1 * Kp + e], sx = g[2 * Kp + e], sy = g[3 * Kp + e];
-    // B operands: -Fr = -(rx Fx + ry Fy), -Fs = -(sx Fx + sy Fy) at node 4 s + rg, F = a u - nu q (negated so
-    // that the volume and lift products share one accumulator)
-    double frb[KS], fsb[KS];
+struct EnsRhsIn {
+    double u[ens_mfma_ks(N)], fr[ens_mfma_ks(N)], fs[ens_mfma_ks(N)], gb[N + 1];
+};
+
+template <int N>
+__device__ __forceinline__ void ens_rhs_load(const EnsArgs& a, const EnsCase& cs, int grp, int lane, EnsRhsIn<N>& in) {
+    constexpr int Np = ens_np(N), KS = ens_mfma_ks(N);
+    const int left = cs.K - grp * 16, c0 = lane & 15, col = c0 < left ? c0 : left - 1, rg = lane >> 4;
+    const size_t arr = size_t(cs.Kp) * Np;
+    const double* u = a.data + cs.off_u + size_t(a.cur) * arr;
+    const size_t to_x = (ENS_QX - a.cur) * arr, to_y = (ENS_QY - a.cur) * arr;
+    const double* ug = u + size_t(grp) * (Np * 16);
+    const double* g = a.geo + cs.off_geo + grp * 16;
+    EnsLane<N> L;
+    ens_lane<N>(a, cs, u, grp, col, rg, L);
+    double um[N + 1], qm[N + 1], ym[N + 1], qx[KS], qy[KS], m[4];
+#pragma unroll
+    for (int k = 0; k <= N; ++k) {
+        um[k] = ug[L.own[k]];
+        qm[k] = (ug + to_x)[L.own[k]];
+        ym[k] = (ug + to_y)[L.own[k]];
+    }
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-        frb[s] = fsb[s] = 0.0;
-        if (4 * s + rg < Np) {
-            const size_t id = nidx(e, 4 * s + rg, Np);
-            const double Fx = ax * u[id] - nu * qx[id], Fy = ay * u[id] - nu * qy[id];
-            frb[s] = -(rx * Fx + ry * Fy);
-            fsb[s] = -(sx * Fx + sy * Fy);
-        }
+        const unsigned at = 64 * s + 16 * rg + col;
+        const bool in_range = 4 * s + rg < Np;
+        in.u[s] = in_range ? ug[at] : 0.0;
+        qx[s] = in_range ? (ug + to_x)[at] : 0.0;
+        qy[s] = in_range ? (ug + to_y)[at] : 0.0;
     }
-    // flux differences at face node 4 s + rg
-    double gb[KSL];
 #pragma unroll
-    for (int s = 0; s < KSL; ++s) {
-        const int idx = 4 * s + rg;
-        gb[s] = 0.0;
-        if (idx < 3 * Nfp) {
-            const int f = idx / Nfp, k = idx - f * Nfp;
-            const int c = cn[f * Kp + e];
-            const int en = c >> 3, fn = (c >> 1) & 3;
-            const bool own_side = c & 1;
-            const double nx = g[(4 + 4 * f) * Kp + e], ny = g[(5 + 4 * f) * Kp + e];
-            const double fs = g[(6 + 4 * f) * Kp + e], tf = g[(7 + 4 * f) * Kp + e];
-            const size_t im = nidx(e, face_node<N>(f, k), Np);
-            const size_t ip = nidx(en, face_node<N>(fn, N - k), Np);
-            const double um = u[im], up = u[ip];
-            const double qnm = nx * qx[im] + ny * qy[im];
-            const double qnp = nx * qx[ip] + ny * qy[ip];
-            const double an = ax * nx + ay * ny;
-            const double fadv = an >= 0.0 ? an * um : an * up;
-            const double qhat = (own_side ? qnp : qnm) - tf * (um - up);
-            gb[s] = fs * ((an * um - nu * qnm) - (fadv - nu * qhat));
-        }
+    for (int i = 0; i < 4; ++i) m[i] = (g + size_t(i) * cs.Kp)[unsigned(col)];
+    __builtin_amdgcn_sched_barrier(0);   // the connectivity has been on its way longest: now the neighbours' values
+#pragma unroll
+    for (int k = 0; k <= N; ++k) qm[k] = L.nx * qm[k] + L.ny * ym[k];
+    double up[N + 1], xp[N + 1], yp[N + 1];
+#pragma unroll
+    for (int k = 0; k <= N; ++k) {
+        up[k] = L.up[L.nbr[k]];
+        xp[k] = (L.up + to_x)[L.nbr[k]];
+        yp[k] = (L.up + to_y)[L.nbr[k]];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const double ax = cs.ax, ay = cs.ay, nu = cs.nu;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        const double Fx = ax * in.u[s] - nu * qx[s], Fy = ay * in.u[s] - nu * qy[s];
+        in.fr[s] = -(m[0] * Fx + m[1] * Fy);
+        in.fs[s] = -(m[2] * Fx + m[3] * Fy);
+    }
+    const double an = ax * L.nx + ay * L.ny;
+#pragma unroll
+    for (int k = 0; k <= N; ++k) {
+        const double qp = L.nx * xp[k] + L.ny * yp[k];
+        const double fadv = an >= 0.0 ? an * um[k] : an * up[k];
+        const double qhat = (L.own_side ? qp : qm[k]) - L.tf * (um[k] - up[k]);
+        in.gb[k] = L.fs * ((an * um[k] - nu * qm[k]) - (fadv - nu * qhat));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int N, bool UPDATE>
+__device__ __forceinline__ void ens_rhs_mfma(const EnsArgs& a, const EnsCase& cs, const double* ops, int grp, int lane,
+                                             const EnsRhsIn<N>& in) {
+    constexpr int Np = ens_np(N), Nfp = N + 1;
+    constexpr int MT = ens_mfma_mt(N), KS = ens_mfma_ks(N);
+    const int rg = lane >> 4;
+    const bool live = (lane & 15) < cs.K - grp * 16;
+    const size_t arr = size_t(cs.Kp) * Np;
+    double* base = a.data + cs.off_u + size_t(grp) * (Np * 16);
+    double* res = base + ENS_RES * arr;
+    const double* DrF = ops;
+    const double* DsF = ops + MT * KS * 64;
+    const double* LF = ops + 2 * MT * KS * 64;
+    double old[KS];
+    if constexpr (UPDATE) {   // in flight under the products
+        const bool has = live && a.rk_a != 0.0;   // the first stage (a = 0) does not read res, so it needs no clearing
+#pragma unroll
+        for (int s = 0; s < KS; ++s) old[s] = has && 4 * s + rg < Np ? res[unsigned(64 * s + lane)] : 0.0;
     }
     d4_t acc[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = d4_t{0, 0, 0, 0};
 #pragma unroll
-    for (int s = 0; s < KSL; ++s)
+    for (int k = 0; k < Nfp; ++k)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[m] = mfma64(LF[(m * KSL + s) * 64 + lane], gb[s], acc[m]);
+        for (int m = 0; m < MT; ++m) acc[m] = mfma64(LF[(m * Nfp + k) * 64 + lane], in.gb[k], acc[m]);
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            acc[m] = mfma64(DrF[(m * KS + s) * 64 + lane], frb[s], acc[m]);
-            acc[m] = mfma64(DsF[(m * KS + s) * 64 + lane], fsb[s], acc[m]);
+            acc[m] = mfma64(DrF[(m * KS + s) * 64 + lane], in.fr[s], acc[m]);
+            acc[m] = mfma64(DsF[(m * KS + s) * 64 + lane], in.fs[s], acc[m]);
         }
-    if (!live) return;
     const double dt = cs.dt;
+    double* un = base + size_t(a.cur ^ 1) * arr;
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int i = 16 * m + rg + 4 * r;
-            if (i >= Np) continue;
-            const size_t id = nidx(e0, i, Np);
-            const double rhs = acc[m][r];
-            if (a.mode == 0) {
-                res[id] = rhs;
+    for (int s = 0; s < KS; ++s) {
+        if (live && 4 * s + rg < Np) {
+            const unsigned at = 64 * s + lane;
+            const double rhs = acc[s / 4][s % 4];
+            if constexpr (UPDATE) {
+                const double rn = a.rk_a * old[s] + dt * rhs;
+                res[at] = rn;
+                un[at] = in.u[s] + a.rk_b * rn;
             } else {
-                const double rn = (a.rk_a == 0.0 ? 0.0 : a.rk_a * res[id]) + dt * rhs;
-                res[id] = rn;
-                un[id] = u[id] + a.rk_b * rn;
+                res[at] = rhs;
             }
         }
+    }
 }
 
 template <int N, int P>
@@ -401,27 +480,45 @@ __device__ void ens_rhs_item(const EnsArgs& a, const EnsCase& cs, const double* 
     }
 }
 
-// MFMA variant: items are runs of 16-element groups, one group per wave; fragments staged into LDS
+// MFMA variant: items are runs of at most kEnsWaves groups of 16 elements, one group per wave.  The fragments travel to
+// LDS by DMA while the waves request their first group's inputs.  PASS 0: q; 1: right-hand side and stage update;
+// 2: right-hand side into res.
 template <int PASS, int N>
 __global__ __launch_bounds__(64 * kEnsWaves) void ens_mfma_kernel(EnsArgs a) {
-    constexpr int nop = (2 * ens_mfma_mt(N) * ens_mfma_ks(N) + ens_mfma_mt(N) * ens_mfma_ksl(N)) * 64;
-    __shared__ double sop[nop];
-    for (int i = threadIdx.x; i < nop; i += 64 * kEnsWaves) sop[i] = a.opsM[N][i];
-    __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    constexpr size_t kBytes =
+        size_t(2 * ens_mfma_mt(N) * ens_mfma_ks(N) + ens_mfma_mt(N) * ens_mfma_ksl(N)) * 64 * sizeof(double);
+    __shared__ __attribute__((aligned(16))) double sop[dma_span(kBytes) / sizeof(double)];
+    dma_stage_to_lds<kBytes>(sop, a.opsM[N]);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int xcd = blockIdx.x & 7, nbx = gridDim.x >> 3, bx = blockIdx.x >> 3;
-    const int lo = a.chunk[xcd], hi = a.chunk[xcd + 1];
-    for (int it = lo + bx; it < hi; it += nbx) {
+    const int lo = a.chunk[xcd] + bx, hi = a.chunk[xcd + 1];
+    std::conditional_t<PASS == 0, EnsQIn<N>, EnsRhsIn<N>> in;
+    EnsCase cs;
+    int grp = 0;
+    // the wave's group of item it, its inputs on their way (false: no group; the same in all lanes)
+    auto request = [&](int it) {
         const EnsItem item = a.items[it];
-        const EnsCase cs = a.cases[item.c];
-        const int ngrp = cs.Kp / 16;
-        for (int t = wave; t < item.nb; t += kEnsWaves) {
-            const int grp = item.b0 + t;
-            if (grp >= ngrp) break;
-            if constexpr (PASS == 0) ens_q_mfma<N>(a, cs, sop, grp, lane);
-            else ens_rhs_mfma<N>(a, cs, sop, grp, lane);
+        cs = a.cases[item.c];
+        grp = item.b0 + wave;
+        const bool work = wave < item.nb && grp * 16 < cs.K;
+        if (work) {
+            if constexpr (PASS == 0) ens_q_load<N>(a, cs, grp, lane, in);
+            else ens_rhs_load<N>(a, cs, grp, lane, in);
         }
-    }
+        return work;
+    };
+    // whole waves only: a matrix instruction must not run with lanes left behind by the stores of the last group
+    auto finish = [&]() {
+        if constexpr (PASS == 0) ens_q_mfma<N>(a, cs, sop, grp, lane, in);
+        else ens_rhs_mfma<N, PASS == 1>(a, cs, sop, grp, lane, in);
+        __builtin_amdgcn_wave_barrier();
+    };
+    const bool first = lo < hi && request(lo);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's share of the fragments has landed
+    __syncthreads();
+    if (first) finish();
+    for (int it = lo + nbx; it < hi; it += nbx)
+        if (request(it)) finish();
 }
 
 // One persistent kernel per (pass, order, split) over that order's items: each is register-allocated for its
@@ -461,7 +558,10 @@ template <int PASS, int N>
 static hipError_t launch_n(int P, const EnsArgs& a, int grid, hipStream_t s) {
     if constexpr (N >= 2) {
         if (P == kEnsMfma) {
-            hipLaunchKernelGGL((ens_mfma_kernel<PASS, N>), dim3(grid), dim3(64 * kEnsWaves), 0, s, a);
+            if (PASS == 1 && a.mode == 0)
+                hipLaunchKernelGGL((ens_mfma_kernel<PASS == 1 ? 2 : 0, N>), dim3(grid), dim3(64 * kEnsWaves), 0, s, a);
+            else
+                hipLaunchKernelGGL((ens_mfma_kernel<PASS, N>), dim3(grid), dim3(64 * kEnsWaves), 0, s, a);
             return hipGetLastError();
         }
     }
@@ -496,13 +596,14 @@ hipError_t launch_ens_rhs(int N, int P, const EnsArgs& a, int grid, hipStream_t 
     return launch_pass<1>(N, P, a, grid, s);
 }
 
-// resident workgroups per CU: LDS (the order's operator table or MFMA fragments) and four waves per SIMD
+// resident workgroups per CU: LDS (the order's operator table or MFMA fragments), and waves per SIMD: four, two for
+// the MFMA kernels of orders 5 to 8 (more than 128 registers)
 int ens_blocks_per_cu(int N, int P) {
     const size_t lds = P == kEnsMfma
         ? size_t(2 * ens_mfma_mt(N) * ens_mfma_ks(N) + ens_mfma_mt(N) * ens_mfma_ksl(N)) * 64 * sizeof(double)
         : size_t(2 * ens_np(N) + 3 * (N + 1)) * kEnsRows * sizeof(double);
     const int by_lds = int((160u * 1024u) / lds);
-    const int by_waves = 16 / kEnsWaves;
+    const int by_waves = (P == kEnsMfma && N >= 5 ? 8 : 16) / kEnsWaves;
     const int b = by_lds < by_waves ? by_lds : by_waves;
     return b > 0 ? b : 1;
 }

@@ -58,7 +58,7 @@ bool ens_split_supported(int N, int P);
 // MFMA fragment tiles of order N: output-row tiles, K steps of Dr/Ds, K steps of LIFT
 inline constexpr int ens_mfma_mt(int N) { return ((N + 1) * (N + 2) / 2 + 15) / 16; }
 inline constexpr int ens_mfma_ks(int N) { return ((N + 1) * (N + 2) / 2 + 3) / 4; }
-inline constexpr int ens_mfma_ksl(int N) { return (3 * (N + 1) + 3) / 4; }
+inline constexpr int ens_mfma_ksl(int N) { return N + 1; }   // point k of the three faces, one row zero
 // pass 1: q = grad u - LIFT(...) for the items of order N in a.chunk; pass 2: right-hand side (+ stage update)
 hipError_t launch_ens_q(int N, int P, const EnsArgs& a, int grid, hipStream_t s);
 hipError_t launch_ens_rhs(int N, int P, const EnsArgs& a, int grid, hipStream_t s);

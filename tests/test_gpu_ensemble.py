@@ -166,3 +166,22 @@ def test_uneven_ensemble_conserves(ctx):
         assert abs(np.sum(J[:, None] * (u @ M)) - t0) <= 1e-12 * max(1.0, abs(t0))
         assert np.sum(J[:, None] * (u @ M) * u) < energy[i]
     ens.close()
+
+
+@pytest.mark.parametrize("N", [4, 5, 6, 7, 8])
+def test_matrix_tiles_group_edges(ctx, N):
+    """last groups of 2, 14, 16 and 8 elements, one to five work items per XCD range (the tolerance of the test above)"""
+    cases = make_cases([(N, nx, ny, 1.0, (0.9, -0.4), 0.004)
+                        for nx, ny in ((3, 3), (5, 3), (4, 6), (20, 13), (3, 3), (16, 31), (24, 40))])
+    ens = ctx.ensemble(cases, tau=TAU, beta=BETA, autotune=False)
+    assert ens.info()["split"][N] == 16
+    oms = [oracle_mesh(c) for c in cases]
+    us = [initial(om, c, 40 + i) for i, (om, c) in enumerate(zip(oms, cases))]
+    for i, u in enumerate(us):
+        ens.set(i, u)
+    ens.rhs()
+    for i, c in enumerate(cases):
+        want, q = oms[i].ldg_rhs(us[i], c["ax"], c["ay"], c["nu"], tau=TAU, beta=BETA, with_q=True)
+        assert np.abs(ens.get(i, 1) - want).max() <= 1e-12 * np.abs(want).max()
+        assert np.abs(ens.get(i, 2) - q).max() <= 1e-12 * np.abs(q).max()
+    ens.close()
