@@ -21,7 +21,7 @@ namespace dg {
 struct LimDev {
     int device = 0;
     double *lgeo = nullptr, *p4 = nullptr, *phi = nullptr, *wbc = nullptr, *mom = nullptr, *invV = nullptr;
-    double* vpos = nullptr;
+    double* posf = nullptr;   // MFMA fragments of the positivity points
     double *p4f = nullptr, *cff = nullptr;   // MFMA fragments of the moment and feature operators
     int npos = 0;
     int *jsel = nullptr, *troubled = nullptr;
@@ -31,7 +31,7 @@ struct LimDev {
     double *tgeo = nullptr, *rsn = nullptr, *tcell = nullptr, *tcv = nullptr, *tvg = nullptr;
     ~LimDev() {
         (void)hipSetDevice(device);
-        for (void* p : {(void*)lgeo, (void*)p4, (void*)phi, (void*)wbc, (void*)mom, (void*)invV, (void*)vpos,
+        for (void* p : {(void*)lgeo, (void*)p4, (void*)phi, (void*)wbc, (void*)mom, (void*)invV, (void*)posf,
                         (void*)jsel, (void*)troubled, (void*)count, (void*)tgeo, (void*)rsn, (void*)tcell,
                         (void*)tcv, (void*)tvg, (void*)p4f, (void*)cff})
             if (p) (void)hipFree(p);
@@ -162,6 +162,13 @@ static LimDev* limiter_for(dgh_ctx c, MeshDev* m) {
         for (int gq = 0; gq < Nfq; ++gq)
             for (int k = 0; k < Nfp; ++k)
                 vpos[size_t(Np + Nq + f * Nfq + gq) * Np + re.fmask[f * Nfp + k]] += re.Vf[size_t(gq) * Nfp + k];
+    // as A fragments: tile t, K step s, lane i + 16 k holds the entry (16 t + i, 4 s + k) of [mean; points]
+    const int NS = lim_ksteps(Np), tiles = (npos + 16) / 16;
+    std::vector<double> posf(size_t(tiles) * NS * 64, 0.0);
+    for (int r = 0; r <= npos; ++r)
+        for (int j = 0; j < Np; ++j)
+            posf[(size_t(r / 16) * NS + j / 4) * 64 + r % 16 + 16 * (j % 4)] =
+                r == 0 ? re.tvb_p4[j] : vpos[size_t(r - 1) * Np + j];
     std::vector<double> p4f, cff;
     limiter_fragments(re, p4f, cff);
     auto L = std::make_shared<LimDev>();
@@ -170,7 +177,7 @@ static LimDev* limiter_for(dgh_ctx c, MeshDev* m) {
     if (!c->upload(&L->p4f, p4f) || (!cff.empty() && !c->upload(&L->cff, cff))) return nullptr;
     const bool ok = c->upload(&L->lgeo, lgeo) && c->upload(&L->jsel, jsel) && c->upload(&L->p4, re.tvb_p4) &&
                     c->upload(&L->phi, re.tvb_phi) && c->upload(&L->wbc, re.tvb_wbc) && c->upload(&L->invV, re.invV) &&
-                    c->upload(&L->vpos, vpos) &&
+                    c->upload(&L->posf, posf) &&
                     c->hip(hipMalloc(reinterpret_cast<void**>(&L->troubled), size_t(groups) * 16 * sizeof(int)),
                            "hipMalloc") &&
                     c->hip(hipMalloc(reinterpret_cast<void**>(&L->count), 2 * sizeof(unsigned)), "hipMalloc");
@@ -196,7 +203,7 @@ static void limiter_args_fill(MeshDev* m, LimDev* L, int nvar, LimArgs& a) {
     a.troubled = L->troubled;
     a.count = L->count;
     a.pcount = L->count + 1;
-    a.vpos = L->vpos;
+    a.posf = L->posf;
     a.npos = L->npos;
     a.p4f = L->p4f;
     a.cff = L->cff;

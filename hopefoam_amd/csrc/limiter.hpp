@@ -33,7 +33,8 @@ struct LimArgs {
     MlpInfer mlp;
     int positivity = 0;              // 1: Zhang-Shu positivity scaling after limiting (4 variables)
     double gamma = 1.4, eps = 1e-10;
-    const double* vpos = nullptr;    // (Np + Nq + 3 Nfq) x Np point evaluation: nodes, cubature, face Gauss
+    const double* posf = nullptr;    // cell mean (row 0) and point evaluation (rows 1..npos: nodes, cubature, face
+                                     // Gauss) as f64 MFMA A fragments [(npos + 16) / 16][lim_ksteps(Np)][64]
     int npos = 0;
     unsigned* pcount = nullptr;      // cells scaled for positivity (accumulated)
     const double* p4f = nullptr;     // moment operator as f64 MFMA A fragments, [lim_msteps(Np)][64]

@@ -104,6 +104,28 @@ def test_positivity_matches_oracle(ctx, N):
     assert r_pts.min() > 0 and p_pts.min() > 0
 
 
+@pytest.mark.parametrize("N", range(1, 9))
+def test_positivity_group_edges(ctx, N):
+    """Every order, a last group of 6 cells, cells far below the bound, at it and away from it; tolerance as above."""
+    vxy, vid = split_quads(7, 5, 0.0, 1.0, 0.0, 1.0, periodic=(False, False))
+    bct = np.full(vid.shape, 2, np.int32)
+    om = OracleMesh(N, vxy, vid, bct)
+    K, Np = 70, (N + 1) * (N + 2) // 2
+    rng = np.random.default_rng(N)
+    q = np.stack([1.0 + 0.2 * rng.uniform(-1, 1, (K, Np)), rng.uniform(-1, 1, (K, Np)), rng.uniform(-1, 1, (K, Np)),
+                  2.6 + 0.3 * rng.uniform(-1, 1, (K, Np))])
+    q[0, 3::9] += 1.5 * rng.uniform(-1, 1, (len(range(3, K, 9)), Np))     # densities below zero
+    q[3, 5::11] += 2.0 * rng.uniform(-1, 1, (len(range(5, K, 11)), Np))   # pressures below zero
+    q[3, 69] += 2.0 * rng.uniform(-1, 1, Np)
+    want, sc = om.positivity(q)
+    f = ctx.mesh(N, vxy, vid, bct).field(4, q)
+    f.mesh.limit(f, M=1e30, positivity=True, flags=False)
+    got = f.download()
+    assert 3 <= sc.sum() < K
+    assert np.array_equal(np.any(got != q, axis=(0, 2)), sc)
+    assert np.abs(got - want).max() <= 1e-13 * np.abs(q).max()
+
+
 def test_limited_euler_steps(ctx):
     """Limiter (TVB + positivity) after every LSERK4 stage of a Roe Euler run from Riemann data: GPU (stage
     kernel + limiter) against the same sequence on the GPU with the limiter replaced by the oracle's."""
