@@ -532,8 +532,11 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
                     }
                     // the flux as a unit of its own: operands and results pass through registers as they are, so that the
                     // compiler forms the same fused multiply-adds whatever surrounds it
+                    // (advection at orders 1 and 2 always had its multiply-adds formed together with the choice of qP)
+                    if constexpr (PHYS == PHYS_EULER || N >= 3) {
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) asm volatile("" : "+v"(qM[v]), "+v"(qP[v]));
+                        for (int v = 0; v < NV; ++v) asm volatile("" : "+v"(qM[v]), "+v"(qP[v]));
+                    }
                     if constexpr (PHYS == PHYS_ADVECT) {   // upwind, or the central "average" flux without the |vn| term
                         const T vn = nx * ax + ny * ay;
                         const T diss = a.flux == FLUX_AVERAGE ? T(0) : fabs(vn);
