@@ -697,8 +697,9 @@ static int check_desc(dgh_ctx c, const dgh_rhs_desc* d, int* nvar) {
 
 // mom_out, p4f: the limiter's moments of the new state written by the stage kernel (bf16x3 stage updates only;
 // dg_limit_fused_moments says when), else null
-static int stage_launch(dgh_ctx c, MeshDev* m, const dgh_rhs_desc* d, const double* qin, double* qout, double* res,
-                        int mode, double ra, double rb, double dt, int nvar, double* mom_out = nullptr,
+// mode, old and res: StageArgs (old is its res_in)
+static int stage_launch(dgh_ctx c, MeshDev* m, const dgh_rhs_desc* d, const double* qin, double* qout,
+                        const double* old, double* res, int mode, double ra, double rb, double dt, int nvar, double* mom_out = nullptr,
                         const double* p4f = nullptr) {
     const RefDev* rd = m->ref;
     const bool f64 = d->prec == DGH_PREC_FP64;
@@ -708,6 +709,7 @@ static int stage_launch(dgh_ctx c, MeshDev* m, const dgh_rhs_desc* d, const doub
     a.mode = mode;
     a.q_in = qin;
     a.q_out = qout;
+    a.res_in = old;
     a.res = res;
     a.geo = f64 ? static_cast<const void*>(m->geo64) : static_cast<const void*>(m->geo32);
     a.conn = m->conn;
@@ -727,7 +729,7 @@ static int stage_launch(dgh_ctx c, MeshDev* m, const dgh_rhs_desc* d, const doub
     a.dt = dt;
     a.block_cap = c->stage_block_cap;
     if (mom_out) {
-        if (!split || mode != 1 || !p4f)
+        if (!split || mode == 0 || !p4f)
             return c->fail(DGH_ERR_ARG, "stage kernel: moments output needs a bf16x3 stage update"), DGH_ERR_ARG;
         a.mom_out = mom_out;
         a.p4f = p4f;
@@ -758,7 +760,7 @@ int dgh_rhs(dgh_ctx c, int mh, const dgh_rhs_desc* d, int q, int rhs) {
     if (fq->mesh != mh || fr->mesh != mh || fq->nvar != nvar || fr->nvar != nvar || q == rhs)
         return c->fail(DGH_ERR_ARG, "dgh_rhs: field/mesh mismatch"), DGH_ERR_ARG;
     (void)hipSetDevice(c->device);
-    return stage_launch(c, m, d, fq->d, fr->d, nullptr, 0, 0.0, 0.0, 0.0, nvar);
+    return stage_launch(c, m, d, fq->d, fr->d, nullptr, nullptr, 0, 0.0, 0.0, 0.0, nvar);
 }
 
 int dgh_lserk4_stage(dgh_ctx c, int mh, const dgh_rhs_desc* d, int q_in, int q_out, int res, int stage, double dt) {
@@ -775,7 +777,7 @@ int dgh_lserk4_stage(dgh_ctx c, int mh, const dgh_rhs_desc* d, int q_in, int q_o
         return c->fail(DGH_ERR_ARG, "dgh_lserk4_stage: bad fields or stage (q_in, q_out and res must differ)"),
                DGH_ERR_ARG;
     (void)hipSetDevice(c->device);
-    return stage_launch(c, m, d, a->d, b->d, r->d, 1, kRK4a[stage], kRK4b[stage], dt, nvar);
+    return stage_launch(c, m, d, a->d, b->d, r->d, r->d, 1, kRK4a[stage], kRK4b[stage], dt, nvar);
 }
 
 // SSP-RK2 of the reference's Euler driver (dgEulerFoam.C:64-123): q1 = q + dt L(q);
@@ -802,9 +804,10 @@ int dgh_ssprk2_stage(dgh_ctx c, int mh, const dgh_rhs_desc* d, int q_in, int q_o
         return c->fail(DGH_ERR_ARG, "dgh_ssprk2_stage: bad fields or stage (q_in, q_out and res must differ)"),
                DGH_ERR_ARG;
     (void)hipSetDevice(c->device);
-    if (stage == 1 && !c->hip(launch_field_diff(b->d, a->d, r->d, a->n, c->ncu, c->stream), "field difference"))
-        return c->last;
-    return stage_launch(c, m, d, a->d, b->d, r->d, 1, kSSPa[stage], kSSPb[stage], dt, nvar);
+    // stage 1 forms q^n - q^(1) as it reads the two (q_out still holds q^n): a pass of its own over three fields was
+    // 19 us at 42 MB a field
+    return stage_launch(c, m, d, a->d, b->d, stage == 1 ? b->d : r->d, r->d, stage == 1 ? 2 : 1, kSSPa[stage],
+                        kSSPb[stage], dt, nvar);
 }
 
 // nsteps LSERK4 steps on q, with the limiter ld (or none) applied to every stage's new state
@@ -826,7 +829,6 @@ static int lserk4_loop(dgh_ctx c, int mh, const dgh_rhs_desc* d, const dgh_lim_d
             !c->hip(hipMalloc(reinterpret_cast<void**>(&w.tmp), fq->n * sizeof(double)), "hipMalloc ws"))
             return c->last;
     }
-    if (!c->hip(hipMemsetAsync(w.res, 0, fq->n * sizeof(double), c->stream), "memset res")) return c->last;
     // bf16x3 stages with a TVB-family limiter: the stage kernel forms the limiter's moments of its new state, and
     // the limiter skips its moments pass (the same bits as the separate pass)
     double* mom = nullptr;
@@ -841,7 +843,10 @@ static int lserk4_loop(dgh_ctx c, int mh, const dgh_rhs_desc* d, const dgh_lim_d
     for (int step = 0; step < nsteps; ++step)
         for (int s = 0; s < 5; ++s) {
             if (!eval_bc(c, m, t0 + (step + kLserkC[s]) * dt)) return c->last;
-            if (int st = stage_launch(c, m, d, cur, nxt, w.res, 1, kRK4a[s], kRK4b[s], dt, nvar, mom, p4f)) return st;
+            // a step's first stage starts the residual (a = 0) and nothing reads the last stage's
+            if (int st = stage_launch(c, m, d, cur, nxt, s == 0 ? nullptr : w.res, s == 4 ? nullptr : w.res, 1, kRK4a[s],
+                                      kRK4b[s], dt, nvar, mom, p4f))
+                return st;
             if (ld) {
                 if (int st = dg_limit_enqueue(c, m, ld, nxt, nvar, false, nullptr, mom != nullptr)) return st;
             }
@@ -878,8 +883,7 @@ int dgh_ssprk2_run(dgh_ctx c, int mh, const dgh_rhs_desc* d, const dgh_lim_desc*
             return c->last;
     }
     // q holds q^n; w.tmp the first stage q^(1); the second stage writes q^(n+1) back into q (dgh_ssprk2_stage).
-    // The first stage scales res by 0: it must hold numbers, not whatever the allocation held.
-    if (!c->hip(hipMemsetAsync(w.res, 0, fq->n * sizeof(double), c->stream), "memset res")) return c->last;
+    // No residual is kept between the stages: the first starts at zero, the second at q^n - q^(1).
     double* mom = nullptr;   // moments formed by bf16x3 stage kernels for a TVB-family limiter (lserk4_loop)
     const double* p4f = nullptr;
     if (ld) {
@@ -890,13 +894,13 @@ int dgh_ssprk2_run(dgh_ctx c, int mh, const dgh_rhs_desc* d, const dgh_lim_desc*
     for (int step = 0; step < nsteps; ++step) {
         // both stages see the boundary data of t^n (dgEulerFoam.C:73)
         if (!eval_bc(c, m, t0 + step * dt)) return c->last;
-        if (int st = stage_launch(c, m, d, fq->d, w.tmp, w.res, 1, kSSPa[0], kSSPb[0], dt, nvar, mom, p4f)) return st;
+        if (int st = stage_launch(c, m, d, fq->d, w.tmp, nullptr, nullptr, 1, kSSPa[0], kSSPb[0], dt, nvar, mom, p4f))
+            return st;
         if (ld) {
             if (int st = dg_limit_enqueue(c, m, ld, w.tmp, nvar, false, nullptr, mom != nullptr)) return st;
         }
-        if (!c->hip(launch_field_diff(fq->d, w.tmp, w.res, fq->n, c->ncu, c->stream), "field difference"))
-            return c->last;
-        if (int st = stage_launch(c, m, d, w.tmp, fq->d, w.res, 1, kSSPa[1], kSSPb[1], dt, nvar, mom, p4f)) return st;
+        if (int st = stage_launch(c, m, d, w.tmp, fq->d, fq->d, nullptr, 2, kSSPa[1], kSSPb[1], dt, nvar, mom, p4f))
+            return st;
         if (ld) {
             if (int st = dg_limit_enqueue(c, m, ld, fq->d, nvar, false, nullptr, mom != nullptr)) return st;
         }

@@ -421,8 +421,9 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
 
         const size_t gbase = size_t(grp) * GS;
         const double* __restrict__ qin_g = a.q_in + gbase;
-        double* __restrict__ out_g = a.q_out + gbase;
-        double* __restrict__ res_g = a.res + gbase;
+        double* out_g = a.q_out + gbase;
+        double* res_g = a.res + gbase;
+        const double* old_g = a.res_in + gbase;
         double rmh[D::MT][4][NV], qmh[D::MT][4][NV];   // residual and q_in of the update
         auto load_update = [&]() {
 #pragma unroll
@@ -432,10 +433,18 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
                     const int j = 16 * m + RowMap<T>::row(rg, r);
 #pragma unroll
                     for (int v = 0; v < NV; ++v) {
-                        rmh[m][r][v] = j < Np ? at_lane(res_g + (v * Np + 16 * m + r) * 16, row8) : 0.0;
+                        rmh[m][r][v] = j < Np && a.res_in ? at_lane(old_g + (v * Np + 16 * m + r) * 16, row8) : 0.0;
                         qmh[m][r][v] = j < Np ? at_lane(qin_g + (v * Np + 16 * m + r) * 16, row8) : 0.0;
                     }
                 }
+            if (a.mode == 2) {
+#pragma unroll
+                for (int m = 0; m < D::MT; ++m)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int v = 0; v < NV; ++v) rmh[m][r][v] -= qmh[m][r][v];
+            }
         };
 
         // ---- faces.  The other side's face nodes of all three faces (lane (col, rg): variable rg) are requested
@@ -623,7 +632,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
                             put_lane(out_g + row, row8, rhs);
                         } else {
                             const double rn = a.rk_a * rmh[m][r][v] + a.dt * rhs;
-                            put_lane(res_g + row, row8, rn);
+                            if (a.res) put_lane(res_g + row, row8, rn);
                             qnew[v] = qmh[m][r][v] + a.rk_b * rn;
                             put_lane(out_g + row, row8, qnew[v]);
                         }
@@ -772,18 +781,6 @@ __global__ void mfma_bf16x3_probe_kernel(const uint4* A, const float* B, float* 
 hipError_t launch_mfma_bf16x3_probe(const unsigned* A, const float* B, float* D3, float* D1, hipStream_t st) {
     hipLaunchKernelGGL(mfma_bf16x3_probe_kernel, dim3(1), dim3(64), 0, st, reinterpret_cast<const uint4*>(A), B, D3,
                        D1);
-    return hipGetLastError();
-}
-
-// out = a - b over n values (the SSP-RK2 second stage's q^n - q^(1) term)
-__global__ __launch_bounds__(256) void field_diff_kernel(const double* __restrict__ a, const double* __restrict__ b,
-                                                         double* __restrict__ out, size_t n) {
-    for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += size_t(gridDim.x) * 256) out[i] = a[i] - b[i];
-}
-
-hipError_t launch_field_diff(const double* a, const double* b, double* out, size_t n, int ncu, hipStream_t st) {
-    const size_t blocks = std::min<size_t>((n + 255) / 256, size_t(8) * ncu);
-    hipLaunchKernelGGL(field_diff_kernel, dim3(unsigned(blocks > 0 ? blocks : 1)), dim3(256), 0, st, a, b, out, n);
     return hipGetLastError();
 }
 

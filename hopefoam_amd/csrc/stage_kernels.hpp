@@ -7,11 +7,15 @@ namespace dg {
 struct StageArgs {
     int K;
     int flux;            // FLUX_* (Euler: LF or ROE)
-    int mode;            // 0: q_out = rhs;  1: LSERK4 stage update
+    // 0: q_out = rhs;  1: stage update  r = a r + dt rhs, q_out = q_in + b r,  r read from res_in and written to res;
+    // 2: the same with r read as res_in - q_in
+    int mode;
     int block_cap;       // > 0: at most this many persistent blocks (rounded down to a multiple of 8, at least 8)
     const double* q_in;  // [nvar][K][Np]
     double* q_out;       // [nvar][K][Np]
-    double* res;         // [nvar][K][Np] (mode 1)
+    const double* res_in;   // [nvar][K][Np]; null: r starts at zero (a = 0).  May be q_out: every entry is read by the
+                            // lane that then writes it
+    double* res;            // null: r is not kept
     const void* geo;     // [16][K] in the compute precision
     const int* conn;     // [3][K]: neighbour*4 + face, or -1 - bc tag
     const void* VqF;     // operator fragments in the compute precision (bf16x3: split fragments, 32-bit words)
@@ -33,7 +37,6 @@ hipError_t launch_stage(int N, int phys, int prec, const StageArgs& a, int ncu, 
 // the FP64 stage on the mirror halves of the operators (stage_sym.hip): VqF the fragments in stage_sym.hpp's order,
 // fmask the node rows (a | b << 8, padded to whole K steps)
 hipError_t launch_stage_sym(int N, int phys, const StageArgs& a, int ncu, hipStream_t st);
-hipError_t launch_field_diff(const double* a, const double* b, double* out, size_t n, int ncu, hipStream_t st);
 hipError_t launch_mfma_layout_probe(double* out, hipStream_t st);
 hipError_t launch_mfma_probe(const double* A, const double* B, double* D64, const float* Af, const float* Bf,
                              float* D32, hipStream_t st);

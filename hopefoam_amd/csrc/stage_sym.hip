@@ -140,14 +140,28 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
                 if (s < KO) y[v][s < KO ? s : 0] = at_lane(src + v * Np * 16, nb[s < KO ? s : 0]);
             }
     };
+    auto load_old = [&](const double* src, double (&x)[NV][KE], double (&y)[NV][KO]) {
+        if (a.res_in) {
+            load_nodes(src, x, y);
+        } else {
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+#pragma unroll
+                for (int s = 0; s < KE; ++s) {
+                    x[v][s] = 0.0;
+                    if (s < KO) y[v][s < KO ? s : 0] = 0.0;
+                }
+        }
+    };
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the fragments and the first group have landed
     __syncthreads();
 
     for (; grp < g_hi; grp += gstride) {
         const int e = grp * 16 + col < K ? grp * 16 + col : K - 1;
         const double* __restrict__ qg = a.q_in + size_t(grp) * GS;
-        double* __restrict__ out_g = a.q_out + size_t(grp) * GS;
-        double* __restrict__ res_g = a.res + size_t(grp) * GS;
+        double* out_g = a.q_out + size_t(grp) * GS;
+        double* res_g = a.res + size_t(grp) * GS;
+        const double* old_g = a.res_in + size_t(grp) * GS;
         const double* qn = kLds ? qw : qg;
         // sums and differences of the node pairs: kept in registers, or formed from LDS for every point tile
         double qe[kLds ? 1 : NV][KE], qo[kLds ? 1 : NV][KO];
@@ -192,7 +206,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
             face_geo(2, nx2, ny2, fs2);
             keep1 = load_face(1, own1, oth1);
             face_geo(1, nx1, ny1, fs1);
-            if constexpr (UPDATE) load_nodes(res_g, ra, rb);
+            if constexpr (UPDATE) load_old(old_g, ra, rb);
         }
 
         d4_t accE[NV][ME], accO[NV][MO];
@@ -390,7 +404,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
         // ---- output: rows 4 s + rg, s = 4 m + r (padding columns keep evolving a copy of element K - 1).  Every load
         // comes before the first store (the compiler keeps loads behind stores that could alias).
         if constexpr (UPDATE) {
-            if constexpr (!kEarly) load_nodes(res_g, ra, rb);
+            if constexpr (!kEarly) load_old(old_g, ra, rb);
             load_nodes(qn, ua, ub);
         }
         if constexpr (kLds) {
@@ -399,31 +413,53 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
             if (grp + gstride < g_hi)
                 dma_to_lds_whole<GS * sizeof(double)>(a.q_in + size_t(grp + gstride) * GS, qw, lane);
         }
+        if constexpr (UPDATE) {
+            if (a.mode == 2) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v)
+                for (int v = 0; v < NV; ++v)
 #pragma unroll
-            for (int s = 0; s < KE; ++s) {
-                const int so = s < KO ? s : 0;
-                const double E = accE[v][s / 4][s % 4], O = s < KO ? accO[v][so / 4][s % 4] : 0.0;
-                double *ov = out_g + v * Np * 16, *rv = res_g + v * Np * 16;
-                const bool on = 4 * s + 3 < D::nrow || 4 * s + rg < D::nrow;
-                const bool pair = s < KO && (4 * s + 3 < D::npair || 4 * s + rg < D::npair);
-                if constexpr (!UPDATE) {
-                    if (on) put_lane(ov, na[s], E + O);
-                    if (pair) put_lane(ov, nb[so], E - O);
-                } else {
-                    const double r1 = a.rk_a * ra[v][s] + a.dt * (E + O);
-                    if (on) {
-                        put_lane(rv, na[s], r1);
-                        put_lane(ov, na[s], ua[v][s] + a.rk_b * r1);
+                    for (int s = 0; s < KE; ++s) {
+                        ra[v][s] -= ua[v][s];
+                        if (s < KO) rb[v][s < KO ? s : 0] -= ub[v][s < KO ? s : 0];
                     }
-                    if (pair) {
-                        const double r2 = a.rk_a * rb[v][so] + a.dt * (E - O);
-                        put_lane(rv, nb[so], r2);
-                        put_lane(ov, nb[so], ub[v][so] + a.rk_b * r2);
-                    }
-                }
             }
+        }
+        // f(row set s of variable v, its even and odd part, whether this lane has row a, row b)
+        auto rows = [&](auto f) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+#pragma unroll
+                for (int s = 0; s < KE; ++s) {
+                    const int so = s < KO ? s : 0;
+                    const double E = accE[v][s / 4][s % 4], O = s < KO ? accO[v][so / 4][s % 4] : 0.0;
+                    const bool on = 4 * s + 3 < D::nrow || 4 * s + rg < D::nrow;
+                    const bool pair = s < KO && (4 * s + 3 < D::npair || 4 * s + rg < D::npair);
+                    f(v, s, so, E, O, on, pair);
+                }
+        };
+        if constexpr (!UPDATE) {
+            rows([&](int v, int s, int so, double E, double O, bool on, bool pair) {
+                double* ov = out_g + v * Np * 16;
+                if (on) put_lane(ov, na[s], E + O);
+                if (pair) put_lane(ov, nb[so], E - O);
+            });
+        } else {
+            rows([&](int v, int s, int so, double E, double O, bool, bool) {
+                ra[v][s] = a.rk_a * ra[v][s] + a.dt * (E + O);
+                if (s < KO) rb[v][so] = a.rk_a * rb[v][so] + a.dt * (E - O);
+            });
+            if (a.res)
+                rows([&](int v, int s, int so, double, double, bool on, bool pair) {
+                    double* rv = res_g + v * Np * 16;
+                    if (on) put_lane(rv, na[s], ra[v][s]);
+                    if (pair) put_lane(rv, nb[so], rb[v][so]);
+                });
+            rows([&](int v, int s, int so, double, double, bool on, bool pair) {
+                double* ov = out_g + v * Np * 16;
+                if (on) put_lane(ov, na[s], ua[v][s] + a.rk_b * ra[v][s]);
+                if (pair) put_lane(ov, nb[so], ub[v][so] + a.rk_b * rb[v][so]);
+            });
+        }
         if constexpr (kLds) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next group has landed
     }
 }
