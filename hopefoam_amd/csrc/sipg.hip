@@ -152,20 +152,40 @@ __global__ __launch_bounds__(256) void norm_finish_kernel(CgState* __restrict__ 
 // in a fixed order (so every block gets the same bits) and applies the finish (INIT while its < 0, else ITER;
 // none for CG_FINISH_NONE); block 0 publishes the result to st_out.  st_in is never written by the same launch,
 // so the blocks cannot see each other's update.  A state that is already done passes through unchanged.
-__device__ void cg_advance(const CgState* __restrict__ st_in, CgState* __restrict__ st_out,
-                           const double* __restrict__ pb, const double* __restrict__ pa, int nb, int mode,
-                           CgState& ls) {
-    // the partials are read together with the state (a done state ignores them), so the two latencies overlap
-    double s[3] = {0.0, 0.0, 0.0};
-    if (mode != CG_FINISH_NONE)
-        for (int b = threadIdx.x; b < nb; b += 256) {
+// Two steps, so that a kernel can put its own loads between them: vector loads return in order, and what is requested
+// first does not wait for the rest.  Nothing is used before the second step (one word of the state per thread, the first
+// two partials as they are).
+struct CgPending {
+    double p[2][3];
+    unsigned long long word;
+};
+constexpr int kCgWords = sizeof(CgState) / 8;
+static_assert(sizeof(CgState) % 8 == 0 && kCgWords <= 256, "one word of the state per thread");
+
+__device__ __forceinline__ void cg_advance_load(const CgState* __restrict__ st_in, const double* __restrict__ pb,
+                                                const double* __restrict__ pa, int nb, bool sums, CgPending& c) {
+    c.word = threadIdx.x < kCgWords ? reinterpret_cast<const unsigned long long*>(st_in)[threadIdx.x] : 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int b = threadIdx.x + 256 * i;
+        const bool in = sums && b < nb;
+        c.p[i][0] = in ? pb[size_t(b) * 2] : 0.0;
+        c.p[i][1] = in ? pb[size_t(b) * 2 + 1] : 0.0;
+        c.p[i][2] = in ? pa[size_t(b) * 2] : 0.0;
+    }
+}
+__device__ __forceinline__ void cg_advance(const CgPending& c, CgState* __restrict__ st_out, const double* __restrict__ pb,
+                                           const double* __restrict__ pa, int nb, bool sums, CgState& ls) {
+    double s[3] = {c.p[0][0] + c.p[1][0], c.p[0][1] + c.p[1][1], c.p[0][2] + c.p[1][2]};
+    if (sums)
+        for (int b = threadIdx.x + 512; b < nb; b += 256) {
             s[0] += pb[size_t(b) * 2];
             s[1] += pb[size_t(b) * 2 + 1];
             s[2] += pa[size_t(b) * 2];
         }
-    if (threadIdx.x == 0) ls = *st_in;
+    if (threadIdx.x < kCgWords) reinterpret_cast<unsigned long long*>(&ls)[threadIdx.x] = c.word;
     __syncthreads();
-    if (!ls.done && mode != CG_FINISH_NONE) {
+    if (!ls.done && sums) {
         block_reduce<3>(s);
         if (threadIdx.x == 0) cg_finish(&ls, ls.its < 0 ? CG_FINISH_INIT : CG_FINISH_ITER, s[0], s[1], s[2]);
     }
@@ -179,7 +199,9 @@ __global__ __launch_bounds__(256) void cg_publish_kernel(const CgState* __restri
                                                          const double* __restrict__ pb, const double* __restrict__ pa,
                                                          int nb) {
     __shared__ CgState ls;
-    cg_advance(st_in, st_out, pb, pa, nb, CG_FINISH_AUTO, ls);
+    CgPending pend;
+    cg_advance_load(st_in, pb, pa, nb, true, pend);
+    cg_advance(pend, st_out, pb, pa, nb, true, ls);
 }
 
 // ---------------------------------------------------------------- operator kernels
@@ -308,6 +330,7 @@ __device__ __forceinline__ void update_load(const SipgArgs<T>& a, const CgLoop<T
     constexpr SipgTiles S(N);
     constexpr int Np = S.Np, KS = S.KS;
     const size_t base = size_t(g) * Np * 16;
+    if constexpr (BLOCK) in.bt = c.bidx[g * 16 + (lane & 15)];   // padded to whole groups
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
         if (4 * s + (lane >> 4) >= Np) continue;
@@ -324,7 +347,6 @@ __device__ __forceinline__ void update_load(const SipgArgs<T>& a, const CgLoop<T
         }
         if constexpr (!BLOCK) in.d[s] = c.dinv[at + lane];
     }
-    if constexpr (BLOCK) in.bt = c.bidx[g * 16 + (lane & 15)];   // padded to whole groups
     load_face_geo<T>(a, g, lane, in.fg);
 }
 
@@ -338,7 +360,10 @@ __device__ __forceinline__ void update_load(const SipgArgs<T>& a, const CgLoop<T
 // per-lane addresses of 32 bits beside a scalar base (order 5, 32768 elements, FP64, per iteration with the apply
 // kernel: block Jacobi 34.2 -> 32.2 us, point Jacobi 32.7 -> 31.5; FP32 corrections 26.2 -> 23.1; order 3, 2640
 // elements: 13.4 -> 12.8).  Requesting the group's first two inverse blocks ahead of the reduction as well costs more in
-// registers than it hides (order 5: 33.3, order 6: 22.2 -> 24.1).
+// registers than it hides (order 5: 33.3, order 6: 22.2 -> 24.1).  The partial sums and the state are
+// requested ahead of the group: vector loads return in order, and behind the group's 40 they came last (order 5 block
+// Jacobi 32.2 -> 32.2, point Jacobi 31.5 -> 30.6; order 4 block 24.0 -> 23.4; order 6, 18432 elements 31.8 -> 30.5; order 3,
+// 2640 elements 12.8 -> 12.5).
 template <int N, typename T, bool BLOCK, bool INIT>
 __global__ __launch_bounds__(256, N <= 6 ? 2 : 1) void cg_update_kernel(SipgArgs<T> a, CgLoop<T> c,
                                                         const CgState* __restrict__ st_in, CgState* __restrict__ st_out,
@@ -355,12 +380,15 @@ __global__ __launch_bounds__(256, N <= 6 ? 2 : 1) void cg_update_kernel(SipgArgs
     const int kq = lane >> 4;
     const int groups = (a.K + 15) >> 4;
     // The trace fragments (LDS DMA) and the first group's inputs do not depend on the CG scalars: they are
-    // requested before the reduction that yields them, so the latencies overlap.
+    // requested before the reduction that yields them, and after the partial sums it needs, so the latencies overlap.
+    CgPending pend;
+    cg_advance_load(st_in, pb_in, c.part_a, nb, !INIT, pend);
     dma_stage_to_lds<kTrBytes>(sA, a.TrF);
     const int g0 = blockIdx.x * 4 + wave;
     UpdateIn<T, KS> in;
     if (g0 < groups) update_load<N, T, BLOCK, INIT>(a, c, g0, lane, in);
-    cg_advance(st_in, st_out, pb_in, c.part_a, nb, INIT ? CG_FINISH_NONE : CG_FINISH_AUTO, ls);
+    __builtin_amdgcn_sched_barrier(0);
+    cg_advance(pend, st_out, pb_in, c.part_a, nb, !INIT, ls);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the fragments have landed (and no DMA outlives the block)
     if (ls.done) return;
     __syncthreads();
