@@ -4,7 +4,7 @@
 // its two slots: while the device packs (or unpacks) one, the worker copies the other from (or to) the caller's memory.
 // One worker copies about 30 GB/s; the first touch of a fresh result array costs as much again; the workers share both.
 // Small transfers stay on the calling thread.  Measured, up / down: 117 MB 38.8 / 45.7 ms -> 2.9 / 3.3 ms, 42 MB 15.5 /
-// 19.8 -> 1.1 / 1.4 ms, 4.2 MB 306 / 825 -> 146 / 153 us, 0.25 MB 27 / 29 -> 23 / 24 us.
+// 19.8 -> 1.1 / 1.5 ms, 4.2 MB 306 / 825 -> 145 / 159 us, 0.25 MB 27 / 29 -> 23 / 25 us, 35 KB 27 / 13 -> 17 / 17 us.
 #include "transfer.hpp"
 
 #include <algorithm>
@@ -88,6 +88,15 @@ hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArr
     const int step = std::max(per, std::min(most, int(kChunkLeast / (size_t(16) * a.Np * sizeof(double)))));
     const int chunks = (tiles + step - 1) / step;
     workers = std::min(workers, chunks);
+    if (chunks == 1) {   // nothing to overlap: no event, no worker
+        if (to_device) std::memcpy(st.slot(0), host, bytes);
+        const hipError_t err = to_device ? launch_unpack_tiles(a, 0, tiles, st.slot(0), s)
+                                         : launch_pack_tiles(a, 0, tiles, st.slot(0), s);
+        const hipError_t done = hipStreamSynchronize(s);
+        if (err != hipSuccess || done != hipSuccess) return err != hipSuccess ? err : done;
+        if (!to_device) std::memcpy(host, st.slot(0), bytes);
+        return hipSuccess;
+    }
     std::atomic<int> failed{int(hipSuccess)};
     auto work = [&](int w) {
         if (w > 0 && hipSetDevice(device) != hipSuccess) {

@@ -13,6 +13,7 @@
 namespace dg {
 
 constexpr int kTileMax = 16 * 45;      // order 8
+constexpr int kTileLoads = (kTileMax + 63) / 64;   // of one lane
 constexpr int kTileStride = 16 * 45 + 16;   // LDS of one wavefront's tile: 16 rows of an odd stride up to 46
 
 template <bool UNPACK>
@@ -27,13 +28,16 @@ __global__ __launch_bounds__(256) void tiles_kernel(NodalArray a, int t0, int t1
         const int live = a.K - 16 * g < 16 ? a.K - 16 * g : 16;
         double* h = host + (a.host_at(t) - h0);
         double* d = a.dev + (size_t(g) * a.nvar + v) * n;
-        if (UNPACK) {
-            for (int i = lane; i < live * a.Np; i += 64) {
-                const int e = i / a.Np;
-                buf[e * P + i - e * a.Np] = h[i];
-            }
-        } else {
-            for (int i = lane; i < n; i += 64) buf[(i & 15) * P + (i >> 4)] = d[i];
+        // the whole tile is requested before any of it is put down: a load across PCIe takes longer than the rest
+        const int count = UNPACK ? live * a.Np : n;
+        const double* src = UNPACK ? h : d;
+        double x[kTileLoads];
+#pragma unroll
+        for (int k = 0; k < kTileLoads; ++k) x[k] = lane + 64 * k < count ? src[lane + 64 * k] : 0.0;
+#pragma unroll
+        for (int k = 0; k < kTileLoads; ++k) {
+            const int i = lane + 64 * k, e = UNPACK ? i / a.Np : i & 15;
+            if (i < count) buf[e * P + (UNPACK ? i - e * a.Np : i >> 4)] = x[k];
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
