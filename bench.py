@@ -93,9 +93,10 @@ def stage_flops(K, Np, Nq, Nfq, nvar):
 
 
 def stage_bytes(K, Np, nvar, wg):
-    """algorithmic HBM bytes of one fused stage: q in/out, res in/out (FP64), geometry
-    (rx ry sx sy J + 3 x (nx ny Js)) in the compute precision, 15 B of connectivity"""
-    return K * (Np * nvar * 32 + 14 * wg + 15)
+    """algorithmic HBM bytes of one fused stage of the LSERK4 loop, the mean over a step's five: q in/out, res in/out
+    (FP64; the first stage reads none, the last writes none), geometry (rx ry sx sy J + 3 x (nx ny Js)) in the
+    compute precision, 15 B of connectivity"""
+    return K * (Np * nvar * 8 * (10 + 8) // 5 + 14 * wg + 15)
 
 
 def run_path(ctx, mesh, q0, prec, dt, steps, warmup, accuracy, x, y, limiter=None, detect=None):

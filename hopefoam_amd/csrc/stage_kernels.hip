@@ -67,10 +67,11 @@ __device__ __forceinline__ f4_t mfma3(const uint4 A, const Split4& B, f4_t c) {
 }
 
 // Persistent blocks: 8 waves (2 per SIMD) up to N = 6, else 4 waves with the full 512-register budget each.  With one
-// flux and one mode per instantiation and scalar group addresses neither kernel spills at two waves per SIMD (with both
-// fluxes in one kernel FP32 spilled 32 registers and bf16x3 needed 456).  Measured, LF, K = 131072, N = 6: FP32 251 ->
-// 172 us, bf16x3 150 us with one wave per SIMD, 134 with two (146 before).  A block's waves take groups apart, so that
-// every compute unit gets one before any gets two: K = 11834, N = 6 FP32 50.8 -> 25.8 us, bf16x3 23.3 -> 20.8 us.  When
+// flux and one mode per instantiation and scalar group addresses neither kernel spills at two waves per SIMD but for 2
+// registers of the instantiation with moments (with both fluxes in one kernel FP32 spilled 32 registers and bf16x3 needed
+// 456).  Measured, LF, K = 131072, N = 6: FP32 251 -> 173 us, bf16x3 150 us with one wave per SIMD, 127 with two (146
+// before).  A block's waves take groups apart, so that every compute unit gets one before any gets two: K = 11834, N = 6
+// FP32 50.8 -> 25.5 us, bf16x3 23.3 -> 20.5 us.  When
 // they fit, the operator fragments are staged into LDS once per block and shared by its waves.
 template <int N, typename T, bool SPLIT = false>
 constexpr int waves_per_block() { return N <= 6 ? 8 : 4; }

@@ -16,11 +16,11 @@
 // 16 elements instead of 600 for about 200 more additions.  Two wavefronts per SIMD (256 registers, N <= 6) hide the
 // gathers and the dependent chains; an f64 FMA then issues every 4.3 clk instead of 5.6.
 // Measured (us per stage; before: whole operators, one wavefront per SIMD, own traces by lane shuffles):
-//   LF, K = 131072:  N = 2  49.4 -> 41.0   3  87.0 -> 71.0   4  119 -> 92.5   5  200 -> 129   6  237 -> 168
-//   LF, K = 32768:   N = 7  185 -> 74      8  228 -> 110
-//   Roe, K = 131072: N = 1  43.1 -> 40.1   2  58.5 -> 43.7   3  103.8 -> 78.0  4  137 -> 99
+//   LF, K = 131072:  N = 2  49.4 -> 40.4   3  87.0 -> 71.0   4  119 -> 92.5   5  200 -> 127   6  237 -> 163
+//   LF, K = 32768:   N = 7  185 -> 73      8  228 -> 112
+//   Roe, K = 131072: N = 1  43.1 -> 40.1   2  58.5 -> 43.7   3  103.8 -> 78.0  4  137 -> 98
 //   small meshes:    N = 4 Roe, K = 1024  20.7 -> 14.2;  N = 4 advection, K = 2048  8.9 -> 6.2
-// Order 1 with the LF flux on large meshes is the exception (34.5 -> 37.3): its 3 nodes fill one tile either way.
+// Order 1 with the LF flux on large meshes is the exception (34.5 -> 36.7): its 3 nodes fill one tile either way.
 //
 // Layout: K step s of the interpolation takes node row 4 s + rg from row group rg; with the f64 accumulator map
 // (register r of row group rg holds row 4 r + rg) that is also the row of accumulator register r of tile m for
@@ -37,7 +37,7 @@
 namespace dg {
 
 // Wavefronts per block, and per SIMD as asked of the register allocation: two per SIMD where the kernel fits 256
-// registers without spilling, one beyond.  At K = 131072 and N = 6 two per SIMD take 168 us, one 192 us; spilling
+// registers without spilling, one beyond.  At K = 131072 and N = 6 two per SIMD take 163 us, one about 190 us; spilling
 // (all face loads ahead of the volume work, both fluxes in one kernel, 64-bit lane addresses) cost more than the
 // second wavefront gave, 229 to 305 us.
 template <int N>
