@@ -365,11 +365,15 @@ __device__ __forceinline__ double admissible_fraction(const double (&m)[4], cons
 // whether its pressure is above the bound by more than rounding, without a quotient; only a group with a cell that fails
 // this goes through the points again with the density scaled, the pressure itself and the bisection.
 // The evaluation bounds it (order 3: 4 x 3 products per tile of 16 rows); before, 256 lanes of a block evaluated the
-// points from LDS between block barriers.  131072 cells, order 3: 63.5 -> 23.4 us, the results bit for bit the same.
+// points from LDS between block barriers.  Four groups a block read the same operator tiles (one group a
+// block: order 3 22.3, 5 20.2, 6 86.9 us).  us per call beyond the limiter's, the results bit for bit the same:
+//   131072 cells: order 2 33 -> 11.4   3 61 -> 21.2   6 625 -> 74.8      32768: 5 52 -> 14.3      8192: 8 72 -> 23.3
 template <int N>
-__global__ __launch_bounds__(64) void positivity_kernel(LimArgs a, double* __restrict__ q) {
+__global__ __launch_bounds__(256) void positivity_kernel(LimArgs a, double* __restrict__ q) {
     constexpr int Np = LShape<N>::Np, NV = 4, NS = lim_ksteps(Np);
-    const int lane = threadIdx.x, col = lane & 15, kg = lane >> 4, g = blockIdx.x;
+    const int lane = threadIdx.x & 63, col = lane & 15, kg = lane >> 4;
+    const int g = int(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (g >= (a.K + 15) >> 4) return;
     const bool live = g * 16 + col < a.K;
     double* qg = q + size_t(g) * NV * Np * 16;
     double b[NV][NS];
@@ -457,19 +461,19 @@ __global__ __launch_bounds__(64) void positivity_kernel(LimArgs a, double* __res
     if (lane == 0 && n) atomicAdd(a.pcount, unsigned(__popcll(n)));
 }
 
-template <int N, int NV>
-static hipError_t launch_positivity(const LimArgs& a, double* q, hipStream_t s) {
-    if constexpr (NV == 4) {
-        if (a.positivity && !a.detect_only)
-            hipLaunchKernelGGL((positivity_kernel<N>), dim3((a.K + 15) / 16), dim3(64), 0, s, a, q);
-    }
-    return hipGetLastError();
-}
-
 // blocks of the wave-per-group kernels: one group per wavefront
 static int lim_grid(const LimArgs& a, int waves) {
     const int groups = (a.K + 15) / 16;
     return (groups + waves - 1) / waves;
+}
+
+template <int N, int NV>
+static hipError_t launch_positivity(const LimArgs& a, double* q, hipStream_t s) {
+    if constexpr (NV == 4) {
+        if (a.positivity && !a.detect_only)
+            hipLaunchKernelGGL((positivity_kernel<N>), dim3(lim_grid(a, 4)), dim3(256), 0, s, a, q);
+    }
+    return hipGetLastError();
 }
 
 template <int N, int NV>
