@@ -244,6 +244,7 @@ bool dgh_ctx_s::fail(int code, const char* fmt, ...) {
 
 bool dgh_ctx_s::hip(hipError_t e, const char* what) {
     if (e == hipSuccess) return true;
+    (void)hipGetLastError();   // the runtime keeps it, and the next launch's check would report it again
     return fail(DGH_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 
