@@ -811,6 +811,11 @@ int dgh_ssprk2_stage(dgh_ctx c, int mh, const dgh_rhs_desc* d, int q_in, int q_o
                         kSSPb[stage], dt, nvar);
 }
 
+// a scratch field of the time loops, allocated when a loop first needs it
+static bool scratch_field(dgh_ctx c, double** p, size_t n) {
+    return *p || c->hip(hipMalloc(reinterpret_cast<void**>(p), n * sizeof(double)), "hipMalloc ws");
+}
+
 // nsteps LSERK4 steps on q, with the limiter ld (or none) applied to every stage's new state
 static int lserk4_loop(dgh_ctx c, int mh, const dgh_rhs_desc* d, const dgh_lim_desc* ld, int q, int nsteps,
                        double dt, float* ms, const char* what) {
@@ -825,11 +830,7 @@ static int lserk4_loop(dgh_ctx c, int mh, const dgh_rhs_desc* d, const dgh_lim_d
     if (ld && ld->detect_only) return c->fail(DGH_ERR_ARG, "%s: a detect-only limiter changes nothing", what), DGH_ERR_ARG;
     (void)hipSetDevice(c->device);
     Workspace& w = m->ws[nvar];
-    if (!w.res) {
-        if (!c->hip(hipMalloc(reinterpret_cast<void**>(&w.res), fq->n * sizeof(double)), "hipMalloc ws") ||
-            !c->hip(hipMalloc(reinterpret_cast<void**>(&w.tmp), fq->n * sizeof(double)), "hipMalloc ws"))
-            return c->last;
-    }
+    if (!scratch_field(c, &w.res, fq->n) || !scratch_field(c, &w.tmp, fq->n)) return c->last;
     // bf16x3 stages with a TVB-family limiter: the stage kernel forms the limiter's moments of its new state, and
     // the limiter skips its moments pass (the same bits as the separate pass)
     double* mom = nullptr;
@@ -878,11 +879,7 @@ int dgh_ssprk2_run(dgh_ctx c, int mh, const dgh_rhs_desc* d, const dgh_lim_desc*
         return c->fail(DGH_ERR_ARG, "dgh_ssprk2_run: a detect-only limiter changes nothing"), DGH_ERR_ARG;
     (void)hipSetDevice(c->device);
     Workspace& w = m->ws[nvar];
-    if (!w.res) {
-        if (!c->hip(hipMalloc(reinterpret_cast<void**>(&w.res), fq->n * sizeof(double)), "hipMalloc ws") ||
-            !c->hip(hipMalloc(reinterpret_cast<void**>(&w.tmp), fq->n * sizeof(double)), "hipMalloc ws"))
-            return c->last;
-    }
+    if (!scratch_field(c, &w.tmp, fq->n)) return c->last;
     // q holds q^n; w.tmp the first stage q^(1); the second stage writes q^(n+1) back into q (dgh_ssprk2_stage).
     // No residual is kept between the stages: the first starts at zero, the second at q^n - q^(1).
     double* mom = nullptr;   // moments formed by bf16x3 stage kernels for a TVB-family limiter (lserk4_loop)

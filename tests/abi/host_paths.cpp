@@ -3,6 +3,7 @@
 #include "fake_hip.hpp"
 
 #include "dgh.h"
+#include "stage_kernels.hpp"
 
 #define CHECK(x)                                                                    \
     do {                                                                            \
@@ -32,9 +33,53 @@ static void error_is_not_kept() {
     CHECK(dgh_destroy(c) == DGH_OK);
 }
 
+// every stage kernel launched from now on reads and writes allocated memory
+static void check_stage_operands() {
+    fake::state().on_launch = [](const std::string& name, void** args) {
+        if (name.find("stage_kernel") == std::string::npos && name.find("stage_sym_kernel") == std::string::npos) return;
+        const dg::StageArgs& a = *static_cast<const dg::StageArgs*>(args[0]);
+        CHECK(a.q_in && a.q_out);
+        CHECK(fake::state().device.count(const_cast<double*>(a.q_in)) && fake::state().device.count(a.q_out));
+    };
+}
+
+// a time loop whose scratch cannot be allocated: each allocation it makes fails once; the loop says so, and the next
+// call runs on memory that is there
+template <typename Run>
+static void failing_scratch(Run run, int fields_needed) {
+    for (int which = 1; which <= fields_needed; ++which) {
+        dgh_ctx c = context();
+        int m = -1, q = -1;
+        CHECK(dgh_mesh_structured(c, 2, 3, 3, 0, 1, 0, 1, 1, 1, 0, &m) == DGH_OK);
+        CHECK(dgh_field_create(c, m, 4, &q) == DGH_OK);
+        check_stage_operands();
+        fake::state().fail_malloc = which;
+        const int before = fake::state().mallocs;
+        CHECK(run(c, m, q) == DGH_ERR_HIP);
+        CHECK(fake::state().mallocs == before + which);
+        CHECK(fake::state().fail_malloc == 0);
+        CHECK(run(c, m, q) == DGH_OK);
+        CHECK(fake::state().mallocs == before + fields_needed + 1);   // no field more than the loop needs
+        CHECK(run(c, m, q) == DGH_OK);
+        CHECK(fake::state().mallocs == before + fields_needed + 1);
+        fake::state().on_launch = nullptr;
+        CHECK(dgh_destroy(c) == DGH_OK);
+        CHECK(fake::state().device.empty());
+    }
+}
+
+static void lserk4_scratch() {   // the residual and the second state
+    failing_scratch([](dgh_ctx c, int m, int q) { return dgh_lserk4_run(c, m, &kEuler, q, 2, 1e-3, nullptr); }, 2);
+}
+static void ssprk2_scratch() {   // the first stage's state
+    failing_scratch([](dgh_ctx c, int m, int q) { return dgh_ssprk2_run(c, m, &kEuler, nullptr, q, 2, 1e-3, nullptr); }, 1);
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> all = {
         {"error_is_not_kept", error_is_not_kept},
+        {"lserk4_scratch", lserk4_scratch},
+        {"ssprk2_scratch", ssprk2_scratch},
     };
     CHECK(argc == 2 && all.count(argv[1]));
     all.at(argv[1])();

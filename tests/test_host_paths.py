@@ -32,3 +32,9 @@ def run(program, name):
 def test_error_is_not_kept(program):
     """an allocation that fails is an error of its own call only"""
     run(program, "error_is_not_kept")
+
+
+@pytest.mark.parametrize("name", ["lserk4_scratch", "ssprk2_scratch"])
+def test_failing_scratch(program, name):
+    """a time loop whose scratch fields cannot be allocated fails, and the next call finds them allocated"""
+    run(program, name)
