@@ -15,6 +15,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "dg_common.hpp"
@@ -49,6 +50,7 @@ struct SipgDev {
     SipgOps<float> s;
     bool have32 = false;
     double* bdata[2] = {nullptr, nullptr};   // Dirichlet and Neumann data of sipg_rhs, allocated when first given
+    std::mutex bdata_mu;                     // one call's data at a time, from its copy until its kernel is done
     double* part = nullptr;
     CgState* st = nullptr;       // [4]: the iteration's two states, the published state, auxiliary norms
     double* part_b[2] = {nullptr, nullptr};   // the update kernel's partials by iteration parity (part holds the
@@ -556,8 +558,10 @@ int dgh_sipg_rhs_neumann(dgh_ctx c, int h, int f, const double* gbc, const doubl
     if (f == b) return c->fail(DGH_ERR_ARG, "dgh_sipg_rhs: f and b must differ"), DGH_ERR_ARG;
     (void)hipSetDevice(c->device);
     const size_t n = size_t(S->K) * 3 * (S->N + 1);
-    // the boundary data's device buffers stay with the handle: an allocation and a free per call cost more than the
-    // kernel
+    // the boundary data's device buffers stay with the handle (an allocation and a free per call cost more than the
+    // kernel): threads that bring data take turns
+    std::unique_lock<std::mutex> turn(S->bdata_mu, std::defer_lock);
+    if (gbc || gnb) turn.lock();
     double* dg[2] = {nullptr, nullptr};
     const double* host[2] = {gbc, gnb};
     bool ok = true;

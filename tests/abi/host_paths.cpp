@@ -2,6 +2,10 @@
 // of them on the runtime of fake_hip.hpp and says what is wrong, if anything, on stderr.
 #include "fake_hip.hpp"
 
+#include <chrono>
+#include <condition_variable>
+#include <thread>
+
 #include "dgh.h"
 #include "stage_kernels.hpp"
 
@@ -75,11 +79,57 @@ static void ssprk2_scratch() {   // the first stage's state
     failing_scratch([](dgh_ctx c, int m, int q) { return dgh_ssprk2_run(c, m, &kEuler, nullptr, q, 2, 1e-3, nullptr); }, 1);
 }
 
+// two threads form right-hand sides of one solver with their own boundary data: from a call's copy of its data to the
+// device until the call is done, nobody else writes there
+static void sipg_rhs_threads() {
+    dgh_ctx c = context();
+    int m = -1, s = -1, f = -1, b[2];
+    CHECK(dgh_mesh_structured(c, 2, 3, 3, 0, 1, 0, 1, 0, 0, DGH_BC_FIXED_VALUE, &m) == DGH_OK);
+    dgh_sipg_desc d = {};
+    d.maxit = 10;
+    d.rtol = 1e-8;
+    CHECK(dgh_sipg_create(c, m, &d, &s) == DGH_OK);
+    CHECK(dgh_field_create(c, m, 1, &f) == DGH_OK);
+    for (int& x : b) CHECK(dgh_field_create(c, m, 1, &x) == DGH_OK);
+    const size_t n = size_t(18) * 3 * 3;
+    std::mutex mu;
+    std::condition_variable cv;
+    std::map<void*, std::thread::id> owner;   // of a destination between the copy and the end of the call
+    bool clash = false;
+    fake::state().on_copy = [&](void* dst, const void*, size_t bytes, hipMemcpyKind kind) {
+        if (kind != hipMemcpyHostToDevice || bytes != n * sizeof(double)) return;
+        std::unique_lock<std::mutex> lock(mu);
+        auto it = owner.find(dst);
+        if (it != owner.end() && it->second != std::this_thread::get_id()) clash = true;
+        owner[dst] = std::this_thread::get_id();
+        cv.notify_all();
+        cv.wait_for(lock, std::chrono::milliseconds(300), [&] { return clash; });   // the other thread's chance
+    };
+    fake::state().on_sync = [&] {
+        std::lock_guard<std::mutex> lock(mu);
+        for (auto it = owner.begin(); it != owner.end();)
+            it = it->second == std::this_thread::get_id() ? owner.erase(it) : std::next(it);
+    };
+    std::vector<double> g[2] = {std::vector<double>(n, 1.0), std::vector<double>(n, 2.0)};
+    std::vector<std::thread> t;
+    for (int i = 0; i < 2; ++i)
+        t.emplace_back([&, i] {
+            for (int k = 0; k < 2; ++k) CHECK(dgh_sipg_rhs_neumann(c, s, f, g[i].data(), g[i].data(), b[i]) == DGH_OK);
+        });
+    for (auto& x : t) x.join();
+    fake::state().on_copy = nullptr;
+    fake::state().on_sync = nullptr;
+    CHECK(!clash);
+    CHECK(dgh_destroy(c) == DGH_OK);
+    CHECK(fake::state().device.empty());
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> all = {
         {"error_is_not_kept", error_is_not_kept},
         {"lserk4_scratch", lserk4_scratch},
         {"ssprk2_scratch", ssprk2_scratch},
+        {"sipg_rhs_threads", sipg_rhs_threads},
     };
     CHECK(argc == 2 && all.count(argv[1]));
     all.at(argv[1])();

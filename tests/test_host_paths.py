@@ -38,3 +38,8 @@ def test_error_is_not_kept(program):
 def test_failing_scratch(program, name):
     """a time loop whose scratch fields cannot be allocated fails, and the next call finds them allocated"""
     run(program, name)
+
+
+def test_sipg_rhs_threads(program):
+    """right-hand sides of one solver formed by two threads at once keep their boundary data apart"""
+    run(program, "sipg_rhs_threads")
