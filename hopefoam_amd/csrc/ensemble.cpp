@@ -507,7 +507,7 @@ extern "C" int dgh_ensemble_run(dgh_ctx c, int h, int nsteps, int use_graph, flo
                 ok = ens_stage(c, *E, cur, 1, kA[s], kB[s]);
                 cur ^= 1;
             }
-        return ens_join(c, *E) && ok;   // also after a failure: nothing may still run when the call returns its error
+        return ens_join(c, *E) && ok;   // also after a failure: the context's stream waits for what was launched
     };
     hipGraphExec_t exec = nullptr;
     if (use_graph) {
@@ -535,6 +535,7 @@ extern "C" int dgh_ensemble_run(dgh_ctx c, int h, int nsteps, int use_graph, flo
     if (use_graph) {
         if (!c->hip(hipGraphLaunch(exec, c->stream), "graph launch")) return c->last;
     } else if (!record(start)) {
+        (void)hipStreamSynchronize(c->stream);   // nothing may still run when the call returns its error
         return c->last;
     }
     if (!c->hip(hipEventRecord(c->ev1, c->stream), "event") || !c->hip(hipEventSynchronize(c->ev1), "sync"))

@@ -17,16 +17,19 @@
 
 namespace fake {
 
-struct Event;
+struct Stream;
+typedef std::map<Stream*, long> Waits;   // work of streams, as the number of launches it reaches to
 struct Stream {
-    long issued = 0, done = 0;                       // launches queued here, and known to have ended
-    std::vector<std::pair<Stream*, long>> waits;     // work of other streams that later work waits for
+    long issued = 0, done = 0;   // launches queued here, and known to have ended
+    Waits waits;                 // what later work here waits for
 };
 struct Event {
-    Stream* s = nullptr;
-    long at = 0;
-    std::vector<std::pair<Stream*, long>> waits;
+    Waits waits;
 };
+inline void add(Waits& w, Stream* s, long at) {
+    long& x = w[s];
+    if (x < at) x = at;
+}
 
 struct State {
     std::recursive_mutex mu;
@@ -45,10 +48,9 @@ inline State& state() {
     static State* s = new State;   // the library registers its kernels before this program's initialisers run
     return *s;
 }
-inline void finish(Stream* s, long at) {
-    if (s->done < at) s->done = at;
-    for (auto& w : s->waits)
-        if (w.first->done < w.second) finish(w.first, w.second);
+inline void finish(const Waits& waits) {
+    for (auto& w : waits)
+        if (w.first->done < w.second) w.first->done = w.second;
 }
 // launches that no synchronisation has waited for
 inline long pending() {
@@ -161,15 +163,15 @@ hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }   // kept: event
 hipError_t hipStreamSynchronize(hipStream_t s) {
     {
         FAKE_LOCK;
-        fake::finish(fs(s), fs(s)->issued);
+        fs(s)->done = fs(s)->issued;
+        fake::finish(fs(s)->waits);
     }
     if (fake::state().on_sync) fake::state().on_sync();
     return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
     FAKE_LOCK;
-    if (fe(e)->s) fs(s)->waits.push_back({fe(e)->s, fe(e)->at});
-    for (auto& w : fe(e)->waits) fs(s)->waits.push_back(w);
+    for (auto& w : fe(e)->waits) fake::add(fs(s)->waits, w.first, w.second);
     return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
@@ -180,15 +182,13 @@ hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0);
 hipError_t hipEventDestroy(hipEvent_t e) { delete fe(e); return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     FAKE_LOCK;
-    fe(e)->s = fs(s);
-    fe(e)->at = fs(s)->issued;
     fe(e)->waits = fs(s)->waits;
+    fake::add(fe(e)->waits, fs(s), fs(s)->issued);
     return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t e) {
     FAKE_LOCK;
-    if (fe(e)->s) fake::finish(fe(e)->s, fe(e)->at);
-    for (auto& w : fe(e)->waits) fake::finish(w.first, w.second);
+    fake::finish(fe(e)->waits);
     return hipSuccess;
 }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 1.f; return hipSuccess; }

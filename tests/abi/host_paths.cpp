@@ -124,12 +124,37 @@ static void sipg_rhs_threads() {
     CHECK(fake::state().device.empty());
 }
 
+// whichever launch of an ensemble call fails, none of those before it is still running when the call returns
+static void ensemble_failing_launch() {
+    dgh_ctx c = context();
+    const dgh_ens_desc d = {1.0, 1.0, 0.3, 0, 0};
+    std::vector<dgh_ens_case> cases;
+    for (int N : {2, 4, 5, 8, 3}) cases.push_back({N, 4, 4, 0, 0, 1, 1, 1.0, 0.5, 1e-3, 1e-4});
+    int e = -1;
+    CHECK(dgh_ensemble_create(c, &d, int(cases.size()), cases.data(), &e) == DGH_OK);
+    CHECK(fake::pending() == 0);
+    for (int which = 1; which <= 24; ++which) {
+        fake::state().fail_launch = which;
+        CHECK(dgh_ensemble_run(c, e, 1, 0, nullptr) == DGH_ERR_HIP);
+        CHECK(fake::state().fail_launch == 0);
+        CHECK(fake::pending() == 0);
+    }
+    for (int which = 1; which <= 10; ++which) {
+        fake::state().fail_launch = which;
+        CHECK(dgh_ensemble_rhs(c, e) == DGH_ERR_HIP);
+        CHECK(fake::pending() == 0);
+    }
+    CHECK(dgh_ensemble_run(c, e, 1, 0, nullptr) == DGH_OK && fake::pending() == 0);
+    CHECK(dgh_destroy(c) == DGH_OK);
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> all = {
         {"error_is_not_kept", error_is_not_kept},
         {"lserk4_scratch", lserk4_scratch},
         {"ssprk2_scratch", ssprk2_scratch},
         {"sipg_rhs_threads", sipg_rhs_threads},
+        {"ensemble_failing_launch", ensemble_failing_launch},
     };
     CHECK(argc == 2 && all.count(argv[1]));
     all.at(argv[1])();

@@ -43,3 +43,8 @@ def test_failing_scratch(program, name):
 def test_sipg_rhs_threads(program):
     """right-hand sides of one solver formed by two threads at once keep their boundary data apart"""
     run(program, "sipg_rhs_threads")
+
+
+def test_ensemble_failing_launch(program):
+    """an ensemble call that fails half-way leaves nothing running"""
+    run(program, "ensemble_failing_launch")
