@@ -35,7 +35,8 @@ __device__ __forceinline__ f4_t mfma4(float a, float b, f4_t c) {
 // fused multiply-adds (each step squares the relative error, so the result is within an ulp of 1 / x), five instructions
 // instead of the eleven of an IEEE division (the densities it is taken of are positive and normal); v_rsq_f64 refined
 // by one coupled step for sqrt(x) and 1 / (2 sqrt(x)) and two residual corrections g += h (x - g g), within an ulp of
-// sqrt(x), in half the instructions of the scaled library square root (0, infinity and NaN come out as themselves).
+// sqrt(x), in half the instructions of the scaled library square root (0 and infinity come out as themselves, a negative
+// number as NaN).  The residual x - g g of a subnormal x is rounded to a multiple of the least number: 0, as it should be.
 // FP32: the hardware's v_rcp_f32 / v_sqrt_f32 (about 1 ulp), far below the FP32 and bf16x3 paths' contraction
 // round-off, in one instruction instead of the ten of an IEEE division or square root.
 __device__ __forceinline__ double inv(double x) {
@@ -45,14 +46,14 @@ __device__ __forceinline__ double inv(double x) {
 }
 __device__ __forceinline__ float inv(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ double fsqrt(double x) {
-    const double y = __builtin_amdgcn_rsq(fmax(x, 1e-300));
+    const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
     const double r = fma(-h, g, 0.5);
     g = fma(g, r, g);
     h = fma(h, r, h);
     g = fma(fma(-g, g, x), h, g);
     g = fma(fma(-g, g, x), h, g);
-    return x < __builtin_huge_val() ? g : x;
+    return __builtin_amdgcn_class(x, 0x260) ? x : g;   // -0, +0, +inf
 }
 __device__ __forceinline__ float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
