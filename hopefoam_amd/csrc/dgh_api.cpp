@@ -79,12 +79,45 @@ void build_fragments(const RefElem& re, std::vector<double>& VqF, std::vector<do
             }
 }
 
+// Fragments of the FP64 stage kernel on whole operators in the order of SymDims (order 1), lanes as below
+template <int N>
+bool build_whole(const RefElem& re, std::vector<double>& F, std::vector<int>& rows) {
+    using D = SymDims<N>;
+    const int Np = re.Np, Nq = re.Nq, Nfq = re.Nfq;
+    if (Np != D::nrow || Nq != D::qrow || Nfq != D::Nfq) return false;
+    F.assign(D::nF, 0.0);
+    size_t at = 0;
+    auto put = [&](int tile, int nr, auto&& val) {
+        for (int l = 0; l < 64; ++l, ++at) {
+            const int i = 16 * tile + (l & 15);
+            if (i < nr) F[at] = val(i, l >> 4);
+        }
+    };
+    for (int t = 0; t < D::TE; ++t)
+        for (int s = 0; s < D::KE; ++s)
+            put(t, Nq, [&](int i, int k) { return 4 * s + k < Np ? re.Vq[size_t(i) * Np + 4 * s + k] : 0.0; });
+    for (int ks = 0; ks < D::KT; ++ks)
+        for (const std::vector<double>* P : {&re.Pr, &re.Ps})
+            for (int m = 0; m < D::ME; ++m)
+                put(m, Np, [&](int i, int k) { return 4 * ks + k < Nq ? (*P)[size_t(i) * Nq + 4 * ks + k] : 0.0; });
+    for (int f : {0, 2, 1})
+        for (int j = 0; j < D::SF; ++j)
+            for (int m = 0; m < D::ME; ++m)
+                put(m, Np, [&](int i, int k) {
+                    return 4 * j + k < Nfq ? re.Lift[size_t(i) * 3 * Nfq + f * Nfq + 4 * j + k] : 0.0;
+                });
+    rows.assign(4 * D::KE, 0);
+    for (int i = 0; i < Np; ++i) rows[i] = i | i << 8;
+    return at == F.size();
+}
+
 // Fragments of the mirror-symmetric FP64 stage kernel in the order of SymDims: lane l of a fragment holds operator
 // row 16 tile + l % 16 and K row 4 step + l / 16.
 template <int N>
 bool build_sym(const RefElem& re, std::vector<double>& F, std::vector<int>& rows) {
     using D = SymDims<N>;
     const RefElem::Mirror& mi = re.mirror;
+    if constexpr (D::whole) return build_whole<N>(re, F, rows);
     if (mi.npair != D::npair || mi.nrow != D::nrow || mi.qpair != D::qpair || mi.qrow != D::qrow) return false;
     const int Nq = re.Nq, Nfq = re.Nfq;
     F.assign(D::nF, 0.0);

@@ -18,9 +18,12 @@
 // Measured (us per stage; before: whole operators, one wavefront per SIMD, own traces by lane shuffles):
 //   LF, K = 131072:  N = 2  49.4 -> 40.4   3  87.0 -> 71.0   4  119 -> 92.5   5  200 -> 127   6  237 -> 163
 //   LF, K = 32768:   N = 7  185 -> 73      8  228 -> 112
-//   Roe, K = 131072: N = 1  43.1 -> 40.1   2  58.5 -> 43.7   3  103.8 -> 78.0  4  137 -> 98
+//   Roe, K = 131072: N = 2  58.5 -> 44.3   3  103.8 -> 78.4  4  137 -> 98.5
 //   small meshes:    N = 4 Roe, K = 1024  20.7 -> 14.2;  N = 4 advection, K = 2048  8.9 -> 6.2
-// Order 1 with the LF flux on large meshes is the exception (34.5 -> 36.7): its 3 nodes fill one tile either way.
+// Order 1 takes the whole operators in this kernel's layout (SymDims::whole): its 3 nodes fill one tile either way, and
+// on the halves large meshes were slower than before (LF: 35.0 -> 36.5 us at K = 131072, 15.0 -> 19.6 at 45000).  Before,
+// on the halves, now:  LF, K = 131072 35.0, 36.5, 30.3;  45000 15.0, 19.6, 12.6;  32768 11.5, 12.1, 9.6;  8192 8.2, 6.8,
+// 5.5;  Roe, K = 131072 43.6, 40.3, 34.4;  advection, K = 524288 39.0, 43.0, 36.7
 //
 // Layout: K step s of the interpolation takes node row 4 s + rg from row group rg; with the f64 accumulator map
 // (register r of row group rg holds row 4 r + rg) that is also the row of accumulator register r of tile m for
@@ -47,7 +50,7 @@ constexpr int sym_per_simd() { return N <= 6 ? 2 : 1; }
 
 // LDS of a block: the operator fragments and, where they fit beside them, one group's nodal values per wavefront (the
 // volume, the own traces and the update all read them from there, so that no registers hold them; at order 8 they do
-// not fit, at order 1 the three nodes per variable are registers' work: 37.3 against 38.5 us at K = 131072)
+// not fit, at order 1 the three nodes per variable are registers' work)
 template <int N, int NV>
 struct SymLds {
     static constexpr size_t frag = dma_span(size_t(SymDims<N>::nF) * sizeof(double));
@@ -90,6 +93,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
     using VF = VolumeFlux<PHYS, double>;
     constexpr int NV = VF::NV, Np = D::Np, Nfp = D::Nfp, Nfq = D::Nfq, SF = D::SF;
     constexpr int KE = D::KE, KO = D::KO, ME = D::ME, MO = D::MO;
+    constexpr int KOA = KO ? KO : 1, MOA = MO ? MO : 1;   // array lengths
     constexpr int WPB = sym_waves<N>();
     constexpr size_t GS = size_t(NV) * Np * 16;
     constexpr size_t kFrBytes = size_t(D::nF) * sizeof(double);
@@ -124,14 +128,14 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
 
     // byte offsets of this lane's node pairs inside a variable's block of a group: unsigned, so that an access is a
     // scalar base plus one 32-bit lane offset
-    unsigned na[KE], nb[KO];
+    unsigned na[KE], nb[KOA];
 #pragma unroll
     for (int s = 0; s < KE; ++s) {
         const unsigned ab = unsigned(a.fmask[4 * s + rg]);
         na[s] = ((ab & 255u) * 16 + col) * 8;
         if (s < KO) nb[s < KO ? s : 0] = ((ab >> 8) * 16 + col) * 8;
     }
-    auto load_nodes = [&](const double* src, double (&x)[NV][KE], double (&y)[NV][KO]) {
+    auto load_nodes = [&](const double* src, double (&x)[NV][KE], double (&y)[NV][KOA]) {
 #pragma unroll
         for (int v = 0; v < NV; ++v)
 #pragma unroll
@@ -140,7 +144,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
                 if (s < KO) y[v][s < KO ? s : 0] = at_lane(src + v * Np * 16, nb[s < KO ? s : 0]);
             }
     };
-    auto load_old = [&](const double* src, double (&x)[NV][KE], double (&y)[NV][KO]) {
+    auto load_old = [&](const double* src, double (&x)[NV][KE], double (&y)[NV][KOA]) {
         if (a.res_in) {
             load_nodes(src, x, y);
         } else {
@@ -164,16 +168,16 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
         const double* old_g = a.res_in + size_t(grp) * GS;
         const double* qn = kLds ? qw : qg;
         // sums and differences of the node pairs: kept in registers, or formed from LDS for every point tile
-        double qe[kLds ? 1 : NV][KE], qo[kLds ? 1 : NV][KO];
+        double qe[kLds ? 1 : NV][KE], qo[kLds ? 1 : NV][KOA];
         if constexpr (!kLds) {
-            double xa[NV][KE], xb[NV][KO];
+            double xa[NV][KE], xb[NV][KOA];
             load_nodes(qg, xa, xb);
 #pragma unroll
             for (int v = 0; v < NV; ++v)
 #pragma unroll
                 for (int s = 0; s < KE; ++s) {
                     const int so = s < KO ? s : 0;
-                    qe[v][s] = xa[v][s] + (s < KO ? xb[v][so] : xa[v][s]);
+                    qe[v][s] = D::whole ? xa[v][s] : xa[v][s] + (s < KO ? xb[v][so] : xa[v][s]);
                     if (s < KO) qo[v][so] = xa[v][s] - xb[v][so];
                 }
         }
@@ -198,7 +202,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
         // they would spill and the SIMD's other wavefront hides them
         double own0[Nfp], oth0[Nfp], own1[Nfp], oth1[Nfp], own2[Nfp], oth2[Nfp], nx0, ny0, fs0, nx1, ny1, fs1, nx2, ny2, fs2;
         bool keep0, keep1, keep2;
-        double ra[NV][KE], rb[NV][KO], ua[NV][KE], ub[NV][KO];
+        double ra[NV][KE], rb[NV][KOA], ua[NV][KE], ub[NV][KOA];
         if constexpr (kEarly) {
             keep0 = load_face(0, own0, oth0);
             keep2 = load_face(2, own2, oth2);
@@ -209,7 +213,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
             if constexpr (UPDATE) load_old(old_g, ra, rb);
         }
 
-        d4_t accE[NV][ME], accO[NV][MO];
+        d4_t accE[NV][ME], accO[NV][MOA];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
 #pragma unroll
@@ -241,7 +245,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
                     double be, bo;
                     if constexpr (kLds) {
                         const double x = at_lane(qw + v * Np * 16, na[s]), y = s < KO ? at_lane(qw + v * Np * 16, nb[so]) : x;
-                        be = x + y;
+                        be = D::whole ? x : x + y;
                         bo = x - y;
                     } else {
                         be = qe[v][s];
@@ -259,7 +263,20 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
                 // zero state is not finite
                 const bool pad = 4 * ks + 3 >= D::qrow && 4 * ks + rg >= D::qrow;
                 double q1[NV], fr1[NV], fs1[NV];
-                if (ks < D::KP) {
+                if constexpr (D::whole) {
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) q1[v] = ce[v][r];
+                    VF::eval(q1, a.ax, a.ay, a.gamma, rx, ry, sx, sy, fr1, fs1);
+                    const double* A = P + size_t(2 * ks) * ME * 64 + lane;
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) {
+                        if (pad) fr1[v] = fs1[v] = 0.0;
+#pragma unroll
+                        for (int m = 0; m < ME; ++m) accE[v][m] = mfma4(A[m * 64], fr1[v], accE[v][m]);
+#pragma unroll
+                        for (int m = 0; m < ME; ++m) accE[v][m] = mfma4(A[(ME + m) * 64], fs1[v], accE[v][m]);
+                    }
+                } else if (ks < D::KP) {
                     double q2[NV], fr2[NV], fs2[NV];
 #pragma unroll
                     for (int v = 0; v < NV; ++v) {
@@ -367,10 +384,17 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
             for (int j = 0; j < SF; ++j) {
                 double b0[NV], b2[NV];
                 face_flux(0, j, false, own0, oth0, keep0, nx0, ny0, fs0, b0);
-                face_flux(2, j, true, own2, oth2, keep2, nx2, ny2, fs2, b2);
+                face_flux(2, j, !D::whole, own2, oth2, keep2, nx2, ny2, fs2, b2);
                 const double* A = L + size_t(j) * (ME + MO) * 64 + lane;
 #pragma unroll
                 for (int v = 0; v < NV; ++v) {
+                    if constexpr (D::whole) {
+#pragma unroll
+                        for (int m = 0; m < ME; ++m) accE[v][m] = mfma4(A[m * 64], b0[v], accE[v][m]);
+#pragma unroll
+                        for (int m = 0; m < ME; ++m) accE[v][m] = mfma4(A[(SF * ME + m) * 64], b2[v], accE[v][m]);
+                        continue;
+                    }
                     const double s = b0[v] + b2[v], d = b0[v] - b2[v];
 #pragma unroll
                     for (int m = 0; m < ME; ++m) accE[v][m] = mfma4(A[m * 64], s, accE[v][m]);
@@ -389,7 +413,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
             for (int j = 0; j < SF; ++j) {
                 double b1[NV];
                 face_flux(1, j, false, own1, oth1, keep1, nx1, ny1, fs1, b1);
-                const double* A = L + size_t(SF + j) * (ME + MO) * 64 + lane;
+                const double* A = L + size_t((D::whole ? 2 : 1) * SF + j) * (ME + MO) * 64 + lane;
 #pragma unroll
                 for (int v = 0; v < NV; ++v) {
 #pragma unroll
@@ -476,7 +500,11 @@ static hipError_t launch_sym_inst(const StageArgs& a, int ncu, hipStream_t st) {
         per_cu = n < 1 ? 1 : n;
     }
     const int groups = (a.K + 15) / 16;
-    int nb = groups < ncu * per_cu ? groups : ncu * per_cu;   // a persistent grid
+    // a persistent grid: a block per group up to one per compute unit, then more only as their wavefronts fill (the
+    // wavefronts of a block take groups apart, so that with more blocks than that each leaves its last SIMDs idle; as
+    // many as are resident, order 1 LF, K = 32768: 11.6 -> 9.6 us, order 2 Roe, K = 11834: 11.3 -> 8.0)
+    const int full = (groups + sym_waves<N>() - 1) / sym_waves<N>(), least = groups < ncu ? groups : ncu;
+    int nb = full < least ? least : full < ncu * per_cu ? full : ncu * per_cu;
     nb = nb < 8 ? 8 : (nb + 7) / 8 * 8;
     if (a.block_cap > 0 && nb > a.block_cap) nb = a.block_cap < 8 ? 8 : a.block_cap / 8 * 8;
     hipLaunchKernelGGL((stage_sym_kernel<N, PHYS, FLUX, UPDATE>), dim3(nb), dim3(threads), 0, st, a);
