@@ -73,13 +73,19 @@ __device__ __forceinline__ f4_t mfma3(const uint4 A, const Split4& B, f4_t c) {
 // before).  A block's waves take groups apart, so that every compute unit gets one before any gets two: K = 11834, N = 6
 // FP32 50.8 -> 25.5 us, bf16x3 23.3 -> 20.5 us.  When
 // they fit, the operator fragments are staged into LDS once per block and shared by its waves.
-template <int N, typename T, bool SPLIT = false>
-constexpr int waves_per_block() { return N <= 6 ? 8 : 4; }
+// bf16x3 advection up to order 4 keeps four: its kernels are short and small enough that several blocks share a compute
+// unit (with eight, order 3: 6.0 -> 7.7 us at K = 2048, 8.7 at 11834).
+template <int N, int NV, typename T, bool SPLIT>
+constexpr int waves_per_block() { return N <= 6 && !(SPLIT && NV == 1 && N <= 4) ? 8 : 4; }
+
+// the kernels that give a block's wavefronts adjacent groups (stage_kernel says when)
+template <int N, int NV, bool SPLIT>
+constexpr bool packs() { return SPLIT && NV == 1 && N <= 4; }
 
 // wavefronts per SIMD that the scheduler may aim at: no more than the block brings (the LDS holds one block), so that
 // it does not trade the batching of loads for an occupancy that cannot be had; small kernels as many as fit
 template <int N, int PHYS, typename T, bool SPLIT>
-constexpr int stage_per_simd() { return PHYS == PHYS_EULER && N >= 3 ? waves_per_block<N, T, SPLIT>() / 4 : 8; }
+constexpr int stage_per_simd() { return PHYS == PHYS_EULER && N >= 3 ? waves_per_block<N, 4, T, SPLIT>() / 4 : 8; }
 
 template <int N, int NV, typename T, bool SPLIT>
 struct StageLds {
@@ -87,7 +93,7 @@ struct StageLds {
     static constexpr int NFI = 4 * D::SF;
     static constexpr int TR_G = NV * 16 + 16;              // padded stride of one Gauss point (bank spread)
     static constexpr size_t trace_wave = size_t(NFI) * TR_G;   // one face: [g][v][col]
-    static constexpr int WPB = waves_per_block<N, T, SPLIT>();
+    static constexpr int WPB = waves_per_block<N, NV, T, SPLIT>();
     static constexpr size_t trace_elems = size_t(WPB) * trace_wave;
     static constexpr size_t budget = 150 * 1024 / sizeof(T);
     // fragment sizes in T-sized units (the bf16x3 fragments count 32-bit words)
@@ -113,7 +119,7 @@ struct StageLds {
 
 // SPLIT: bf16x3 split products for the three contractions (T = float for everything else)
 template <int N, int PHYS, typename T, bool SPLIT, bool MOM, int FLUX, bool UPDATE>
-__global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
+__global__ __launch_bounds__((64 * waves_per_block<N, VolumeFlux<PHYS, T>::NV, T, SPLIT>()))
     __attribute__((amdgpu_waves_per_eu(1, stage_per_simd<N, PHYS, T, SPLIT>())))
     void stage_kernel(StageArgs a) {
     using D = Dims<N>;
@@ -188,7 +194,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
     const int bx = blockIdx.x >> 3;
     const int g_lo = int((long long)groups * xcd / 8);
     const int g_hi = int((long long)groups * (xcd + 1) / 8);
-    constexpr int WPB = waves_per_block<N, T, SPLIT>();
+    constexpr int WPB = waves_per_block<N, NV, T, SPLIT>();
 
 
     // The connectivity of the next group is fetched one iteration ahead.  With the prefetch buffer, so are its
@@ -196,7 +202,12 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
     // by the next group, and since vector memory operations complete in order, waiting for any of them early
     // would also wait for the DMA.
     const int gstride = nbx * WPB;
-    int grp = g_lo + wave * nbx + bx;   // a block's wavefronts nbx groups apart: a small mesh spreads over the chip first
+    // A block's wavefronts nbx groups apart, so that a small mesh spreads over the chip first; adjacent groups for bf16x3
+    // advection (up to order 4) once every wavefront has one, for what its faces then find in the cache (order 1,
+    // K = 131072: 10.9 -> 9.6 us, order 3: 18.5 -> 18.0), and at orders 1 and 2 always (see launch_inst)
+    const bool packed = packs<N, NV, SPLIT>() && (N <= 2 || groups >= int(gridDim.x) * WPB);
+    const int wstep = packed ? 1 : nbx, bstep = packed ? WPB : 1;
+    int grp = g_lo + wave * wstep + bx * bstep;
     int cn_next[3] = {0, 0, 0};
     T geo_next[4] = {T(0), T(0), T(0), T(0)};
     if (grp < g_hi) {
@@ -448,6 +459,14 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
             }
         };
 
+        // Where the registers allow it the update's loads are requested here and arrive behind the faces: advection in
+        // bf16x3, and in FP32 up to order 3 (order 3, K = 11834: 7.3 -> 6.8 us), Euler in bf16x3 up to order 2 (order 1
+        // LF, K = 262144: 48.5 -> 46.5 us; order 2 Roe, K = 32768: 14.6 -> 13.4).  Beyond, the registers cost more than
+        // the wait: FP32 LF, K = 131072, order 1 26.5 -> 29.7, order 3 57.7 -> 61; FP32 advection, order 4, K = 216
+        // 7.0 -> 7.6.
+        constexpr bool kHoist = SPLIT ? NV == 1 || N <= 2 : NV == 1 && N <= 3;
+        if constexpr (UPDATE && kHoist) load_update();
+
         // ---- faces.  The other side's face nodes of all three faces (lane (col, rg): variable rg) are requested
         // together, so their latency is paid once and behind other work rather than once per face: bf16x3 requests
         // them at the group start (above) and holds them through the volume phase, FP32 with one wave per SIMD before
@@ -609,7 +628,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
         // order and with its fragments (so the two give the same bits); rows beyond Np enter as zeros.  (FP32 and FP64
         // leave the moments to the limiter's own kernel.)
         // every load of the update before its first store: the compiler keeps loads behind stores that could alias
-        if constexpr (UPDATE) load_update();
+        if constexpr (UPDATE && !kHoist) load_update();
         const bool want_mom = kMom;   // the launcher takes this instantiation for a moments output and an update
         double mpart[kMom ? NV : 1][4];   // the moments' per-lane partial sums (lim_moments.hpp)
 #pragma unroll
@@ -657,7 +676,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, T, SPLIT>()))
 // XCD gets the same share), capped by the number of element groups.
 template <int N, int PHYS, typename T, bool SPLIT, bool MOM, int FLUX, bool UPDATE>
 static hipError_t launch_inst(const StageArgs& a, int ncu, hipStream_t st) {
-    constexpr int threads = 64 * waves_per_block<N, T, SPLIT>();
+    constexpr int threads = 64 * waves_per_block<N, VolumeFlux<PHYS, T>::NV, T, SPLIT>();
     static int per_cu = -1;
     if (per_cu < 0) {
         int n = 0;
@@ -666,8 +685,15 @@ static hipError_t launch_inst(const StageArgs& a, int ncu, hipStream_t st) {
             n = 1;
         per_cu = n < 1 ? 1 : n;
     }
+    // A block per group up to one per compute unit, then more only as their wavefronts fill (the wavefronts take groups
+    // apart, so that with more blocks than that each leaves its last SIMDs idle: FP32, K = 11834, order 2 LF 11.7 -> 9.8 us,
+    // order 3 16.9 -> 13.9).  bf16x3 advection at orders 1 and 2 starts with full blocks: another block's copy of the
+    // operators takes longer than a group does (order 2, K = 2048: 5.9 -> 5.6 us).
+    constexpr int wpb = threads / 64;
+    constexpr bool pack = packs<N, VolumeFlux<PHYS, T>::NV, SPLIT>() && N <= 2;
     const int groups = (a.K + 15) / 16;
-    int nb = groups < ncu * per_cu ? groups : ncu * per_cu;
+    const int full = (groups + wpb - 1) / wpb, least = pack ? 0 : groups < ncu ? groups : ncu;
+    int nb = full < least ? least : full < ncu * per_cu ? full : ncu * per_cu;
     nb = nb < 8 ? 8 : (nb + 7) / 8 * 8;
     if (a.block_cap > 0 && nb > a.block_cap) nb = a.block_cap < 8 ? 8 : a.block_cap / 8 * 8;
     hipLaunchKernelGGL((stage_kernel<N, PHYS, T, SPLIT, MOM, FLUX, UPDATE>), dim3(nb), dim3(threads), 0, st, a);
