@@ -365,7 +365,7 @@ __device__ __forceinline__ void update_load(const SipgArgs<T>& a, const CgLoop<T
 // Jacobi 32.2 -> 32.2, point Jacobi 31.5 -> 30.6; order 4 block 24.0 -> 23.4; order 6, 18432 elements 31.8 -> 30.5; order 3,
 // 2640 elements 12.8 -> 12.5).
 template <int N, typename T, bool BLOCK, bool INIT>
-__global__ __launch_bounds__(256, N <= 6 ? 2 : 1) void cg_update_kernel(SipgArgs<T> a, CgLoop<T> c,
+__global__ __launch_bounds__(256, N <= 3 ? 4 : N <= 6 ? 2 : 1) void cg_update_kernel(SipgArgs<T> a, CgLoop<T> c,
                                                         const CgState* __restrict__ st_in, CgState* __restrict__ st_out,
                                                         const double* __restrict__ pb_in, double* __restrict__ pb_out) {
     constexpr SipgTiles S(N);
