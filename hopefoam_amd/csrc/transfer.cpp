@@ -4,7 +4,8 @@
 // its two slots: while the device packs (or unpacks) one, the worker copies the other from (or to) the caller's memory.
 // One worker copies about 30 GB/s; the first touch of a fresh result array costs as much again; the workers share both.
 // Small transfers stay on the calling thread.  Measured, up / down: 117 MB 38.8 / 45.7 ms -> 2.9 / 3.3 ms, 42 MB 15.5 /
-// 19.8 -> 1.1 / 1.5 ms, 4.2 MB 306 / 825 -> 145 / 159 us, 0.25 MB 27 / 29 -> 23 / 25 us, 35 KB 27 / 13 -> 17 / 17 us.
+// 19.8 -> 1.1 / 1.5 ms, 4.2 MB 306 / 825 -> 145 / 159 us, 0.7 MB 55 / 61 -> 36 / 38 us, 0.24 MB 25 / 27 -> 21 / 22 us;
+// pageable copies of 1 to 80 KB took 12 to 30 us (by where the caller's memory lies), these take 13 to 16.
 #include "transfer.hpp"
 
 #include <algorithm>
@@ -18,9 +19,10 @@
 namespace dg {
 
 // Data that pays for one more worker (a thread costs some tens of microseconds to start: with a worker per 2 MiB a field
-// of 4 MB took 210 us up, with one 146), and the smallest chunk worth a launch of its own.
+// of 4 MB took 210 us up, with one 146), and the smallest chunk worth a launch of its own (0.3 MB in two chunks 30 / 28 us,
+// in one 24 / 26).
 static constexpr size_t kWorkerBytes = size_t(8) << 20;
-static constexpr size_t kChunkLeast = size_t(256) << 10;
+static constexpr size_t kChunkLeast = size_t(512) << 10;
 
 bool Staging::ready() {
     if (mem) return true;
@@ -88,11 +90,11 @@ hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArr
     const int step = std::max(per, std::min(most, int(kChunkLeast / (size_t(16) * a.Np * sizeof(double)))));
     const int chunks = (tiles + step - 1) / step;
     workers = std::min(workers, chunks);
-    if (chunks == 1) {   // nothing to overlap: no event, no worker
+    if (chunks == 1) {   // nothing to overlap
         if (to_device) std::memcpy(st.slot(0), host, bytes);
-        const hipError_t err = to_device ? launch_unpack_tiles(a, 0, tiles, st.slot(0), s)
-                                         : launch_pack_tiles(a, 0, tiles, st.slot(0), s);
-        const hipError_t done = hipStreamSynchronize(s);
+        const hipError_t err = to_device ? launch_unpack_tiles(a, 0, tiles, st.slot(0), s, st.ev[0])
+                                         : launch_pack_tiles(a, 0, tiles, st.slot(0), s, st.ev[0]);
+        const hipError_t done = err == hipSuccess ? hipEventSynchronize(st.ev[0]) : hipStreamSynchronize(s);
         if (err != hipSuccess || done != hipSuccess) return err != hipSuccess ? err : done;
         if (!to_device) std::memcpy(host, st.slot(0), bytes);
         return hipSuccess;
@@ -133,8 +135,8 @@ hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArr
             range(c, t0, t1, h, nb);
             double* slot = st.slot(2 * w + k);
             if (to_device) std::memcpy(slot, h, nb);
-            if (!check(to_device ? launch_unpack_tiles(a, t0, t1, slot, s) : launch_pack_tiles(a, t0, t1, slot, s)) ||
-                !check(hipEventRecord(st.ev[2 * w + k], s)))
+            const hipEvent_t ev = st.ev[2 * w + k];
+            if (!check(to_device ? launch_unpack_tiles(a, t0, t1, slot, s, ev) : launch_pack_tiles(a, t0, t1, slot, s, ev)))
                 break;
             pending[k] = c;
         }

@@ -34,9 +34,9 @@ struct Staging {
     double* slot(int i) const { return mem + size_t(i) * (kSlotBytes / sizeof(double)); }
 };
 
-// tiles [t0, t1) of a from / to the packed host order at host (device-accessible memory)
-hipError_t launch_unpack_tiles(const NodalArray& a, int t0, int t1, const double* host, hipStream_t s);
-hipError_t launch_pack_tiles(const NodalArray& a, int t0, int t1, double* host, hipStream_t s);
+// tiles [t0, t1) of a from / to the packed host order at host (device-accessible memory); done is recorded with the kernel
+hipError_t launch_unpack_tiles(const NodalArray& a, int t0, int t1, const double* host, hipStream_t s, hipEvent_t done);
+hipError_t launch_pack_tiles(const NodalArray& a, int t0, int t1, double* host, hipStream_t s, hipEvent_t done);
 
 // the whole array from / to host memory, ordered behind the work on stream s and complete on return
 hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArray& a, double* host, bool to_device);
