@@ -358,29 +358,50 @@ __device__ __forceinline__ double admissible_fraction(const double (&m)[4], cons
     return lo;
 }
 
-// One wavefront per group of 16 cells (lane: cell lane % 16, nodes 4 s + lane / 16).  The state at the points is the
+// About that fraction, to choose the point that is bisected first: (p - ec) rho is a quadratic in t, positive at 0
+__device__ __forceinline__ double fraction_estimate(const double (&m)[4], const double (&x)[4], double gamma, double ec) {
+    const double d0 = x[0] - m[0], d1 = x[1] - m[1], d2 = x[2] - m[2], d3 = x[3] - m[3], g1 = gamma - 1.0;
+    const double f0 = g1 * (m[3] * m[0] - 0.5 * (m[1] * m[1] + m[2] * m[2])) - ec * m[0];
+    const double f1 = g1 * (d3 * m[0] + m[3] * d0 - (m[1] * d1 + m[2] * d2)) - ec * d0;
+    const double f2 = g1 * (d3 * d0 - 0.5 * (d1 * d1 + d2 * d2));
+    const double t = 2.0 * f0 / (sqrt(fmax(f1 * f1 - 4.0 * f0 * f2, 0.0)) - f1);
+    return t >= 0.0 ? t : 0.0;   // not a number: first
+}
+
+// One wavefront screens a group of 16 cells (lane: cell lane % 16, nodes 4 s + lane / 16).  The state at the points is the
 // point operator times the group's nodal values on the matrix cores, 16 rows at a time (posf: row 0 the cell mean, then
 // the points; register r of a tile is row 16 t + 4 r + lane / 16, all four variables in the same lane).  Nearly every
-// group is admissible everywhere: a first pass over the tiles takes the least density and asks of each point only
+// group is admissible everywhere: the pass over the tiles takes the least density and asks of each point only
 // whether its pressure is above the bound by more than rounding, without a quotient; only a group with a cell that fails
-// this goes through the points again with the density scaled, the pressure itself and the bisection.
-// The evaluation bounds it (order 3: 4 x 3 products per tile of 16 rows); before, 256 lanes of a block evaluated the
-// points from LDS between block barriers.  Four groups a block read the same operator tiles (one group a
-// block: order 3 22.3, 5 20.2, 6 86.9 us).  us per call beyond the limiter's, the results bit for bit the same:
-//   131072 cells: order 2 33 -> 11.4   3 61 -> 21.2   6 625 -> 74.8      32768: 5 52 -> 14.3      8192: 8 72 -> 23.3
-template <int N>
-__global__ __launch_bounds__(256) void positivity_kernel(LimArgs a, double* __restrict__ q) {
+// this goes through the points again, with the density scaled, the pressure itself and the bisection.
+// The evaluation bounds the screening (order 3: 4 x 3 products per tile of 16 rows).  Four groups a block (W = 1) read the
+// same operator tiles (one group a block, K = 131072: order 3 22.3 us, 6 86.9); with few groups W = 4 wavefronts share one
+// group's tiles.
+// The bisection bounds a group that fails: 60 dependent pressures are about 5 us.  A tile's point of the least estimated
+// fraction is bisected first and the fraction found passed to the cell's other lanes after each tile, so that the other
+// points mostly end at one look; the block's wavefronts share the tiles of the groups that fail, unless so many of
+// the four fail that each does better with its own.  us per limiter call on a fresh copy of its input, with no cell,
+// half of them and all of them failing; 256 lanes a group, a wavefront a group that bisects alone, now:
+//   order 6, K = 2048:    none 35.2, 28.6, 21.4   half 91, 400, 44    all 81, 434, 44
+//   order 2, K = 11834:   none 18.8, 17.9, 17.0   half 55, 88, 42     all 50, 88, 42
+//   order 3, K = 131072:  none 102, 62.8, 61.7    half 461, 484, 206  all 479, 502, 210
+template <int N, int W>
+__global__ __launch_bounds__(256, W == 1 && N <= 4 ? 4 : 1) void positivity_kernel(LimArgs a, double* __restrict__ q) {
     constexpr int Np = LShape<N>::Np, NV = 4, NS = lim_ksteps(Np);
+    __shared__ double mean[4][NV][16], least[4][16], frac[2][4][16];   // of groups that fail: cell means, least densities
+    __shared__ int failed[4];
     const int lane = threadIdx.x & 63, col = lane & 15, kg = lane >> 4;
-    const int g = int(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (g >= (a.K + 15) >> 4) return;
-    const bool live = g * 16 + col < a.K;
-    double* qg = q + size_t(g) * NV * Np * 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int groups = (a.K + 15) >> 4, tiles = (a.npos + 16) / 16;
+    constexpr int G = 4 / W;   // groups of a block, screened by W wavefronts each
+    const int g0 = int(blockIdx.x) * G, own = wave / W, part = wave % W;
     double b[NV][NS];
+    auto load = [&](const double* qg) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v)
+        for (int v = 0; v < NV; ++v)
 #pragma unroll
-        for (int s = 0; s < NS; ++s) b[v][s] = 4 * s + kg < Np ? qg[unsigned(v * Np * 16 + 64 * s + lane)] : 0.0;
+            for (int s = 0; s < NS; ++s) b[v][s] = 4 * s + kg < Np ? qg[unsigned(v * Np * 16 + 64 * s + lane)] : 0.0;
+    };
     const double* F = a.posf + lane;
     auto points = [&](int t, lim_d4 (&x)[NV]) {
         double f[NS];
@@ -393,73 +414,148 @@ __global__ __launch_bounds__(256) void positivity_kernel(LimArgs a, double* __re
 #pragma unroll
             for (int v = 0; v < NV; ++v) x[v] = mfma_f64(f[s], b[v][s], x[v]);
     };
-    const int tiles = (a.npos + 16) / 16;
-    double m[4] = {0.0, 0.0, 0.0, 0.0}, ec = 0.0, rmin = 1e300;
-    bool adm = false, fails = false;
-    for (int t = 0; t < tiles; ++t) {
-        lim_d4 x[NV];
-        points(t, x);
-        if (t == 0) {
+    double m[4] = {0.0, 0.0, 0.0, 0.0}, ec = 0.0;
+    bool adm = false;
+    auto bound = [&]() {
+        const double pb = pressure(m[0], m[1], m[2], m[3], a.gamma);
+        adm = m[0] > 0.0 && pb > 0.0;
+        ec = fmin(a.eps, fmin(m[0], pb));
+    };
+
+    // ---- screening
+    const int g = g0 + own;
+    bool any = false;
+    if (g < groups) {
+        double rmin = 1e300;
+        bool fails = false;
+        load(q + size_t(g) * NV * Np * 16);
+        for (int t = 0; t < tiles; t += t == 0 && part ? part : W) {
+            lim_d4 x[NV];
+            points(t, x);
+            if (t == 0) {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) m[v] = __shfl(x[v][0], col, 64);
-            const double pb = pressure(m[0], m[1], m[2], m[3], a.gamma);
-            adm = m[0] > 0.0 && pb > 0.0;
-            ec = fmin(a.eps, fmin(m[0], pb));
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = 16 * t + 4 * r + kg;
-            if (row >= 1 && row <= a.npos) {
-                const double rho = x[0][r], m2 = 0.5 * (x[1][r] * x[1][r] + x[2][r] * x[2][r]), e = x[3][r] * rho;
-                rmin = fmin(rmin, rho);
-                // (p - ec) rho > 0 by more than the rounding of either form
-                const double d = (a.gamma - 1.0) * (e - m2) - ec * rho;
-                const double err = 1e-12 * (fabs(a.gamma - 1.0) * (fabs(e) + m2) + fabs(ec * rho));
-                fails |= !(rho > 0.0 && d > err);
+                for (int v = 0; v < NV; ++v) m[v] = __shfl(x[v][0], col, 64);
+                bound();
+                if (part) continue;   // the points of tile 0 are the group's first wavefront's
             }
-        }
-    }
-    fails = live && adm && (fails || rmin < ec);
-    if (__ballot(fails) == 0ull) return;
-    // density
-    rmin = fmin(rmin, __shfl_xor(rmin, 16, 64));
-    rmin = fmin(rmin, __shfl_xor(rmin, 32, 64));
-    const bool s1 = adm && rmin < ec;
-    const double t1 = s1 ? (m[0] - ec) / (m[0] - rmin) : 1.0;
-    if (s1) {
 #pragma unroll
-        for (int s = 0; s < NS; ++s) b[0][s] = m[0] + t1 * (b[0][s] - m[0]);
-    }
-    if (kg + 4 * (NS - 1) >= Np) b[0][NS - 1] = 0.0;
-    __builtin_amdgcn_wave_barrier();
-    // pressure
-    double tmin = 1.0;
-    for (int t = 0; t < tiles; ++t) {
-        lim_d4 x[NV];
-        points(t, x);
-        if (adm)
             for (int r = 0; r < 4; ++r) {
                 const int row = 16 * t + 4 * r + kg;
-                const double ux[4] = {x[0][r], x[1][r], x[2][r], x[3][r]};
-                if (row < 1 || row > a.npos || pressure(ux[0], ux[1], ux[2], ux[3], a.gamma) >= ec) continue;
-                tmin = fmin(tmin, admissible_fraction(m, ux, a.gamma, ec, tmin));
+                if (row >= 1 && row <= a.npos) {
+                    const double rho = x[0][r], m2 = 0.5 * (x[1][r] * x[1][r] + x[2][r] * x[2][r]), e = x[3][r] * rho;
+                    rmin = fmin(rmin, rho);
+                    // (p - ec) rho > 0 by more than the rounding of either form
+                    const double d = (a.gamma - 1.0) * (e - m2) - ec * rho;
+                    const double err = 1e-12 * (fabs(a.gamma - 1.0) * (fabs(e) + m2) + fabs(ec * rho));
+                    fails |= !(rho > 0.0 && d > err);
+                }
             }
+        }
+        fails = g * 16 + col < a.K && adm && (fails || rmin < ec);
+        any = __ballot(fails) != 0ull;
+        if (W > 1 || any) {
+            rmin = fmin(rmin, __shfl_xor(rmin, 16, 64));
+            rmin = fmin(rmin, __shfl_xor(rmin, 32, 64));
+            if (kg == 0) {
+                least[wave][col] = rmin;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) mean[wave][v][col] = m[v];
+            }
+        }
+    }
+    // ---- groups that fail: every wavefront takes every fourth tile of each, or, when that makes more rounds, each its own
+    // (at orders 1 and 2, of two and three tiles, always, without waiting for the others)
+    constexpr bool kSolo = W == 1 && N <= 2;
+    bool alone = kSolo;
+    if constexpr (kSolo) {
+        if (!any) return;
         __builtin_amdgcn_wave_barrier();
+    } else {
+        if (lane == 0) failed[wave] = any;
+        __syncthreads();
+        alone = W == 1 && (failed[0] + failed[1] + failed[2] + failed[3]) * ((tiles + 3) / 4) >= tiles;
     }
-    tmin = fmin(tmin, __shfl_xor(tmin, 16, 64));
-    tmin = fmin(tmin, __shfl_xor(tmin, 32, 64));
-    const bool s2 = adm && tmin < 1.0, scaled = live && (s1 || s2);
-    if (scaled) {
+    int buf = 0;   // buffer of frac: written again only behind the next group's barrier
+    for (int k = 0; k < (alone ? 1 : G); ++k) {
+        const int i = alone ? wave : k;
+        int fail = kSolo;
+        for (int w = 0; w < W && !kSolo; ++w) fail |= failed[i * W + w];
+        if (!fail) continue;
+        double* qg = q + size_t(g0 + i) * NV * Np * 16;
+        const bool live = (g0 + i) * 16 + col < a.K;
+        if (G > 1) load(qg);
 #pragma unroll
-        for (int v = 0; v < NV; ++v)
+        for (int v = 0; v < NV; ++v) m[v] = mean[i * W][v][col];
+        bound();
+        double rmin = least[i * W][col];
+        for (int w = 1; w < W; ++w) rmin = fmin(rmin, least[i * W + w][col]);
+        // density
+        const bool s1 = adm && rmin < ec;
+        const double t1 = s1 ? (m[0] - ec) / (m[0] - rmin) : 1.0;
+        if (s1) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s)
-                if (4 * s + kg < Np)
-                    qg[unsigned(v * Np * 16 + 64 * s + lane)] = s2 ? m[v] + tmin * (b[v][s] - m[v]) : b[v][s];
+            for (int s = 0; s < NS; ++s) b[0][s] = m[0] + t1 * (b[0][s] - m[0]);
+        }
+        if (kg + 4 * (NS - 1) >= Np) b[0][NS - 1] = 0.0;
+        __builtin_amdgcn_wave_barrier();
+        // pressure
+        double tmin = 1.0;
+        for (int t = alone ? 0 : wave; t < tiles; t += alone ? 1 : 4) {
+            lim_d4 x[NV];
+            points(t, x);
+            if (adm) {
+                unsigned need = 0;
+                double first[4] = {0.0, 0.0, 0.0, 0.0}, te = 2.0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = 16 * t + 4 * r + kg;
+                    const double ux[4] = {x[0][r], x[1][r], x[2][r], x[3][r]};
+                    if (row >= 1 && row <= a.npos && !(pressure(ux[0], ux[1], ux[2], ux[3], a.gamma) >= ec)) {
+                        need |= 1u << r;
+                        const double e = fmin(fraction_estimate(m, ux, a.gamma, ec), 1.0);
+                        if (e < te) {
+                            te = e;
+#pragma unroll
+                            for (int v = 0; v < NV; ++v) first[v] = ux[v];
+                        }
+                    }
+                }
+                if (need) {
+                    tmin = fmin(tmin, admissible_fraction(m, first, a.gamma, ec, tmin));
+                    for (int r = 0; r < 4; ++r) {
+                        const double ux[4] = {x[0][r], x[1][r], x[2][r], x[3][r]};
+                        if (need >> r & 1) tmin = fmin(tmin, admissible_fraction(m, ux, a.gamma, ec, tmin));
+                    }
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            tmin = fmin(tmin, __shfl_xor(tmin, 16, 64));
+            tmin = fmin(tmin, __shfl_xor(tmin, 32, 64));
+        }
+        if (!alone) {
+            if (kg == 0) frac[buf][wave][col] = tmin;
+            __syncthreads();   // also: every wavefront has read the group
+            for (int w = 0; w < 4; ++w) tmin = fmin(tmin, frac[buf][w][col]);
+            buf ^= 1;
+        }
+        const bool s2 = adm && tmin < 1.0, scaled = live && (s1 || s2);
+        if (scaled) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                if (alone || v == wave) {
+#pragma unroll
+                    for (int s = 0; s < NS; ++s)
+                        if (4 * s + kg < Np)
+                            qg[unsigned(v * Np * 16 + 64 * s + lane)] = s2 ? m[v] + tmin * (b[v][s] - m[v]) : b[v][s];
+                }
+        }
+        const unsigned long long n = __ballot(kg == 0 && scaled);
+        if (lane == 0 && (alone || wave == 0) && n) atomicAdd(a.pcount, unsigned(__popcll(n)));
     }
-    const unsigned long long n = __ballot(kg == 0 && scaled);
-    if (lane == 0 && n) atomicAdd(a.pcount, unsigned(__popcll(n)));
 }
+
+// up to this many groups (two for a compute unit) a group has a block of its own
+constexpr int kShareGroups = 512;
 
 // blocks of the wave-per-group kernels: one group per wavefront
 static int lim_grid(const LimArgs& a, int waves) {
@@ -470,8 +566,13 @@ static int lim_grid(const LimArgs& a, int waves) {
 template <int N, int NV>
 static hipError_t launch_positivity(const LimArgs& a, double* q, hipStream_t s) {
     if constexpr (NV == 4) {
-        if (a.positivity && !a.detect_only)
-            hipLaunchKernelGGL((positivity_kernel<N>), dim3(lim_grid(a, 4)), dim3(256), 0, s, a, q);
+        if (a.positivity && !a.detect_only) {
+            const int groups = lim_grid(a, 1);
+            if (groups <= kShareGroups)
+                hipLaunchKernelGGL((positivity_kernel<N, 4>), dim3(groups), dim3(256), 0, s, a, q);
+            else
+                hipLaunchKernelGGL((positivity_kernel<N, 1>), dim3(lim_grid(a, 4)), dim3(256), 0, s, a, q);
+        }
     }
     return hipGetLastError();
 }
