@@ -24,23 +24,22 @@ namespace dg {
 static constexpr size_t kWorkerBytes = size_t(8) << 20;
 static constexpr size_t kChunkLeast = size_t(512) << 10;
 
-bool Staging::ready() {
-    if (mem) return true;
+bool Staging::ready(int n) {
+    if (slots >= n) return true;
     if (failed) return false;
-    if (hipHostMalloc(reinterpret_cast<void**>(&mem), kSlots * kSlotBytes, hipHostMallocCoherent) != hipSuccess) {
+    double* m = nullptr;
+    failed = hipHostMalloc(reinterpret_cast<void**>(&m), size_t(n) * kSlotBytes, hipHostMallocCoherent) != hipSuccess;
+    for (int i = 0; i < n && !failed; ++i)
+        if (!ev[i]) failed = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) != hipSuccess;
+    if (failed) {
         (void)hipGetLastError();
-        mem = nullptr;
-        failed = true;
+        if (m) (void)hipHostFree(m);
         return false;
     }
-    for (hipEvent_t& e : ev)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            e = nullptr;
-            failed = true;
-        }
-    if (failed) release();
-    return mem != nullptr;
+    if (mem) (void)hipHostFree(mem);   // of fewer slots; no transfer is under way
+    mem = m;
+    slots = n;
+    return true;
 }
 
 void Staging::release() {
@@ -50,6 +49,7 @@ void Staging::release() {
     }
     if (mem) (void)hipHostFree(mem);
     mem = nullptr;
+    slots = 0;
 }
 
 // without pinned memory: one pageable copy of the whole array, reordered by the host
@@ -78,10 +78,9 @@ static hipError_t transfer_pageable(hipStream_t s, const NodalArray& a, double* 
 
 hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArray& a, double* host, bool to_device) {
     std::lock_guard<std::mutex> lock(st.mu);
-    if (!st.ready()) return transfer_pageable(s, a, host, to_device);
     const int tiles = a.nvar * a.tiles_per_var();
     const size_t bytes = size_t(a.nvar) * a.K * a.Np * sizeof(double);
-    // chunks: whole tiles, at most one slot; workers: one per two slots' worth of data, at most one per two slots
+    // chunks: whole tiles, at most one slot; workers: one per kWorkerBytes, at most one per two slots
     int workers = int(std::min<size_t>(Staging::kSlots / 2, bytes / kWorkerBytes));
     if (workers < 1) workers = 1;
     const int most = int(Staging::kSlotBytes / (size_t(16) * a.Np * sizeof(double)));
@@ -90,6 +89,7 @@ hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArr
     const int step = std::max(per, std::min(most, int(kChunkLeast / (size_t(16) * a.Np * sizeof(double)))));
     const int chunks = (tiles + step - 1) / step;
     workers = std::min(workers, chunks);
+    if (!st.ready(chunks == 1 ? 1 : Staging::kSlots)) return transfer_pageable(s, a, host, to_device);
     if (chunks == 1) {   // nothing to overlap
         if (to_device) std::memcpy(st.slot(0), host, bytes);
         const hipError_t err = to_device ? launch_unpack_tiles(a, 0, tiles, st.slot(0), s, st.ev[0])
@@ -165,8 +165,9 @@ hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArr
 hipError_t fetch_small(hipStream_t s, Staging& st, void* host, const void* dev, size_t bytes, void* host2,
                        const void* dev2, size_t bytes2) {
     std::lock_guard<std::mutex> lock(st.mu);
-    const bool pinned = st.mem && bytes <= Staging::kSlotBytes && bytes2 <= Staging::kSlotBytes;
-    void *a = pinned ? st.slot(0) : host, *b = pinned ? st.slot(1) : host2;
+    const size_t at2 = (bytes + 63) / 64 * 64;
+    const bool pinned = st.mem && at2 + bytes2 <= size_t(st.slots) * Staging::kSlotBytes;
+    void *a = pinned ? st.slot(0) : host, *b = pinned ? reinterpret_cast<char*>(st.slot(0)) + at2 : host2;
     hipError_t err = hipSuccess;
     if (dev) err = hipMemcpyAsync(a, dev, bytes, hipMemcpyDeviceToHost, s);
     if (dev2 && err == hipSuccess) err = hipMemcpyAsync(b, dev2, bytes2, hipMemcpyDeviceToHost, s);

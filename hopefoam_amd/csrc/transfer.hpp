@@ -20,16 +20,18 @@ struct NodalArray {
     }
 };
 
-// Pinned staging memory of a context, allocated with its first transfer and freed with the context: kSlots slots, two
-// per worker, so that the copy of one slot overlaps the device's work on the other.
+// Pinned staging memory of a context, allocated with the first transfer that needs it and freed with the context: one slot
+// for transfers of one chunk, else kSlots, two per worker, so that the copy of one slot overlaps the device's work on the
+// other.
 struct Staging {
     static constexpr int kSlots = 16;
     static constexpr size_t kSlotBytes = size_t(1) << 20;   // 16 MiB in all
     std::mutex mu;                 // one transfer at a time
     double* mem = nullptr;
+    int slots = 0;                 // of mem
     hipEvent_t ev[kSlots] = {};
-    bool failed = false;           // no pinned memory: transfers go through pageable copies
-    bool ready();
+    bool failed = false;           // no (more) pinned memory: transfers go through pageable copies
+    bool ready(int n);             // n slots and their events are there
     void release();
     double* slot(int i) const { return mem + size_t(i) * (kSlotBytes / sizeof(double)); }
 };

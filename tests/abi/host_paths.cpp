@@ -148,6 +148,28 @@ static void ensemble_failing_launch() {
     CHECK(dgh_destroy(c) == DGH_OK);
 }
 
+// pinned staging memory: one slot of 1 MiB for transfers of one chunk, all sixteen once a transfer has several, given
+// back with the context
+static void staging_as_needed() {
+    dgh_ctx c = context();
+    int m = -1, f = -1, big = -1, g = -1;
+    CHECK(dgh_mesh_structured(c, 2, 3, 3, 0, 1, 0, 1, 1, 1, 0, &m) == DGH_OK);
+    CHECK(dgh_field_create(c, m, 4, &f) == DGH_OK);
+    CHECK(fake::state().pinned_bytes == 0);
+    std::vector<double> a(size_t(18) * 6 * 4, 1.0);
+    CHECK(dgh_field_upload(c, f, a.data()) == DGH_OK && dgh_field_download(c, f, a.data()) == DGH_OK);
+    CHECK(fake::state().pinned_bytes == size_t(1) << 20);
+    CHECK(dgh_mesh_structured(c, 8, 64, 32, 0, 1, 0, 1, 1, 1, 0, &big) == DGH_OK);
+    CHECK(dgh_field_create(c, big, 4, &g) == DGH_OK);
+    std::vector<double> b(size_t(4096) * 45 * 4, 1.0);
+    CHECK(dgh_field_upload(c, g, b.data()) == DGH_OK);
+    CHECK(fake::state().pinned_bytes == size_t(16) << 20);
+    CHECK(dgh_field_download(c, f, a.data()) == DGH_OK);
+    CHECK(fake::state().pinned_bytes == size_t(16) << 20 && fake::state().pinned.size() == 1);
+    CHECK(dgh_destroy(c) == DGH_OK);
+    CHECK(fake::state().pinned.empty());
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> all = {
         {"error_is_not_kept", error_is_not_kept},
@@ -155,6 +177,7 @@ int main(int argc, char** argv) {
         {"ssprk2_scratch", ssprk2_scratch},
         {"sipg_rhs_threads", sipg_rhs_threads},
         {"ensemble_failing_launch", ensemble_failing_launch},
+        {"staging_as_needed", staging_as_needed},
     };
     CHECK(argc == 2 && all.count(argv[1]));
     all.at(argv[1])();

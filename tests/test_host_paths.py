@@ -48,3 +48,8 @@ def test_sipg_rhs_threads(program):
 def test_ensemble_failing_launch(program):
     """an ensemble call that fails half-way leaves nothing running"""
     run(program, "ensemble_failing_launch")
+
+
+def test_staging_as_needed(program):
+    """a context takes as much pinned memory as its transfers need"""
+    run(program, "staging_as_needed")
