@@ -954,6 +954,17 @@ int dgh_lserk4_run_limited(dgh_ctx c, int mh, const dgh_rhs_desc* d, const dgh_l
     return lserk4_loop(c, mh, d, ld, q, nsteps, dt, ms, "dgh_lserk4_run_limited");
 }
 
+int dgh_selftest_field_raw(dgh_ctx c, int fh, double* raw) {
+    if (!c || !raw) return DGH_ERR_ARG;
+    FieldDev* f = c->field(fh);
+    if (!f) return c->last;
+    (void)hipSetDevice(c->device);
+    return c->hip(hipMemcpyAsync(raw, f->d, f->n * sizeof(double), hipMemcpyDeviceToHost, c->stream), "d2h") &&
+                   c->hip(hipStreamSynchronize(c->stream), "sync")
+               ? DGH_OK
+               : c->last;
+}
+
 int dgh_selftest_mfma(dgh_ctx c, double* err64, double* err32) {
     if (!c || !err64 || !err32) return DGH_ERR_ARG;
     (void)hipSetDevice(c->device);

@@ -479,6 +479,22 @@ extern "C" int dgh_ensemble_get(dgh_ctx c, int h, int i, int what, double* out) 
     return ens_copy(c, *E, i, ENS_QY, out + n, false);
 }
 
+extern "C" int dgh_selftest_ensemble_raw(dgh_ctx c, int h, int i, double* raw) {
+    if (!c) return DGH_ERR_ARG;
+    EnsDev* E = ens_get(c, h);
+    if (!E) return c->last;
+    if (i < 0 || i >= int(E->hc.size()) || !raw)
+        return c->fail(DGH_ERR_ARG, "dgh_selftest_ensemble_raw: case %d", i), DGH_ERR_ARG;
+    (void)hipSetDevice(c->device);
+    const size_t n = size_t(E->hc[i].Kp) * E->hc[i].Np;
+    return c->hip(hipMemcpyAsync(raw, E->data + E->cases[i].off_u + size_t(E->cur) * n, n * sizeof(double),
+                                 hipMemcpyDeviceToHost, c->stream),
+                  "d2h") &&
+                   c->hip(hipStreamSynchronize(c->stream), "sync")
+               ? DGH_OK
+               : c->last;
+}
+
 extern "C" int dgh_ensemble_rhs(dgh_ctx c, int h) {
     if (!c) return DGH_ERR_ARG;
     EnsDev* E = ens_get(c, h);

@@ -154,6 +154,8 @@ def lib():
         "dgh_ensemble_rhs": [vp, C.c_int],
         "dgh_ensemble_run": [vp, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_float)],
         "dgh_ensemble_info": [vp, C.c_int, vp, vp, vp, vp],
+        "dgh_selftest_field_raw": [vp, C.c_int, _dp],
+        "dgh_selftest_ensemble_raw": [vp, C.c_int, C.c_int, _dp],
         "dgh_selftest_mfma": [vp, C.POINTER(C.c_double), C.POINTER(C.c_double)],
         "dgh_selftest_mfma_layout": [vp, _dp],
         "dgh_selftest_mfma_bf16x3": [vp, C.POINTER(C.c_double), C.POINTER(C.c_double)],
@@ -467,6 +469,13 @@ class Field:
         c._ck(c.L.dgh_field_download(c.h, self.h, out), "dgh_field_download")
         return out.reshape(self.shape)
 
+    def raw(self):
+        """the device's groups of 16 elements with their padding, [group][var][node][element]"""
+        out = np.empty((-(-self.mesh.K // 16), self.nvar, self.mesh.Np, 16))
+        c = self.mesh.ctx
+        c._ck(c.L.dgh_selftest_field_raw(c.h, self.h, out.reshape(-1)), "dgh_selftest_field_raw")
+        return out
+
     def copy_from(self, other):
         c = self.mesh.ctx
         c._ck(c.L.dgh_field_copy(c.h, self.h, other.h), "dgh_field_copy")
@@ -599,6 +608,14 @@ class Ensemble:
         out = np.empty(n)
         self.ctx._ck(self.ctx.L.dgh_ensemble_get(self.ctx.h, self.h, i, what, out), "dgh_ensemble_get")
         return out.reshape((2, c["K"], c["Np"]) if what == 2 else (c["K"], c["Np"]))
+
+    def raw(self, i):
+        """the state of case i as the device holds it, [group][node][element], K padded to 64"""
+        c = self.cases[i]
+        out = np.empty((-(-c["K"] // 64) * 4, c["Np"], 16))
+        self.ctx._ck(self.ctx.L.dgh_selftest_ensemble_raw(self.ctx.h, self.h, i, out.reshape(-1)),
+                     "dgh_selftest_ensemble_raw")
+        return out
 
     def rhs(self):
         self.ctx._ck(self.ctx.L.dgh_ensemble_rhs(self.ctx.h, self.h), "dgh_ensemble_rhs")

@@ -389,6 +389,12 @@ int dgh_selftest_mfma_bf16x3(dgh_ctx ctx, double* err3, double* err1);
  * f64 then f32, 4 blocks of 64 lanes x 4 registers (1024 values) */
 int dgh_selftest_mfma_layout(dgh_ctx ctx, double* raw);
 
+/* the field as the device holds it, groups of 16 elements with the padding: value (e, v, n) at
+ * ((e / 16 * nvar + v) * Np + n) * 16 + e % 16, nvar * Np * (K rounded up to 16) values */
+int dgh_selftest_field_raw(dgh_ctx ctx, int field, double* raw);
+/* the same of the state of case i of an ensemble (one variable, K rounded up to 64) */
+int dgh_selftest_ensemble_raw(dgh_ctx ctx, int ens, int i, double* raw);
+
 #ifdef __cplusplus
 }
 #endif
