@@ -561,6 +561,17 @@ extern "C" int dgh_ensemble_run(dgh_ctx c, int h, int nsteps, int use_graph, flo
     return DGH_OK;
 }
 
+extern "C" int dgh_ensemble_set_split(dgh_ctx c, int h, int N, int P) {
+    if (!c) return DGH_ERR_ARG;
+    EnsDev* E = ens_get(c, h);
+    if (!E) return c->last;
+    if (N < 1 || N > 8 || !E->grid[N] || std::find(kSplits, kSplits + 5, P) == kSplits + 5 || !ens_split_supported(N, P))
+        return c->fail(DGH_ERR_ARG, "dgh_ensemble_set_split: order %d, shape %d", N, P), DGH_ERR_ARG;
+    (void)hipSetDevice(c->device);
+    E->split[N] = P;
+    return ens_finalize_items(c, *E) ? DGH_OK : c->last;
+}
+
 extern "C" int dgh_ensemble_info(dgh_ctx c, int h, int* split, double* tune_us, long long* dofs, int* nitems) {
     if (!c) return DGH_ERR_ARG;
     EnsDev* E = ens_get(c, h);

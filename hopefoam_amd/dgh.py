@@ -153,6 +153,7 @@ def lib():
         "dgh_ensemble_get": [vp, C.c_int, C.c_int, C.c_int, _dp],
         "dgh_ensemble_rhs": [vp, C.c_int],
         "dgh_ensemble_run": [vp, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_float)],
+        "dgh_ensemble_set_split": [vp, C.c_int, C.c_int, C.c_int],
         "dgh_ensemble_info": [vp, C.c_int, vp, vp, vp, vp],
         "dgh_selftest_field_raw": [vp, C.c_int, _dp],
         "dgh_selftest_ensemble_raw": [vp, C.c_int, C.c_int, _dp],
@@ -625,6 +626,10 @@ class Ensemble:
         self.ctx._ck(self.ctx.L.dgh_ensemble_run(self.ctx.h, self.h, nsteps, int(graph), C.byref(ms)),
                      "dgh_ensemble_run")
         return ms.value
+
+    def set_split(self, N, P):
+        """tile shape P (1, 2, 4, 8; 16: MFMA tiles) for the cases of order N"""
+        self.ctx._ck(self.ctx.L.dgh_ensemble_set_split(self.ctx.h, self.h, N, P), "dgh_ensemble_set_split")
 
     def info(self):
         split = np.zeros(9, np.int32)

@@ -374,6 +374,9 @@ int dgh_ensemble_run(dgh_ctx ctx, int ens, int nsteps, int use_graph, float* ms)
  * absent); tune_us[9 x 5]: autotuner time per stage of each order's cases for 1, 2, 4, 8 waves and MFMA tiles
  * (0: not measured or not available); dofs: sum of K Np; nitems: work items.  Any pointer may be NULL. */
 int dgh_ensemble_info(dgh_ctx ctx, int ens, int* split, double* tune_us, long long* dofs, int* nitems);
+/* takes tile shape P (as in split above) for the cases of order N, whatever the autotuner found; DGH_ERR_ARG for a shape
+ * that the order does not have */
+int dgh_ensemble_set_split(dgh_ctx ctx, int ens, int N, int P);
 
 /* ---- diagnostics ---------------------------------------------------------------------- */
 /* caps the persistent grid of the stage kernel at blocks (rounded down to a multiple of 8, at least 8; 0: as many
