@@ -45,22 +45,11 @@ template <typename T>
 constexpr int mfma_row(int rg, int r) {
     return sizeof(T) == 8 ? rg + 4 * r : 4 * rg + r;
 }
-// Node supplied by row group k' at K step s of the interpolation GEMM.  With the f64 row map this is also
-// the output row 16 m + mfma_row(k', r) for s = 4 m + r, so the FP64 stage update reuses the B fragments
-// as q_in.
-template <typename T>
-constexpr int gemm1_node(int s, int kq) {
-    return 4 * s + kq;
-}
-// inverse: the (row group, register) holding accumulator row i
-template <typename T>
-constexpr int mfma_rg(int i) {
-    return sizeof(T) == 8 ? i % 4 : i / 4;
-}
-template <typename T>
-constexpr int mfma_reg(int i) {
-    return sizeof(T) == 8 ? i / 4 : i % 4;
-}
+// Node supplied by row group k' at K step s of the interpolation GEMM of the FP32 and bf16x3 stage kernels.
+constexpr int gemm1_node(int s, int kq) { return 4 * s + kq; }
+// inverse of mfma_row<float>: the (row group, register) holding accumulator row i
+constexpr int mfma_rg32(int i) { return i / 4; }
+constexpr int mfma_reg32(int i) { return i % 4; }
 
 // Node k of face f of the reference triangle of order N, in the order of RefElem::fmask (face 0 along s = -1,
 // face 1 the hypotenuse, face 2 along r = -1), as a compile-time function so that the stage kernels look nothing

@@ -29,9 +29,8 @@ std::vector<T> cast_vec(const std::vector<double>& v) {
     return std::vector<T>(v.begin(), v.end());
 }
 
-// Operator fragments in the per-lane order of the 16x16x4 MFMA operands (see stage_kernels.hip);
-// PF depends on the accumulator row map of the precision it is built for.
-template <typename T>
+// Operator fragments of the FP32 stage kernel in the per-lane order of the 16x16x4 MFMA operands (see
+// stage_kernels.hip); PF follows the accumulator's row map.
 void build_fragments(const RefElem& re, std::vector<double>& VqF, std::vector<double>& PF, std::vector<double>& LF) {
     const int Np = re.Np, Nq = re.Nq, Nfq = re.Nfq;
     const int MT = round_up(Np, 16) / 16, QT = round_up(Nq, 16) / 16;
@@ -41,7 +40,7 @@ void build_fragments(const RefElem& re, std::vector<double>& VqF, std::vector<do
     for (int t = 0; t < QT; ++t)
         for (int s = 0; s < KS1; ++s)
             for (int l = 0; l < 64; ++l) {
-                const int i = 16 * t + (l & 15), k = gemm1_node<T>(s, l >> 4);
+                const int i = 16 * t + (l & 15), k = gemm1_node(s, l >> 4);
                 if (i < Nq && k < Np) VqF[(size_t(t) * KS1 + s) * 64 + l] = re.Vq[size_t(i) * Np + k];
             }
     // face-trace tiles: accumulator row i of tile tf is held by (row group rg, register r); it is the own
@@ -49,8 +48,8 @@ void build_fragments(const RefElem& re, std::vector<double>& VqF, std::vector<do
     for (int tf = 0; tf < FT; ++tf)
         for (int s1 = 0; s1 < KS1; ++s1)
             for (int l = 0; l < 64; ++l) {
-                const int i = l & 15, node = gemm1_node<T>(s1, l >> 4);
-                const int rg = mfma_rg<T>(i), r = mfma_reg<T>(i);
+                const int i = l & 15, node = gemm1_node(s1, l >> 4);
+                const int rg = mfma_rg32(i), r = mfma_reg32(i);
                 const int st = 4 * tf + r, g = 4 * (st % SF) + rg, f = st / SF;
                 if (st >= KSF || g >= Nfq || node >= Np) continue;
                 double w = 0.0;
@@ -64,7 +63,7 @@ void build_fragments(const RefElem& re, std::vector<double>& VqF, std::vector<do
             for (int m = 0; m < MT; ++m)
                 for (int w = 0; w < 2; ++w)
                     for (int l = 0; l < 64; ++l) {
-                        const int j = 16 * m + (l & 15), p = 16 * t + mfma_row<T>(l >> 4, r);
+                        const int j = 16 * m + (l & 15), p = 16 * t + mfma_row<float>(l >> 4, r);
                         const std::vector<double>& P = w == 0 ? re.Pr : re.Ps;
                         if (j < Np && p < Nq)
                             PF[((((size_t(t) * 4 + r) * MT + m) * 2 + w) * 64) + l] = P[size_t(j) * Nq + p];
@@ -198,12 +197,11 @@ void put_split(std::vector<uint32_t>& v, size_t slot, const double (&x)[4]) {
     v[slot * 4 + 3] = l[2] | uint32_t(l[3]) << 16;
 }
 
-// The operators of build_fragments<float> as bf16x3 fragments of v_mfma_f32_16x16x16_bf16: element e of K16
+// The operators of build_fragments as bf16x3 fragments of v_mfma_f32_16x16x16_bf16: element e of K16
 // step S is the FP32 kernel's K4 step 4 S + e (interpolation, lift) or register e of cubature tile t
 // (projection), so the kernels feed the B operands from the same registers as the FP32 kernel.
 void build_split_fragments(const RefElem& re, std::vector<uint32_t>& VqS, std::vector<uint32_t>& PS,
                            std::vector<uint32_t>& LS) {
-    using T = float;
     const int Np = re.Np, Nq = re.Nq, Nfq = re.Nfq;
     const int MT = round_up(Np, 16) / 16, QT = round_up(Nq, 16) / 16;
     const int KS1 = round_up(Np, 4) / 4, SF = round_up(Nfq, 4) / 4, KSF = 3 * SF;
@@ -215,7 +213,7 @@ void build_split_fragments(const RefElem& re, std::vector<uint32_t>& VqS, std::v
             for (int l = 0; l < 64; ++l) {
                 const int i = 16 * t + (l & 15);
                 for (int e = 0; e < 4; ++e) {
-                    const int s = 4 * S + e, k = gemm1_node<T>(s, l >> 4);
+                    const int s = 4 * S + e, k = gemm1_node(s, l >> 4);
                     x[e] = (s < KS1 && i < Nq && k < Np) ? re.Vq[size_t(i) * Np + k] : 0.0;
                 }
                 put_split(VqS, (size_t(t) * KS16 + S) * 64 + l, x);
@@ -224,10 +222,10 @@ void build_split_fragments(const RefElem& re, std::vector<uint32_t>& VqS, std::v
         for (int S = 0; S < KS16; ++S)
             for (int l = 0; l < 64; ++l) {
                 const int i = l & 15;
-                const int rg = mfma_rg<T>(i), r = mfma_reg<T>(i);
+                const int rg = mfma_rg32(i), r = mfma_reg32(i);
                 const int st = 4 * tf + r, g = 4 * (st % SF) + rg, f = st / SF;
                 for (int e = 0; e < 4; ++e) {
-                    const int s1 = 4 * S + e, node = gemm1_node<T>(s1, l >> 4);
+                    const int s1 = 4 * S + e, node = gemm1_node(s1, l >> 4);
                     x[e] = 0.0;
                     if (s1 >= KS1 || st >= KSF || g >= Nfq || node >= Np) continue;
                     for (int k = 0; k < re.Nfp; ++k)
@@ -243,7 +241,7 @@ void build_split_fragments(const RefElem& re, std::vector<uint32_t>& VqS, std::v
                     const std::vector<double>& P = w == 0 ? re.Pr : re.Ps;
                     const int j = 16 * m + (l & 15);
                     for (int e = 0; e < 4; ++e) {
-                        const int p = 16 * t + mfma_row<T>(l >> 4, e);
+                        const int p = 16 * t + mfma_row<float>(l >> 4, e);
                         x[e] = (j < Np && p < Nq) ? P[size_t(j) * Nq + p] : 0.0;
                     }
                     put_split(PS, ((size_t(t) * MT + m) * 2 + w) * 64 + l, x);
@@ -310,7 +308,7 @@ RefDev* dgh_ctx_s::refdev(int N) {
         fail(DGH_ERR_UNSUPPORTED, "order N=%d: the reference element is not mirror symmetric", N);
         return nullptr;
     }
-    build_fragments<float>(rd->re, VqF32, PF32, LF32);
+    build_fragments(rd->re, VqF32, PF32, LF32);
     build_split_fragments(rd->re, VqS, PS, LS);
     bool ok = upload(&rd->Vf64, rd->re.Vf) && upload(&rd->VqF32, cast_vec<float>(VqF32)) &&
               upload(&rd->PF32, cast_vec<float>(PF32)) && upload(&rd->LF32, cast_vec<float>(LF32)) &&
@@ -748,12 +746,12 @@ static int stage_launch(dgh_ctx c, MeshDev* m, const dgh_rhs_desc* d, const doub
     a.geo = f64 ? static_cast<const void*>(m->geo64) : static_cast<const void*>(m->geo32);
     a.conn = m->conn;
     const bool split = d->prec == DGH_PREC_BF16X3;
-    // FP64: the mirror-half fragments and node rows of stage_sym.hip
+    // FP64: the fragments and node rows of stage_sym.hip
     a.VqF = f64 ? static_cast<const void*>(rd->symF) : split ? static_cast<const void*>(rd->VqS) : rd->VqF32;
     a.PF = f64 ? nullptr : split ? static_cast<const void*>(rd->PS) : rd->PF32;
     a.LF = f64 ? nullptr : split ? static_cast<const void*>(rd->LS) : rd->LF32;
     a.Vf = f64 ? static_cast<const void*>(rd->Vf64) : static_cast<const void*>(rd->Vf32);
-    a.fmask = f64 ? rd->symRows : rd->fmask;
+    a.rows = f64 ? rd->symRows : nullptr;
     a.bcq = (m->bcq && m->bc_nvar == nvar) ? m->bcq : nullptr;
     a.ax = d->ax;
     a.ay = d->ay;

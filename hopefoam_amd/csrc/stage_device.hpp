@@ -14,8 +14,6 @@ typedef float f4_t __attribute__((ext_vector_type(4)));
 template <typename T>
 struct Vec4;
 template <>
-struct Vec4<double> { typedef d4_t type; };
-template <>
 struct Vec4<float> { typedef f4_t type; };
 
 // Row of the 16x16 accumulator held in register r of a lane of row group rg (= lane / 16).

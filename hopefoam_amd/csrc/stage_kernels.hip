@@ -1,4 +1,5 @@
 // DG right-hand side + fused LSERK4 stage kernels for gfx950 (CDNA4), FP32 and bf16x3 (FP64: stage_sym.hip).
+// T, the type of the contractions and fluxes, is float throughout.
 //
 // One wavefront owns 16 elements (one per MFMA column).  Per element e the kernel evaluates
 // the reference's over-integrated weak form
@@ -17,7 +18,7 @@
 // low-storage RK update  res = a res + dt rhs;  q_out = q_in + b res  in FP64.
 //
 // MFMA 16x16x4 operand layout: A[i][k] in lane i + 16k, B[k][j] in lane j + 16k, D[i][j] in lane
-// j + 16 rg, register r with i = mfma_row<T>(rg, r) (dg_common.hpp; f32 and f64 differ).  Operator
+// j + 16 rg, register r with i = mfma_row<T>(rg, r) (dg_common.hpp).  Operator
 // fragments are pre-arranged on the host in exactly the per-lane order, so every A load is a
 // contiguous 64-lane vector load.
 #include <hip/hip_runtime.h>
@@ -258,7 +259,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, VolumeFlux<PHYS, T>::NV, T
             for (int v = 0; v < NV; ++v)
 #pragma unroll
                 for (int s = 0; s < D::KS1; ++s)
-                    qd[v][s] = gemm1_node<T>(s, rg) < Np ? at_lane(qg + (v * Np + 4 * s) * 16, lane8) : 0.0;
+                    qd[v][s] = gemm1_node(s, rg) < Np ? at_lane(qg + (v * Np + 4 * s) * 16, lane8) : 0.0;
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int v = 0; v < NV; ++v)
@@ -319,7 +320,7 @@ __global__ __launch_bounds__((64 * waves_per_block<N, VolumeFlux<PHYS, T>::NV, T
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int s1 = 4 * S + e < D::KS1 ? 4 * S + e : 0;
-                        x[e] = (4 * S + e < D::KS1 && gemm1_node<T>(s1, rg) < Np) ? qb[v][s1] - q0[v] : T(0);
+                        x[e] = (4 * S + e < D::KS1 && gemm1_node(s1, rg) < Np) ? qb[v][s1] - q0[v] : T(0);
                     }
                     qs[v][S] = split4(x[0], x[1], x[2], x[3]);
                 }

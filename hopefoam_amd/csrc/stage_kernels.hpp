@@ -22,7 +22,7 @@ struct StageArgs {
     const void* PF;
     const void* LF;
     const void* Vf;      // [Nfq][Nfp]
-    const int* fmask;    // [3][Nfp]
+    const int* rows;     // FP64: node rows a | b << 8 in stage_sym.hpp's order, padded to whole K steps
     const double* bcq;   // fixedValue nodal ghost values [nvar][K][3][Nfp] or null
     double ax, ay, gamma;
     double rk_a, rk_b, dt;
@@ -34,8 +34,7 @@ struct StageArgs {
 };
 
 hipError_t launch_stage(int N, int phys, int prec, const StageArgs& a, int ncu, hipStream_t st);
-// the FP64 stage on the mirror halves of the operators (stage_sym.hip): VqF the fragments in stage_sym.hpp's order,
-// fmask the node rows (a | b << 8, padded to whole K steps)
+// the FP64 stage on the mirror halves of the operators (stage_sym.hip): VqF the fragments in stage_sym.hpp's order
 hipError_t launch_stage_sym(int N, int phys, const StageArgs& a, int ncu, hipStream_t st);
 hipError_t launch_mfma_layout_probe(double* out, hipStream_t st);
 hipError_t launch_mfma_probe(const double* A, const double* B, double* D64, const float* Af, const float* Bf,

@@ -131,7 +131,7 @@ __global__ __launch_bounds__(64 * sym_waves<N>(), sym_per_simd<N>()) void stage_
     unsigned na[KE], nb[KOA];
 #pragma unroll
     for (int s = 0; s < KE; ++s) {
-        const unsigned ab = unsigned(a.fmask[4 * s + rg]);
+        const unsigned ab = unsigned(a.rows[4 * s + rg]);
         na[s] = ((ab & 255u) * 16 + col) * 8;
         if (s < KO) nb[s < KO ? s : 0] = ((ab >> 8) * 16 + col) * 8;
     }
