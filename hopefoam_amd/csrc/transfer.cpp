@@ -4,8 +4,9 @@
 // its two slots: while the device packs (or unpacks) one, the worker copies the other from (or to) the caller's memory.
 // One worker copies about 30 GB/s; the first touch of a fresh result array costs as much again; the workers share both.
 // Small transfers stay on the calling thread.  Measured, up / down: 117 MB 38.8 / 45.7 ms -> 2.9 / 3.3 ms, 42 MB 15.5 /
-// 19.8 -> 1.1 / 1.5 ms, 4.2 MB 306 / 825 -> 145 / 159 us, 0.7 MB 55 / 61 -> 36 / 38 us, 0.24 MB 25 / 27 -> 21 / 22 us;
-// pageable copies of 1 to 80 KB took 12 to 30 us (by where the caller's memory lies), these take 13 to 16.
+// 19.8 -> 1.1 / 1.5 ms, 4.2 MB 306 / 825 -> 145 / 155 us, 0.8 MB 62 / 69 -> 42 / 50 us, 0.3 MB 30 / 32 -> 24 / 27 us.
+// Pageable copies of 1 to 80 KB took 12 to 30 us, by where the caller's memory lies, these take 15 to 17; upload, right-hand
+// side and download in a row 47 -> 38 us at 40 KB, 61 -> 47 at 16 KB.
 #include "transfer.hpp"
 
 #include <algorithm>
@@ -19,10 +20,10 @@
 namespace dg {
 
 // Data that pays for one more worker (a thread costs some tens of microseconds to start: with a worker per 2 MiB a field
-// of 4 MB took 210 us up, with one 146), and the smallest chunk worth a launch of its own (0.3 MB in two chunks 30 / 28 us,
-// in one 24 / 26).
+// of 4 MB took 210 us up, with one 146), and the smallest chunks worth a launch of their own (0.3 MB in two chunks 30 / 28 us,
+// in one 24 / 26; smaller down, where the first touch of the caller's memory may overlap with the next chunk's copy).
 static constexpr size_t kWorkerBytes = size_t(8) << 20;
-static constexpr size_t kChunkLeast = size_t(512) << 10;
+static constexpr size_t kChunkUp = size_t(512) << 10, kChunkDown = size_t(384) << 10;
 
 bool Staging::ready(int n) {
     if (slots >= n) return true;
@@ -86,15 +87,20 @@ hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArr
     const int most = int(Staging::kSlotBytes / (size_t(16) * a.Np * sizeof(double)));
     // (a transfer of a few slots is cut finer, so that the copies and the device's work overlap)
     const int per = std::max(1, std::min(most, (tiles + 4 * workers - 1) / (4 * workers)));
-    const int step = std::max(per, std::min(most, int(kChunkLeast / (size_t(16) * a.Np * sizeof(double)))));
-    const int chunks = (tiles + step - 1) / step;
+    const int least = std::max(per, std::min(most, int((to_device ? kChunkUp : kChunkDown) / (size_t(16) * a.Np * sizeof(double)))));
+    int chunks = (tiles + least - 1) / least;
+    const int step = (tiles + chunks - 1) / chunks;   // equal chunks
+    chunks = (tiles + step - 1) / step;
     workers = std::min(workers, chunks);
-    if (!st.ready(chunks == 1 ? 1 : Staging::kSlots)) return transfer_pageable(s, a, host, to_device);
-    if (chunks == 1) {   // nothing to overlap
+    if (!st.ready(2 * workers)) return transfer_pageable(s, a, host, to_device);
+    // One chunk: nothing to overlap.  (Waiting for the kernel's own completion signal, an event handed to its launch, is 2.5 us
+    // shorter, but the next synchronisation of the stream then takes 8: upload, right-hand side, download of 16 KB 47 -> 44
+    // us, time loop and download 120 -> 122, upload and synchronise 16.6 -> 22.6.)
+    if (chunks == 1) {
         if (to_device) std::memcpy(st.slot(0), host, bytes);
-        const hipError_t err = to_device ? launch_unpack_tiles(a, 0, tiles, st.slot(0), s, st.ev[0])
-                                         : launch_pack_tiles(a, 0, tiles, st.slot(0), s, st.ev[0]);
-        const hipError_t done = err == hipSuccess ? hipEventSynchronize(st.ev[0]) : hipStreamSynchronize(s);
+        const hipError_t err = to_device ? launch_unpack_tiles(a, 0, tiles, st.slot(0), s)
+                                         : launch_pack_tiles(a, 0, tiles, st.slot(0), s);
+        const hipError_t done = hipStreamSynchronize(s);
         if (err != hipSuccess || done != hipSuccess) return err != hipSuccess ? err : done;
         if (!to_device) std::memcpy(host, st.slot(0), bytes);
         return hipSuccess;
@@ -135,8 +141,8 @@ hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArr
             range(c, t0, t1, h, nb);
             double* slot = st.slot(2 * w + k);
             if (to_device) std::memcpy(slot, h, nb);
-            const hipEvent_t ev = st.ev[2 * w + k];
-            if (!check(to_device ? launch_unpack_tiles(a, t0, t1, slot, s, ev) : launch_pack_tiles(a, t0, t1, slot, s, ev)))
+            if (!check(to_device ? launch_unpack_tiles(a, t0, t1, slot, s) : launch_pack_tiles(a, t0, t1, slot, s)) ||
+                !check(hipEventRecord(st.ev[2 * w + k], s)))
                 break;
             pending[k] = c;
         }

@@ -5,7 +5,6 @@
 // across PCIe itself (512 contiguous bytes per instruction), so that the reordering, the padding and the copy are one
 // pass; PCIe bounds it (57 GB/s each way).  Before, the host reordered element by element in one thread: a field of
 // 117 MB took 46 ms to download.
-#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include "dg_common.hpp"
@@ -64,22 +63,19 @@ __global__ __launch_bounds__(256) void tiles_kernel(NodalArray a, int t0, int t1
     }
 }
 
-// The event takes the dispatch's own completion signal: a synchronisation behind it (of the stream, or of an event recorded
-// after it) is a packet more to wait for, 16 against 13.5 us for a field of a few KB.
 template <bool UNPACK>
-static hipError_t launch_tiles(const NodalArray& a, int t0, int t1, double* host, hipStream_t s, hipEvent_t done) {
+static hipError_t launch_tiles(const NodalArray& a, int t0, int t1, double* host, hipStream_t s) {
     if (16 * a.Np > kTileMax || t1 <= t0) return hipErrorInvalidValue;
     const int blocks = (t1 - t0 + 3) / 4;
-    hipExtLaunchKernelGGL((tiles_kernel<UNPACK>), dim3(blocks < 1024 ? blocks : 1024), dim3(256), 0, s, nullptr, done, 0, a,
-                          t0, t1, host);
+    hipLaunchKernelGGL((tiles_kernel<UNPACK>), dim3(blocks < 1024 ? blocks : 1024), dim3(256), 0, s, a, t0, t1, host);
     return hipGetLastError();
 }
 
-hipError_t launch_unpack_tiles(const NodalArray& a, int t0, int t1, const double* host, hipStream_t s, hipEvent_t done) {
-    return launch_tiles<true>(a, t0, t1, const_cast<double*>(host), s, done);
+hipError_t launch_unpack_tiles(const NodalArray& a, int t0, int t1, const double* host, hipStream_t s) {
+    return launch_tiles<true>(a, t0, t1, const_cast<double*>(host), s);
 }
-hipError_t launch_pack_tiles(const NodalArray& a, int t0, int t1, double* host, hipStream_t s, hipEvent_t done) {
-    return launch_tiles<false>(a, t0, t1, host, s, done);
+hipError_t launch_pack_tiles(const NodalArray& a, int t0, int t1, double* host, hipStream_t s) {
+    return launch_tiles<false>(a, t0, t1, host, s);
 }
 
 }  // namespace dg

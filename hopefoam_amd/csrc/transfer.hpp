@@ -20,9 +20,8 @@ struct NodalArray {
     }
 };
 
-// Pinned staging memory of a context, allocated with the first transfer that needs it and freed with the context: one slot
-// for transfers of one chunk, else kSlots, two per worker, so that the copy of one slot overlaps the device's work on the
-// other.
+// Pinned staging memory of a context, allocated with the first transfer that needs it and freed with the context: two slots
+// per worker, so that the copy of one overlaps the device's work on the other, at most kSlots.
 struct Staging {
     static constexpr int kSlots = 16;
     static constexpr size_t kSlotBytes = size_t(1) << 20;   // 16 MiB in all
@@ -36,9 +35,9 @@ struct Staging {
     double* slot(int i) const { return mem + size_t(i) * (kSlotBytes / sizeof(double)); }
 };
 
-// tiles [t0, t1) of a from / to the packed host order at host (device-accessible memory); done is recorded with the kernel
-hipError_t launch_unpack_tiles(const NodalArray& a, int t0, int t1, const double* host, hipStream_t s, hipEvent_t done);
-hipError_t launch_pack_tiles(const NodalArray& a, int t0, int t1, double* host, hipStream_t s, hipEvent_t done);
+// tiles [t0, t1) of a from / to the packed host order at host (device-accessible memory)
+hipError_t launch_unpack_tiles(const NodalArray& a, int t0, int t1, const double* host, hipStream_t s);
+hipError_t launch_pack_tiles(const NodalArray& a, int t0, int t1, double* host, hipStream_t s);
 
 // the whole array from / to host memory, ordered behind the work on stream s and complete on return
 hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArray& a, double* host, bool to_device);

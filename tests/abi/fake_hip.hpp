@@ -91,13 +91,6 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipSt
     if (st.on_launch) st.on_launch(st.kernels[f], args);
     return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t e, hipStream_t s);
-hipError_t hipExtLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t m, hipStream_t s, hipEvent_t, hipEvent_t stop,
-                              int) {
-    const hipError_t e = hipLaunchKernel(f, g, b, args, m, s);
-    if (e == hipSuccess && stop) return hipEventRecord(stop, s);
-    return e;
-}
 hipError_t hipGetLastError() {
     FAKE_LOCK;
     const hipError_t e = fake::state().last;

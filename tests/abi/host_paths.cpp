@@ -148,8 +148,8 @@ static void ensemble_failing_launch() {
     CHECK(dgh_destroy(c) == DGH_OK);
 }
 
-// pinned staging memory: one slot of 1 MiB for transfers of one chunk, all sixteen once a transfer has several, given
-// back with the context
+// pinned staging memory: two slots of 1 MiB, two more for every further worker of a larger transfer, given back with the
+// context
 static void staging_as_needed() {
     dgh_ctx c = context();
     int m = -1, f = -1, big = -1, g = -1;
@@ -158,14 +158,23 @@ static void staging_as_needed() {
     CHECK(fake::state().pinned_bytes == 0);
     std::vector<double> a(size_t(18) * 6 * 4, 1.0);
     CHECK(dgh_field_upload(c, f, a.data()) == DGH_OK && dgh_field_download(c, f, a.data()) == DGH_OK);
-    CHECK(fake::state().pinned_bytes == size_t(1) << 20);
+    CHECK(fake::state().pinned_bytes == size_t(2) << 20);
     CHECK(dgh_mesh_structured(c, 8, 64, 32, 0, 1, 0, 1, 1, 1, 0, &big) == DGH_OK);
     CHECK(dgh_field_create(c, big, 4, &g) == DGH_OK);
     std::vector<double> b(size_t(4096) * 45 * 4, 1.0);
     CHECK(dgh_field_upload(c, g, b.data()) == DGH_OK);
-    CHECK(fake::state().pinned_bytes == size_t(16) << 20);
+    CHECK(fake::state().pinned_bytes == size_t(2) << 20);
+    for (int n : {2, 16}) {   // workers: one for every 8 MiB, at most eight
+        const int K = 2 * 64 * 16 * n;
+        CHECK(dgh_mesh_structured(c, 8, 64, 16 * n, 0, 1, 0, 1, 1, 1, 0, &big) == DGH_OK);
+        CHECK(dgh_field_create(c, big, 4, &g) == DGH_OK);
+        b.assign(size_t(K) * 45 * 4, 1.0);
+        CHECK(dgh_field_upload(c, g, b.data()) == DGH_OK);
+        const size_t workers = std::max<size_t>(1, std::min<size_t>(8, b.size() * sizeof(double) >> 23));
+        CHECK(fake::state().pinned_bytes == 2 * workers << 20);
+    }
     CHECK(dgh_field_download(c, f, a.data()) == DGH_OK);
-    CHECK(fake::state().pinned_bytes == size_t(16) << 20 && fake::state().pinned.size() == 1);
+    CHECK(fake::state().pinned.size() == 1);
     CHECK(dgh_destroy(c) == DGH_OK);
     CHECK(fake::state().pinned.empty());
 }

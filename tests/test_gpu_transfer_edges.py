@@ -1,5 +1,5 @@
-"""Field transfers around the sizes at which they are cut differently: one chunk up to 512 KiB, several beyond, the last one
-short; upload, download and a kernel that reads the field come one after the other without a wait in between."""
+"""Field transfers around the sizes at which they are cut differently: one chunk up to 512 KiB (down 384), several equal ones
+beyond; upload, download and a kernel that reads the field come one after the other without a wait in between."""
 import numpy as np
 import pytest
 
@@ -8,11 +8,14 @@ from hopefoam_amd import Context
 pytestmark = pytest.mark.gpu
 
 
-# tiles of 16 elements: 3584 bytes at order 6, 5760 at order 8; 146 and 91 of them make a chunk
-@pytest.mark.parametrize("N,nx,ny,nvar", [(6, 18, 16, 4),    # 144 tiles: one chunk
+# tiles of 16 elements: 3584 bytes at order 6, 5760 at order 8; 146 and 91 of them make a chunk up, 109 and 68 one down
+@pytest.mark.parametrize("N,nx,ny,nvar", [(6, 18, 16, 4),    # 144 tiles: one chunk up, two down
                                           (6, 73, 4, 4),     # 148 tiles of which one in 37 is ragged: two chunks
-                                          (8, 182, 4, 1),    # 91 tiles: exactly one chunk
-                                          (8, 184, 4, 1),    # 92 tiles: the second chunk is one tile
+                                          (6, 18, 12, 4),    # 108 tiles: one chunk
+                                          (8, 182, 4, 1),    # 91 tiles: exactly one chunk up
+                                          (8, 184, 4, 1),    # 92 tiles: two chunks
+                                          (8, 137, 4, 1),    # 69 tiles: one up, two down, 35 and 34
+                                          (8, 365, 4, 1),    # 183 tiles: three of 61
                                           (8, 16, 15, 3)])   # 90 tiles of three variables
 def test_chunk_edges(N, nx, ny, nvar):
     with Context(0) as ctx:
