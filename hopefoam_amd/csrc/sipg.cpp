@@ -218,12 +218,15 @@ static void element_block(const RefElem& re, const std::vector<double>& Srr, con
                     Dn[size_t(q) * Np + j] += w * (ar * re.Dr[size_t(node) * Np + j] + as * re.Ds[size_t(node) * Np + j]);
             }
         for (int q = 0; q < Nfq; ++q) {
-            const double w = js * re.gw[q];
-            const double* v = &V1[size_t(q) * Np];
-            const double* d = &Dn[size_t(q) * Np];
-            for (int i = 0; i < Np; ++i)
-                for (int j = 0; j < Np; ++j)
-                    blk[size_t(i) * Np + j] += w * fac * (-tau * v[i] * v[j] + v[i] * d[j] + d[i] * v[j]);
+            const double w = js * re.gw[q] * fac;
+            const double* __restrict v = &V1[size_t(q) * Np];
+            const double* __restrict d = &Dn[size_t(q) * Np];
+            // (unaliased rows: with overlap checks around each row the loop took a third longer in some layouts of the code)
+            for (int i = 0; i < Np; ++i) {
+                double* __restrict row = &blk[size_t(i) * Np];
+                const double tv = -tau * v[i], vi = v[i], di = d[i];
+                for (int j = 0; j < Np; ++j) row[j] += w * (tv * v[j] + vi * d[j] + di * v[j]);
+            }
         }
     }
 }
