@@ -67,7 +67,7 @@ __device__ __forceinline__ d4_t mfma64(double a, double b, d4_t c) {
 // one for the neighbours'.  Microseconds per stage (both passes) of 7 to 13 cases of one order, elements in all, with a
 // face's points running over the K steps, face geometry per point and the loads left where the products need them -> now:
 //   order 8, 50048: 82 -> 60    6, 36136: 41.6 -> 35.5    5, 30076: 30.4 -> 28.9    4, 16404: 15.2 -> 12.7
-//   order 7, 20780: 42 -> 43 (nine matrix steps of the lift in place of six)         3, 20918: 12.2 -> 11.1
+//   order 7, 20634: 32.4 -> 27.5 (the lift takes eight matrix steps in place of six)   3, 20918: 12.2 -> 11.1
 template <int N>
 struct EnsLane {
     const double *up;       // u of the neighbour's node 0

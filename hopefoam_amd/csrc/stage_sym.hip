@@ -12,12 +12,16 @@
 // the value, with half the operator entry), so no lane branches.
 //
 // Why: on gfx950 f64 MFMA (64 clk each) and f64 VALU instructions do not overlap, neither in one wavefront nor
-// between the wavefronts of a SIMD, so their sum bounds the kernel.  At N = 6 the halves take 324 MFMA per group of
-// 16 elements instead of 600 for about 200 more additions.  Two wavefronts per SIMD (256 registers, N <= 6) hide the
-// gathers and the dependent chains; an f64 FMA then issues every 4.3 clk instead of 5.6.
+// between the wavefronts of a SIMD, so their times add.  At N = 6 the halves take 324 MFMA per group of 16 elements
+// instead of 600 for about 200 more additions.  Two wavefronts per SIMD (256 registers, N <= 6) hide most of the gathers
+// and the dependent chains; an f64 FMA then issues every 4.3 clk instead of 5.6.
+// Account of the some 44,000 clk that a SIMD has per group at N = 6, K = 131072 (163 to 169 us at 2.1 GHz): 20,700 of
+// matrix products, 8,600 of 2,000 f64 VALU instructions, about 5,000 of 1,200 other VALU instructions.  The other 10,000
+// are waits that the second wavefront does not cover (the counters name memory: 17 % of the wavefronts' time) and LDS,
+// scalar and branch issue, which they do not tell apart.
 // Measured (us per stage; before: whole operators, one wavefront per SIMD, own traces by lane shuffles):
 //   LF, K = 131072:  N = 2  49.4 -> 40.4   3  87.0 -> 71.0   4  119 -> 92.5   5  200 -> 127   6  237 -> 163
-//   LF, K = 32768:   N = 7  185 -> 73      8  228 -> 112
+//   LF, K = 32768:   N = 7  185 -> 73      8  228 -> 110 (112 since its first stage reads, its last writes no residual)
 //   Roe, K = 131072: N = 2  58.5 -> 44.3   3  103.8 -> 78.4  4  137 -> 98.5
 //   small meshes:    N = 4 Roe, K = 1024  20.7 -> 14.2;  N = 4 advection, K = 2048  8.9 -> 6.2
 // Order 1 takes the whole operators in this kernel's layout (SymDims::whole): its 3 nodes fill one tile either way, and

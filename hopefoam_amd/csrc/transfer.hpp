@@ -24,7 +24,7 @@ struct NodalArray {
 // per worker, so that the copy of one overlaps the device's work on the other, at most kSlots.
 struct Staging {
     static constexpr int kSlots = 16;
-    static constexpr size_t kSlotBytes = size_t(1) << 20;   // 16 MiB in all
+    static constexpr size_t kSlotBytes = size_t(1) << 20;   // 16 MiB with every slot
     std::mutex mu;                 // one transfer at a time
     double* mem = nullptr;
     int slots = 0;                 // of mem
