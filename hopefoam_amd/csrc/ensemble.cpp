@@ -161,11 +161,16 @@ static void build_items(const EnsDev& E, const std::vector<int>& use, const int*
 }
 
 static bool upload_items(dgh_ctx c, EnsDev& E, const std::vector<EnsItem>& items) {
-    if (!c->hip(hipStreamSynchronize(c->stream), "sync")) return false;   // no launch may still read the old list
+    EnsItem* list = nullptr;
+    if (!c->hip(hipStreamSynchronize(c->stream), "sync") ||   // no launch may still read the old list
+        !upload_table(c, &list, items)) {
+        if (list) (void)hipFree(list);
+        return false;
+    }
     if (E.items) (void)hipFree(E.items);
-    E.items = nullptr;
+    E.items = list;
     E.nitems = int(items.size());
-    return upload_table(c, &E.items, items);
+    return true;
 }
 
 static EnsArgs ens_args(const EnsDev& E) {
@@ -568,8 +573,15 @@ extern "C" int dgh_ensemble_set_split(dgh_ctx c, int h, int N, int P) {
     if (N < 1 || N > 8 || !E->grid[N] || std::find(kSplits, kSplits + 5, P) == kSplits + 5 || !ens_split_supported(N, P))
         return c->fail(DGH_ERR_ARG, "dgh_ensemble_set_split: order %d, shape %d", N, P), DGH_ERR_ARG;
     (void)hipSetDevice(c->device);
+    const int split = E->split[N];
+    int chunk[9][9];
+    std::memcpy(chunk, E->chunk, sizeof chunk);
     E->split[N] = P;
-    return ens_finalize_items(c, *E) ? DGH_OK : c->last;
+    if (ens_finalize_items(c, *E)) return DGH_OK;
+    // the list and the graphs are still those of the old shape
+    E->split[N] = split;
+    std::memcpy(E->chunk, chunk, sizeof chunk);
+    return c->last;
 }
 
 extern "C" int dgh_ensemble_info(dgh_ctx c, int h, int* split, double* tune_us, long long* dofs, int* nitems) {

@@ -7,6 +7,7 @@
 #include <thread>
 
 #include "dgh.h"
+#include "ensemble.hpp"
 #include "stage_kernels.hpp"
 
 #define CHECK(x)                                                                    \
@@ -148,6 +149,38 @@ static void ensemble_failing_launch() {
     CHECK(dgh_destroy(c) == DGH_OK);
 }
 
+// a shape that cannot be taken for want of memory leaves the ensemble as it was
+static void ensemble_failing_shape() {
+    dgh_ctx c = context();
+    const dgh_ens_desc d = {1.0, 1.0, 0.3, 0, 0};
+    std::vector<dgh_ens_case> cases;
+    for (int N : {3, 5}) cases.push_back({N, 4, 4, 0, 0, 1, 1, 1.0, 0.5, 1e-3, 1e-4});
+    int e = -1;
+    CHECK(dgh_ensemble_create(c, &d, int(cases.size()), cases.data(), &e) == DGH_OK);
+    std::vector<std::string> seen;
+    bool listed = true;
+    fake::state().on_launch = [&](const std::string& name, void** args) {
+        const auto* a = static_cast<const dg::EnsArgs*>(args[0]);
+        const auto it = fake::state().device.find(const_cast<dg::EnsItem*>(a->items));
+        std::string s = name;
+        for (int x : a->chunk) s += " " + std::to_string(x);
+        seen.push_back(s);
+        listed = listed && it != fake::state().device.end() && it->second >= size_t(a->chunk[8]) * sizeof(dg::EnsItem);
+    };
+    CHECK(dgh_ensemble_run(c, e, 1, 0, nullptr) == DGH_OK && listed);
+    const std::vector<std::string> before = seen;
+    fake::state().fail_malloc = 1;
+    CHECK(dgh_ensemble_set_split(c, e, 5, 8) == DGH_ERR_HIP && fake::state().fail_malloc == 0);
+    seen.clear();
+    CHECK(dgh_ensemble_run(c, e, 1, 0, nullptr) == DGH_OK && listed && seen == before);
+    CHECK(dgh_ensemble_set_split(c, e, 5, 8) == DGH_OK);
+    seen.clear();
+    CHECK(dgh_ensemble_run(c, e, 1, 0, nullptr) == DGH_OK && listed && seen != before);
+    fake::state().on_launch = nullptr;
+    CHECK(dgh_destroy(c) == DGH_OK);
+    CHECK(fake::state().device.empty());
+}
+
 // pinned staging memory: two slots of 1 MiB, two more for every further worker of a larger transfer, given back with the
 // context
 static void staging_as_needed() {
@@ -186,6 +219,7 @@ int main(int argc, char** argv) {
         {"ssprk2_scratch", ssprk2_scratch},
         {"sipg_rhs_threads", sipg_rhs_threads},
         {"ensemble_failing_launch", ensemble_failing_launch},
+        {"ensemble_failing_shape", ensemble_failing_shape},
         {"staging_as_needed", staging_as_needed},
     };
     CHECK(argc == 2 && all.count(argv[1]));

@@ -50,6 +50,11 @@ def test_ensemble_failing_launch(program):
     run(program, "ensemble_failing_launch")
 
 
+def test_ensemble_failing_shape(program):
+    """a tile shape that cannot be taken for want of memory leaves the ensemble's work list and shapes as they were"""
+    run(program, "ensemble_failing_shape")
+
+
 def test_staging_as_needed(program):
     """a context takes as much pinned memory as its transfers need"""
     run(program, "staging_as_needed")
