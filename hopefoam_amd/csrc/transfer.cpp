@@ -89,7 +89,9 @@ hipError_t transfer_array(int device, hipStream_t s, Staging& st, const NodalArr
     const int per = std::max(1, std::min(most, (tiles + 4 * workers - 1) / (4 * workers)));
     const int least = std::max(per, std::min(most, int((to_device ? kChunkUp : kChunkDown) / (size_t(16) * a.Np * sizeof(double)))));
     int chunks = (tiles + least - 1) / least;
-    const int step = (tiles + chunks - 1) / chunks;   // equal chunks
+    // Equal chunks, but for the larger uploads: there what is left over makes a short last chunk, and so a short launch after
+    // the host's last copy (4.2 MB up 146 us in equal chunks, 142 so, 6.7 MB 212 and 204; down 150 and 154, 219 and 224)
+    const int step = to_device && least == per ? least : (tiles + chunks - 1) / chunks;
     chunks = (tiles + step - 1) / step;
     workers = std::min(workers, chunks);
     if (!st.ready(2 * workers)) return transfer_pageable(s, a, host, to_device);
