@@ -686,15 +686,17 @@ static hipError_t launch_inst(const StageArgs& a, int ncu, hipStream_t st) {
             n = 1;
         per_cu = n < 1 ? 1 : n;
     }
-    // A block per group up to one per compute unit, then more only as their wavefronts fill (the wavefronts take groups
-    // apart, so that with more blocks than that each leaves its last SIMDs idle: FP32, K = 11834, order 2 LF 11.7 -> 9.8 us,
-    // order 3 16.9 -> 13.9).  bf16x3 advection at orders 1 and 2 starts with full blocks: another block's copy of the
-    // operators takes longer than a group does (order 2, K = 2048: 5.9 -> 5.6 us).
+    // A block per group up to one per compute unit, then one more for every compute unit as their wavefronts fill (the
+    // wavefronts take groups apart, so that with more blocks than that each leaves its last SIMDs idle: FP32, K = 11834,
+    // order 2 LF 11.7 -> 9.8 us, order 3 16.9 -> 13.9; with fewer some compute units hold a block more than the others: K =
+    // 36000, order 2 LF, 288 blocks 19.2, 512 15.6).  bf16x3 advection at orders 1 and 2 starts with full blocks: another
+    // block's copy of the operators takes longer than a group does (order 2, K = 2048: 5.9 -> 5.6 us).
     constexpr int wpb = threads / 64;
     constexpr bool pack = packs<N, VolumeFlux<PHYS, T>::NV, SPLIT>() && N <= 2;
     const int groups = (a.K + 15) / 16;
     const int full = (groups + wpb - 1) / wpb, least = pack ? 0 : groups < ncu ? groups : ncu;
-    int nb = full < least ? least : full < ncu * per_cu ? full : ncu * per_cu;
+    const int even = full <= ncu ? full : (full + ncu - 1) / ncu * ncu;
+    int nb = even < least ? least : even < ncu * per_cu ? even : ncu * per_cu;
     nb = nb < 8 ? 8 : (nb + 7) / 8 * 8;
     if (a.block_cap > 0 && nb > a.block_cap) nb = a.block_cap < 8 ? 8 : a.block_cap / 8 * 8;
     hipLaunchKernelGGL((stage_kernel<N, PHYS, T, SPLIT, MOM, FLUX, UPDATE>), dim3(nb), dim3(threads), 0, st, a);

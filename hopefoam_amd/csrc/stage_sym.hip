@@ -504,11 +504,14 @@ static hipError_t launch_sym_inst(const StageArgs& a, int ncu, hipStream_t st) {
         per_cu = n < 1 ? 1 : n;
     }
     const int groups = (a.K + 15) / 16;
-    // a persistent grid: a block per group up to one per compute unit, then more only as their wavefronts fill (the
-    // wavefronts of a block take groups apart, so that with more blocks than that each leaves its last SIMDs idle; as
-    // many as are resident, order 1 LF, K = 32768: 11.6 -> 9.6 us, order 2 Roe, K = 11834: 11.3 -> 8.0)
+    // a persistent grid: a block per group up to one per compute unit, then one more for every compute unit as their
+    // wavefronts fill (the wavefronts of a block take groups apart, so that with more blocks than that each leaves its last
+    // SIMDs idle; as many as are resident -> as here, order 1 LF, K = 32768: 11.6 -> 9.6 us, order 2 Roe, K = 11834: 11.3
+    // -> 8.0; with fewer some compute units hold a block more than the others: order 2 LF, K = 20174, 320 blocks 11.6, 512
+    // 11.0, order 1 9.0 and 8.4)
     const int full = (groups + sym_waves<N>() - 1) / sym_waves<N>(), least = groups < ncu ? groups : ncu;
-    int nb = full < least ? least : full < ncu * per_cu ? full : ncu * per_cu;
+    const int even = full <= ncu ? full : (full + ncu - 1) / ncu * ncu;
+    int nb = even < least ? least : even < ncu * per_cu ? even : ncu * per_cu;
     nb = nb < 8 ? 8 : (nb + 7) / 8 * 8;
     if (a.block_cap > 0 && nb > a.block_cap) nb = a.block_cap < 8 ? 8 : a.block_cap / 8 * 8;
     hipLaunchKernelGGL((stage_sym_kernel<N, PHYS, FLUX, UPDATE>), dim3(nb), dim3(threads), 0, st, a);
